@@ -24,14 +24,15 @@ struct MlpAdam {
 };
 
 bool       mlp_dims_supported(const MlpDims &d);
-// Samples per block of launch_mlp_grad (the number of per-block partials is ceil(count / this))
-int        mlp_grad_block(const MlpDims &d);
+// Blocks of launch_mlp_grad for a batch of count samples: the rows of its partials
+int        mlp_grad_blocks(int count);
 // Batch gradient of the mean squared error over samples idx[first .. first+count) (idx null: first .. first+count);
-// inv_norm = 1 / (count * no).  Writes nblocks per-block partials [nblocks][nparams] and loss partials.
+// inv_norm = 1 / (count * no).  Writes a row of nparams gradient entries and the loss per block,
+// partial [mlp_grad_blocks(count)][nparams + 1].
 hipError_t launch_mlp_grad(const MlpDims &d, const float *theta, const float *X, const float *T, const int *idx, int first, int count, float inv_norm,
-                           float *partial, float *loss_partial, int *nblocks, hipStream_t s);
-hipError_t launch_mlp_reduce_adam(int np, int nblocks, const float *partial, const float *loss_partial, float *grad, float *loss, float *theta, float *m,
-                                  float *v, const MlpAdam &adam, bool apply, hipStream_t s);
+                           float *partial, hipStream_t s);
+hipError_t launch_mlp_reduce_adam(int np, int nblocks, const float *partial, float *grad, float *loss, float *theta, float *m, float *v,
+                                  const MlpAdam &adam, bool apply, hipStream_t s);
 hipError_t launch_mlp_predict(const MlpDims &d, const float *theta, const float *X, int n, float *Y, hipStream_t s);
 hipError_t launch_sgs_model_samples(long long n, const double *train, const double *filtered, const double *G, const double *A, const CeedMiGas &gas,
                                     float *X, double *S, hipStream_t s);

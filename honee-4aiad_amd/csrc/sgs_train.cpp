@@ -47,7 +47,7 @@ struct HoneeMiMlp_ {
   int         np;
   hipStream_t s = nullptr;
   float      *theta = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr, *loss = nullptr;
-  float      *partial = nullptr, *loss_partial = nullptr;
+  float      *partial = nullptr;
   int         partial_blocks = 0;
   long long   step           = 0;
   // staging of host inputs
@@ -60,9 +60,7 @@ struct HoneeMiMlp_ {
 static int ensure_partials(HoneeMiMlp p, int nblocks) {
   if (nblocks <= p->partial_blocks) return 0;
   if (p->partial) HIPCHK(hipFree(p->partial));
-  if (p->loss_partial) HIPCHK(hipFree(p->loss_partial));
-  HIPCHK(hipMalloc((void **)&p->partial, sizeof(float) * (size_t)nblocks * p->np));
-  HIPCHK(hipMalloc((void **)&p->loss_partial, sizeof(float) * nblocks));
+  HIPCHK(hipMalloc((void **)&p->partial, sizeof(float) * (size_t)nblocks * (p->np + 1)));
   p->partial_blocks = nblocks;
   return 0;
 }
@@ -91,17 +89,16 @@ static int stage(HoneeMiMlp p, int n, const float *X, const float *T, int mem_ty
 // Gradient (and optionally an Adam step) on samples idx[first .. first+count) of dX/dT
 static int batch(HoneeMiMlp p, const float *dX, const float *dT, const int *idx, int first, int count, const HoneeMiMlpTrainOptions *o, bool adam,
                  float *loss_dst) {
-  const int tpb = mlp_grad_block(p->d), nb = (count + tpb - 1) / tpb;
+  const int nb = mlp_grad_blocks(count);
   if (ensure_partials(p, nb)) return 1;
-  int nblocks = 0;
-  HIPCHK(launch_mlp_grad(p->d, p->theta, dX, dT, idx, first, count, 1.0f / ((float)count * p->d.no), p->partial, p->loss_partial, &nblocks, p->s));
+  HIPCHK(launch_mlp_grad(p->d, p->theta, dX, dT, idx, first, count, 1.0f / ((float)count * p->d.no), p->partial, p->s));
   MlpAdam a{};
   if (adam) {
     p->step++;
     a = MlpAdam{o->lr, o->beta1, o->beta2, o->eps, (float)(1.0 - pow((double)o->beta1, (double)p->step)),
                 (float)(1.0 - pow((double)o->beta2, (double)p->step))};
   }
-  HIPCHK(launch_mlp_reduce_adam(p->np, nblocks, p->partial, p->loss_partial, p->grad, loss_dst, p->theta, p->m, p->v, a, adam, p->s));
+  HIPCHK(launch_mlp_reduce_adam(p->np, nb, p->partial, p->grad, loss_dst, p->theta, p->m, p->v, a, adam, p->s));
   return 0;
 }
 
@@ -239,7 +236,7 @@ int HoneeMiMlpDestroy(HoneeMiMlp *mlp) {
   HoneeMiMlp p = *mlp;
   if (!p) return 0;
   if (p->s) (void)hipStreamSynchronize(p->s);
-  for (void *a : {(void *)p->theta, (void *)p->m, (void *)p->v, (void *)p->grad, (void *)p->loss, (void *)p->partial, (void *)p->loss_partial,
+  for (void *a : {(void *)p->theta, (void *)p->m, (void *)p->v, (void *)p->grad, (void *)p->loss, (void *)p->partial,
                   (void *)p->X, (void *)p->T, (void *)p->idx})
     if (a) (void)hipFree(a);
   if (p->s) (void)hipStreamDestroy(p->s);

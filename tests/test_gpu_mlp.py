@@ -149,3 +149,19 @@ def test_two_hidden_layers_adam_and_training():
     assert np.all(np.isfinite(hist)) and hist[-1] < 0.05 * hist[0], (hist[0], hist[-1])
     student.close()
     teacher.close()
+
+
+@pytest.mark.parametrize("dims", [(6, 20, 6), DIMS2])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 65, 512 * 64 - 3, 512 * 64 + 19])
+def test_loss_grad_at_group_edges(n, dims):
+    """Batches around one wave's 16 samples, one block's 64 and one pass of the largest grid (512 blocks)."""
+    _say(f"mlp group edges n={n} dims={dims}")
+    rng = np.random.default_rng(100 + n)
+    mlp = TR.Mlp(alpha=ALPHA, seed=23, dims=dims)
+    X, T = rng.normal(size=(n, 6)).astype(np.float32), rng.normal(size=(n, 6)).astype(np.float32)
+    loss, g = mlp.loss_grad(X, T)
+    loss_ref, g_ref = O.mlp_loss_grad(_f64(mlp.params), _f64(X), _f64(T), float(np.float32(ALPHA)), dims)
+    assert abs(loss - loss_ref) < 1e-5 * loss_ref
+    # FP32 sums as above: 5e-5 relative (2-norm)
+    assert np.linalg.norm(g - g_ref) < 5e-5 * np.linalg.norm(g_ref), np.linalg.norm(g - g_ref) / np.linalg.norm(g_ref)
+    mlp.close()
