@@ -215,10 +215,6 @@ struct Contract5 {
   }
 };
 
-// Multi-component basis stage: the element's LDS stage X[slot][Q^3] holds one slot per (field component, point);
-// every pass treats NC components together, so each 1D coefficient row is read from LDS once per pass and the NC
-// independent contractions overlap their LDS latency.  Barriers are block-wide; a pass reads other threads' slots only
-// after a barrier that follows their writes.
 // Cross-lane access for the 4 x 4 x 4 element (P = Q = 4, one 64-lane wave per element, lane = qx + 4 qy + 16 qz):
 // the four lanes of an x line form a DPP quad and the sixteen lanes of an xy slab form a DPP row.  dpp_d<CTRL> returns
 // the double held by the lane that the DPP control CTRL selects (quad_perm broadcast 0x00, 0x55, 0xAA, 0xFF of quad
@@ -434,194 +430,57 @@ struct ContractPairs {
   }
 };
 
-// ZX: the z passes of the 4 x 4 x 4 element also across lanes (v_permlane swaps) instead of through LDS; measured
-// faster for the FP32 Jacobian and slower for the FP64 operators
-template <int P, int Q, bool ZX = false>
-struct Stage {
-  using D = Dims<P, Q>;
-  static constexpr int Q3 = D::Q3;
-  const double *B;   // [Q][P]
-  const double *Dc;  // [Q][Q]
+// Basis stage of the 4 x 4 x 4 element with every pass across the lanes of the element's wave (x: DPP quad broadcasts, y: DPP
+// row rotations, z: v_permlane swaps); X[slot][point] only parks values across the point body.  Measured faster than the
+// matrix-core passes (StageMF) for the FP32 Jacobian and slower for the FP64 operators.
+struct StageX {
+  static constexpr int Q3 = 64;
+  const double *B;   // [4][4] interpolation B[q][n]
+  const double *Dc;  // [4][4] collocated derivative
   double (*X)[Q3];
   int t, qx, qy, qz;
 
-  __device__ Stage(const double *B_, const double *Dc_, const double *, double (*X_)[Q3], int t_) : B(B_), Dc(Dc_), X(X_), t(t_) {
-    qx = t % Q;
-    qy = (t / Q) % Q;
-    qz = t / (Q * Q);
+  __device__ StageX(const double *B_, const double *Dc_, const double *, double (*X_)[Q3], int t_) : B(B_), Dc(Dc_), X(X_), t(t_) {
+    qx = t & 3;
+    qy = (t >> 2) & 3;
+    qz = t >> 4;
   }
 
-  // interp() followed by grad(dst, gdst)
+  // Node values u[c] (lane = node a + 4 b + 16 c) -> quadrature-point values in slots dst..
   template <int NC>
-  __device__ void interp_grad(const double (&u)[NC], int s0, int s1, int dst, int gdst) {
-    interp<NC>(u, s0, s1, dst);
-    grad<NC>(dst, gdst);
+  __device__ void interp(const double (&u)[NC], int dst) {
+    const RowRot rr(qy);
+    double       bx[4], by[4], bz[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      bx[i] = B[qx * 4 + i];
+      by[i] = B[qy * 4 + rr.y[i]];
+      bz[i] = B[qz * 4 + i];
+    }
+#pragma unroll
+    for (int c = 0; c < NC; c++) X[dst + c][t] = z_contract(bz, row_contract(by, quad_contract(bx, u[c])));
   }
 
-  // Interpolate NC components from node values u[c] (threads t < P^3) to this thread's quadrature point, leaving the
-  // results in slots dst..dst+NC-1.  Slots s0..s0+NC-1 and s1..s1+NC-1 are scratch; dst may equal s1 but not s0.
-  // Ends without a barrier: only this thread's own dst slots are written by the last pass.
+  // Values (slots dst..) and collocated reference gradients (slots gdst + NC d + c)
   template <int NC>
-  __device__ void interp(const double (&u)[NC], int s0, int s1, int dst) {
-    if constexpr (P == 4 && Q == 4 && ZX) {  // all three passes across the lanes of the element's wave
-      const RowRot rr(qy);
-      double       bx[4], by[4], bz[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        bx[i] = B[qx * 4 + i];
-        by[i] = B[qy * 4 + rr.y[i]];
-        bz[i] = B[qz * 4 + i];
-      }
-#pragma unroll
-      for (int c = 0; c < NC; c++) X[dst + c][t] = z_contract(bz, row_contract(by, quad_contract(bx, u[c])));
-      return;
-    } else if constexpr (P == 4 && Q == 4) {  // x and y passes across lanes, z through LDS (slot s0)
-      const RowRot rr(qy);
-      double       bx[4], by[4], bz[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        bx[i] = B[qx * 4 + i];
-        by[i] = B[qy * 4 + rr.y[i]];
-        bz[i] = B[qz * 4 + i];
-      }
-#pragma unroll
-      for (int c = 0; c < NC; c++) X[s0 + c][t] = row_contract(by, quad_contract(bx, u[c]));
-      __syncthreads();
-      double r[NC];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double acc = 0;
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc += bz[i] * X[s0 + c][(i * 4 + qy) * 4 + qx];
-        r[c] = acc;
-      }
-#pragma unroll
-      for (int c = 0; c < NC; c++) X[dst + c][t] = r[c];
-      return;
-    }
-    if (t < D::P3) {
-#pragma unroll
-      for (int c = 0; c < NC; c++) X[s0 + c][t] = u[c];
-    }
+  __device__ void interp_grad(const double (&u)[NC], int dst, int gdst) {
+    interp<NC>(u, dst);
     __syncthreads();
-    if (t < D::PPQ) {  // x: s1[k][j][ix] = sum_a B[ix][a] u[k][j][a]
-      const int ix = t % Q, kj = t / Q;
-      double    b[P];
+    const RowRot rr(qy);
+    double       dx[4], dy[4], dz[4];
 #pragma unroll
-      for (int i = 0; i < P; i++) b[i] = B[ix * P + i];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double acc = 0;
-#pragma unroll
-        for (int i = 0; i < P; i++) acc += b[i] * X[s0 + c][kj * P + i];
-        X[s1 + c][t] = acc;
-      }
-    }
-    __syncthreads();
-    if (t < D::PQQ) {  // y: s0[k][iy][ix] = sum_b B[iy][b] s1[k][b][ix]
-      const int ix = t % Q, iy = (t / Q) % Q, k = t / (Q * Q);
-      double    b[P];
-#pragma unroll
-      for (int i = 0; i < P; i++) b[i] = B[iy * P + i];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double acc = 0;
-#pragma unroll
-        for (int i = 0; i < P; i++) acc += b[i] * X[s1 + c][(k * P + i) * Q + ix];
-        X[s0 + c][t] = acc;
-      }
-    }
-    __syncthreads();
-    {  // z: value at (qx, qy, qz)
-      double b[P];
-#pragma unroll
-      for (int i = 0; i < P; i++) b[i] = B[qz * P + i];
-      double r[NC];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double acc = 0;
-#pragma unroll
-        for (int i = 0; i < P; i++) acc += b[i] * X[s0 + c][(i * Q + qy) * Q + qx];
-        r[c] = acc;
-      }
-#pragma unroll
-      for (int c = 0; c < NC; c++) X[dst + c][t] = r[c];
-    }
-  }
-
-  // Collocated reference gradient of the NC quadrature-point fields in slots src.. (written before the last barrier
-  // or by this thread): slot gdst + NC*d + c receives d/dX_d of component c.  Starts with a barrier.
-  template <int NC>
-  __device__ void grad(int src, int gdst) {
-    __syncthreads();
-    if constexpr (P == 4 && Q == 4 && ZX) {  // derivatives across the lanes of the element's wave from this lane's value
-      const RowRot rr(qy);
-      double       dx[4], dy[4], dz[4];
-#pragma unroll
-      for (int m = 0; m < 4; m++) {
-        dx[m] = Dc[qx * 4 + m];
-        dy[m] = Dc[qy * 4 + rr.y[m]];
-        dz[m] = Dc[qz * 4 + m];
-      }
-      double g[3][NC];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        const double v = X[src + c][t];
-        g[0][c]        = quad_contract(dx, v);
-        g[1][c]        = row_contract(dy, v);
-        g[2][c]        = z_contract(dz, v);
-      }
-#pragma unroll
-      for (int d = 0; d < 3; d++)
-#pragma unroll
-        for (int c = 0; c < NC; c++) X[gdst + NC * d + c][t] = g[d][c];
-      return;
-    } else if constexpr (P == 4 && Q == 4) {  // x and y derivatives across lanes from this lane's value, z through LDS
-      const RowRot rr(qy);
-      double       dx[4], dy[4], dz[4];
-#pragma unroll
-      for (int m = 0; m < 4; m++) {
-        dx[m] = Dc[qx * 4 + m];
-        dy[m] = Dc[qy * 4 + rr.y[m]];
-        dz[m] = Dc[qz * 4 + m];
-      }
-      double g[3][NC];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        const double v  = X[src + c][t];
-        double       gz = 0;
-#pragma unroll
-        for (int m = 0; m < 4; m++) gz += dz[m] * X[src + c][(m * 4 + qy) * 4 + qx];
-        g[0][c] = quad_contract(dx, v);
-        g[1][c] = row_contract(dy, v);
-        g[2][c] = gz;
-      }
-#pragma unroll
-      for (int d = 0; d < 3; d++)
-#pragma unroll
-        for (int c = 0; c < NC; c++) X[gdst + NC * d + c][t] = g[d][c];
-      return;
-    }
-    double dx[Q], dy[Q], dz[Q];
-#pragma unroll
-    for (int m = 0; m < Q; m++) {
-      dx[m] = Dc[qx * Q + m];
-      dy[m] = Dc[qy * Q + m];
-      dz[m] = Dc[qz * Q + m];
+    for (int m = 0; m < 4; m++) {
+      dx[m] = Dc[qx * 4 + m];
+      dy[m] = Dc[qy * 4 + rr.y[m]];
+      dz[m] = Dc[qz * 4 + m];
     }
     double g[3][NC];
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-      double gx = 0, gy = 0, gz = 0;
-#pragma unroll
-      for (int m = 0; m < Q; m++) {
-        gx += dx[m] * X[src + c][(qz * Q + qy) * Q + m];
-        gy += dy[m] * X[src + c][(qz * Q + m) * Q + qx];
-        gz += dz[m] * X[src + c][(m * Q + qy) * Q + qx];
-      }
-      g[0][c] = gx;
-      g[1][c] = gy;
-      g[2][c] = gz;
+      const double v = X[dst + c][t];
+      g[0][c]        = quad_contract(dx, v);
+      g[1][c]        = row_contract(dy, v);
+      g[2][c]        = z_contract(dz, v);
     }
 #pragma unroll
     for (int d = 0; d < 3; d++)
@@ -629,158 +488,229 @@ struct Stage {
       for (int c = 0; c < NC; c++) X[gdst + NC * d + c][t] = g[d][c];
   }
 
-  // Transpose of interp (+ collocated gradient) for NC components: the quadrature-point values are in slots v0..
-  // (HAS_V) and the reference-gradient test weights in slots g0 + NC*d + c (HAS_G), all written before the call.
-  // Returns in r[c] (threads t < P^3) sum_q B3(q,n) v_c(q) + sum_q sum_d G3_d(q,n) g_{d,c}(q) for node n = t.
-  // Uses slots v0.. and g0.. as scratch (needs g0 + 2*NC <= slot count when !HAS_G).  Starts and ends with a barrier.
+  // Transpose: node contributions r[c] = B3^T (v_c + sum_d Dc_d^T g_{d,c}) from slots v0.. and g0 + NC d + c
   template <int NC, bool HAS_V, bool HAS_G>
   __device__ void transpose(int v0, int g0, double (&r)[NC]) {
     __syncthreads();
-    if constexpr (P == 4 && Q == 4 && ZX) {  // all passes across the lanes of the element's wave
-      const RowRot rr(qy);
-      double       bxT[4], byT[4], bzT[4];
+    const RowRot rr(qy);
+    double       bxT[4], byT[4], bzT[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        bxT[i] = B[i * 4 + qx];
-        byT[i] = B[rr.y[i] * 4 + qy];
-        bzT[i] = B[i * 4 + qz];
-      }
-      double dxT[4], dyT[4], dzT[4];
-      if (HAS_G) {
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-          dxT[m] = Dc[m * 4 + qx];
-          dyT[m] = Dc[rr.y[m] * 4 + qy];
-          dzT[m] = Dc[m * 4 + qz];
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double w = HAS_V ? X[v0 + c][t] : 0.0;
-        if (HAS_G) {
-          w += z_contract(dzT, X[g0 + 2 * NC + c][t]);
-          w += quad_contract(dxT, X[g0 + c][t]);
-          w += row_contract(dyT, X[g0 + NC + c][t]);
-        }
-        r[c] = quad_contract(bxT, row_contract(byT, z_contract(bzT, w)));
-      }
-      __syncthreads();
-      return;
-    } else if constexpr (P == 4 && Q == 4) {  // z passes through LDS (slot v0 as scratch), x and y passes across lanes
-      const RowRot rr(qy);
-      double       w[NC];
-#pragma unroll
-      for (int c = 0; c < NC; c++) w[c] = HAS_V ? X[v0 + c][t] : 0.0;
-      if (HAS_G) {
-        double dxT[4], dyT[4], dz[4];
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-          dxT[m] = Dc[m * 4 + qx];
-          dyT[m] = Dc[rr.y[m] * 4 + qy];
-          dz[m]  = Dc[m * 4 + qz];
-        }
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-          double acc = w[c];
-#pragma unroll
-          for (int m = 0; m < 4; m++) acc += dz[m] * X[g0 + 2 * NC + c][(m * 4 + qy) * 4 + qx];
-          acc += quad_contract(dxT, X[g0 + c][t]);
-          acc += row_contract(dyT, X[g0 + NC + c][t]);
-          w[c] = acc;
-        }
-        __syncthreads();
-      }
-#pragma unroll
-      for (int c = 0; c < NC; c++) X[v0 + c][t] = w[c];
-      __syncthreads();
-      double bz[4], byT[4], bxT[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        bz[i]  = B[i * 4 + qz];
-        byT[i] = B[rr.y[i] * 4 + qy];
-        bxT[i] = B[i * 4 + qx];
-      }
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double acc = 0;
-#pragma unroll
-        for (int z = 0; z < 4; z++) acc += bz[z] * X[v0 + c][(z * 4 + qy) * 4 + qx];
-        r[c] = quad_contract(bxT, row_contract(byT, acc));
-      }
-      __syncthreads();
-      return;
+    for (int i = 0; i < 4; i++) {
+      bxT[i] = B[i * 4 + qx];
+      byT[i] = B[rr.y[i] * 4 + qy];
+      bzT[i] = B[i * 4 + qz];
     }
-    double w[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) w[c] = HAS_V ? X[v0 + c][t] : 0.0;
+    double dxT[4], dyT[4], dzT[4];
     if (HAS_G) {
-      double dx[Q], dy[Q], dz[Q];
 #pragma unroll
-      for (int m = 0; m < Q; m++) {
-        dx[m] = Dc[m * Q + qx];
-        dy[m] = Dc[m * Q + qy];
-        dz[m] = Dc[m * Q + qz];
+      for (int m = 0; m < 4; m++) {
+        dxT[m] = Dc[m * 4 + qx];
+        dyT[m] = Dc[rr.y[m] * 4 + qy];
+        dzT[m] = Dc[m * 4 + qz];
       }
+    }
 #pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double acc = w[c];
+    for (int c = 0; c < NC; c++) {
+      double w = HAS_V ? X[v0 + c][t] : 0.0;
+      if (HAS_G) {
+        w += z_contract(dzT, X[g0 + 2 * NC + c][t]);
+        w += quad_contract(dxT, X[g0 + c][t]);
+        w += row_contract(dyT, X[g0 + NC + c][t]);
+      }
+      r[c] = quad_contract(bxT, row_contract(byT, z_contract(bzT, w)));
+    }
+    __syncthreads();
+  }
+};
+
+// One line per thread: the basis stage of every element but the 4 x 4 x 4 one.  A pass along a direction gives each thread
+// whole lines of single components: it reads a line's values from LDS, applies the 1D table and writes the line back in
+// place, so a pass moves 2 values per output where one output per thread moves a whole line for each.  The tables come
+// through the scalar cache into scalar registers (the same entry for every lane), not through LDS.  The lines of all
+// components of all the block's elements are dealt out over the block's NT threads.
+//
+// X[element][slot][point]: node (i, j, k) of an element sits at point i + Q (j + Q k), so that a line's pass is in place
+// for P < Q too.  The slots are an odd number of values apart (kSlot), which spreads the components of a line over the
+// banks where Q is even.
+// Bound by LDS at the 5 x 5 x 5 element and by instruction issue at the 3 x 3 x 3 one (address arithmetic is formed once per
+// phase).  Measured against one output per thread with the tables in LDS: IFunction at 40^3 p=4 886 -> 662 us, IJacobian
+// 663 -> 541 us, explicit residual at 64^3 p=2 388 -> 330 us, residual and Jacobian pair at 64 x 64 x 48 p=1 298 -> 296 us.
+// Reading and writing the L-vector and E-vector through LDS in fully coalesced order as well was slower (p=2 pair at 48^3
+// 648 -> 667 us each): the index arithmetic costs more than the cache lines.
+template <int P, int Q, int EPB, int NST>
+struct LineStage {
+  static constexpr int Q2 = Q * Q, Q3 = Q2 * Q, kSlot = Q3 | 1;
+  static constexpr int NT = (EPB * Q3 + 63) / 64 * 64;  // threads of the block
+  using Table = const __attribute__((address_space(4))) double *;
+  Table   B;   // [Q][P]
+  Table   Dc;  // [Q][Q]
+  double *X;   // [EPB][NST][kSlot]
+  int     tid;
+
+  __device__ LineStage(const double *B_, const double *Dc_, double (*X_)[NST][kSlot], int tid_)
+      : B((Table)(unsigned long long)B_), Dc((Table)(unsigned long long)Dc_), X(&X_[0][0][0]), tid(tid_) {}
+
+  // Point of node t of an element
+  __device__ static int node(int t) {
+    if constexpr (P == Q) return t;
+    return t % P + Q * ((t / P) % P + Q * (t / (P * P)));
+  }
+
+  // The thread's lines among the LA x LB lines at a SA + b SB of NC components of every element: line r of the thread starts
+  // at[r] past slot 0 of the first element.  In the last round, the lanes of a wave that run out of lines repeat the wave's
+  // last one (a wave reads its lines before it writes any, and the copies write the same values), so that the rounds are
+  // straight-line code whose loads overlap; a wave without any line skips the round.
+  template <int NC, int LA, int LB, int SA, int SB>
+  struct Lines {
+    static constexpr int L = LA * LB, N = EPB * NC * L, R = (N + NT - 1) / NT;
+    int  at[R];
+    bool last;  // whether the thread's wave has a line in the last round
+
+    __device__ explicit Lines(int tid) : last(true) {
 #pragma unroll
-        for (int m = 0; m < Q; m++) {
-          acc += dx[m] * X[g0 + c][(qz * Q + qy) * Q + m];
-          acc += dy[m] * X[g0 + NC + c][(qz * Q + m) * Q + qx];
-          acc += dz[m] * X[g0 + 2 * NC + c][(m * Q + qy) * Q + qx];
+      for (int r = 0; r < R; r++) {
+        int k = tid + r * NT;
+        if (r == R - 1 && N % NT != 0) {
+          last = NT == 64 || (k & ~63) < N;
+          k    = k < N ? k : N - 1;
         }
-        w[c] = acc;
+        const int m = k % L, c = k / L;
+        at[r] = (EPB == 1 ? c : c / NC * NST + c % NC) * kSlot + m % LA * SA + m / LA * SB;
       }
+    }
+  };
+  template <int N>
+  __device__ static void get(const double *x, int stride, double (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = x[i * stride];
+  }
+  template <int N>
+  __device__ static void put(double *x, int stride, const double (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; i++) x[i * stride] = v[i];
+  }
+  // For each of the thread's lines: f(its values of the arrays at offsets o[], pointer), after the loads of all its lines
+  template <int NI, int NARR, class LN, class F>
+  __device__ static void each(const LN &ln, double *x, const int (&o)[NARR], int stride, F &&f) {
+    constexpr int R = LN::R;
+    if (R == 1 && !ln.last) return;
+    double in[R][NARR][NI];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (r < R - 1 || NT == 64 || ln.last)
+#pragma unroll
+        for (int j = 0; j < NARR; j++) get(x + ln.at[r] + o[j], stride, in[r][j]);
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (r < R - 1 || NT == 64 || ln.last) f(in[r], x + ln.at[r]);
+  }
+  // x <- T x (or T^T x) along the lines
+  template <int NI, int NO, bool TR, class LN>
+  __device__ static void pass(Table T, const LN &ln, double *x, int stride) {
+    each<NI, 1>(ln, x, {0}, stride, [&](const double (&in)[1][NI], double *y) {
+      double out[NO];
+      apply<TR, false>(T, in[0], out), put(y, stride, out);
+    });
+  }
+  // out (+)= T in, or T^T in, of a row-major table
+  template <bool TR, bool ADD, int NI, int NO>
+  __device__ static void apply(Table T, const double (&in)[NI], double (&out)[NO]) {
+#pragma unroll
+    for (int o = 0; o < NO; o++) {
+      double acc = ADD ? out[o] : T[TR ? o : o * NI] * in[0];
+#pragma unroll
+      for (int i = ADD ? 0 : 1; i < NI; i++) acc += T[TR ? i * NO + o : o * NI + i] * in[i];
+      out[o] = acc;
+    }
+  }
+
+  // Node values in slots u0.. (written before the call) -> point values there; with GRAD also the reference gradient, d/dX_d
+  // of component c in slot g0 + NC d + c; with NC2 > 0 a second field's values in slots u1...  Starts and ends with a barrier.
+  template <int NC, bool GRAD, int NC2 = 0>
+  __device__ void interp_grad(int u0, int g0, int u1 = 0) const {
+    constexpr int M = NC2 > 0 ? NC2 : 1;
+    const Lines<NC, P, P, Q, Q2> lx(tid);
+    const Lines<NC, Q, P, 1, Q2> ly(tid);
+    const Lines<NC, Q, Q, 1, Q>  lz(tid);
+    const Lines<M, P, P, Q, Q2>  mx(tid);
+    const Lines<M, Q, P, 1, Q2>  my(tid);
+    const Lines<M, Q, Q, 1, Q>   mz(tid);
+    double *const x0 = X + u0 * kSlot, *const x1 = X + u1 * kSlot;
+    __syncthreads();
+    pass<P, Q, false>(B, lx, x0, 1);
+    if constexpr (NC2 > 0) pass<P, Q, false>(B, mx, x1, 1);
+    __syncthreads();
+    pass<P, Q, false>(B, ly, x0, Q);
+    if constexpr (NC2 > 0) pass<P, Q, false>(B, my, x1, Q);
+    __syncthreads();
+    if constexpr (GRAD) {
+      double *const g = x0 + (g0 - u0) * kSlot;
+      each<P, 1>(lz, x0, {0}, Q2, [&](const double (&in)[1][P], double *x) {
+        double out[Q], d[Q];
+        apply<false, false>(B, in[0], out), put(x, Q2, out);
+        apply<false, false>(Dc, out, d), put(x + (g - x0) + 2 * NC * kSlot, Q2, d);
+      });
+      if constexpr (NC2 > 0) pass<P, Q, false>(B, mz, x1, Q2);
       __syncthreads();
-    }
-    const int sa = v0, sb = g0, sc = g0 + NC;
-#pragma unroll
-    for (int c = 0; c < NC; c++) X[sa + c][t] = w[c];
-    __syncthreads();
-    if (t < D::PQQ) {  // z^T: sb[c][iy][ix] = sum_qz B[qz][c] w[qz][iy][ix]
-      const int ix = t % Q, iy = (t / Q) % Q, cz = t / (Q * Q);
-      double    b[Q];
-#pragma unroll
-      for (int z = 0; z < Q; z++) b[z] = B[z * P + cz];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double acc = 0;
-#pragma unroll
-        for (int z = 0; z < Q; z++) acc += b[z] * X[sa + c][(z * Q + iy) * Q + ix];
-        X[sb + c][t] = acc;
-      }
+      const Lines<NC, Q, Q, Q, Q2> gx(tid);
+      const Lines<NC, Q, Q, 1, Q2> gy(tid);
+      each<Q, 1>(gx, x0, {0}, 1, [&](const double (&in)[1][Q], double *x) {
+        double d[Q];
+        apply<false, false>(Dc, in[0], d), put(x + (g - x0), 1, d);
+      });
+      each<Q, 1>(gy, x0, {0}, Q, [&](const double (&in)[1][Q], double *x) {
+        double d[Q];
+        apply<false, false>(Dc, in[0], d), put(x + (g - x0) + NC * kSlot, Q, d);
+      });
+    } else {
+      pass<P, Q, false>(B, lz, x0, Q2);
+      if constexpr (NC2 > 0) pass<P, Q, false>(B, mz, x1, Q2);
     }
     __syncthreads();
-    if (t < D::PPQ) {  // y^T: sc[c][b][ix] = sum_qy B[qy][b] sb[c][qy][ix]
-      const int ix = t % Q, bb = (t / Q) % P, cz = t / (Q * P);
-      double    b[Q];
+  }
+
+  // Value weights in slots v0.. (HAS_V) and reference-gradient weights in slots g0 + NC d + c (HAS_G) -> node
+  // contributions at the node points of slots v0..  Starts and ends with a barrier.
+  template <int NC, bool HAS_V, bool HAS_G>
+  __device__ void transpose(int v0, int g0) const {
+    static_assert(HAS_V || HAS_G, "no weights");
+    const Lines<NC, Q, Q, Q, Q2> lx(tid);
+    double *const                x0 = X + v0 * kSlot;
+    const int                    g  = (g0 - v0) * kSlot;
+    __syncthreads();
+    if constexpr (HAS_G) {
+      const Lines<NC, Q, Q, 1, Q>  lz(tid);
+      const Lines<NC, Q, Q, 1, Q2> ly(tid);
+      // w = Dc^T g (+ the values at the line's place): value and gradient lines
+      auto add = [&](const double (&in)[2][Q], double *x, int stride) {
+        double w[Q];
 #pragma unroll
-      for (int y = 0; y < Q; y++) b[y] = B[y * P + bb];
+        for (int i = 0; i < Q; i++) w[i] = in[0][i];
+        apply<true, true>(Dc, in[1], w), put(x, stride, w);
+      };
+      if constexpr (HAS_V)
+        each<Q, 2>(lz, x0, {0, g + 2 * NC * kSlot}, Q2, [&](const double (&in)[2][Q], double *x) { add(in, x, Q2); });
+      else
+        each<Q, 1>(lz, x0, {g + 2 * NC * kSlot}, Q2, [&](const double (&in)[1][Q], double *x) {
+          double w[Q];
+          apply<true, false>(Dc, in[0], w), put(x, Q2, w);
+        });
+      __syncthreads();
+      each<Q, 2>(ly, x0, {0, g + NC * kSlot}, Q, [&](const double (&in)[2][Q], double *x) { add(in, x, Q); });
+      __syncthreads();
+      each<Q, 2>(lx, x0, {0, g}, 1, [&](const double (&in)[2][Q], double *x) {
+        double w[Q], out[P];
 #pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double acc = 0;
-#pragma unroll
-        for (int y = 0; y < Q; y++) acc += b[y] * X[sb + c][(cz * Q + y) * Q + ix];
-        X[sc + c][t] = acc;
-      }
+        for (int i = 0; i < Q; i++) w[i] = in[0][i];
+        apply<true, true>(Dc, in[1], w), apply<true, false>(B, w, out), put(x, 1, out);
+      });
+    } else {
+      pass<Q, P, true>(B, lx, x0, 1);
     }
     __syncthreads();
-#pragma unroll
-    for (int c = 0; c < NC; c++) r[c] = 0;
-    if (t < D::P3) {  // x^T: r[c][b][a] = sum_qx B[qx][a] sc[c][b][qx]
-      const int a = t % P, cb = t / P;
-      double    b[Q];
-#pragma unroll
-      for (int x = 0; x < Q; x++) b[x] = B[x * P + a];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double acc = 0;
-#pragma unroll
-        for (int x = 0; x < Q; x++) acc += b[x] * X[sc + c][cb * Q + x];
-        r[c] = acc;
-      }
-    }
+    pass<Q, P, true>(B, Lines<NC, P, Q, 1, Q2>(tid), x0, Q);
+    __syncthreads();
+    pass<Q, P, true>(B, Lines<NC, P, P, 1, Q>(tid), x0, Q2);
     __syncthreads();
   }
 };
@@ -812,7 +742,7 @@ struct StageMF {
 
   // Node values u[c] (lane = node a + 4 b + 16 c) -> quadrature-point values in slots dst..
   template <int NC>
-  __device__ void interp(const double (&u)[NC], int, int, int dst) {
+  __device__ void interp(const double (&u)[NC], int dst) {
     const RowRot rr(qy);
     double       by[4];
 #pragma unroll
@@ -825,7 +755,7 @@ struct StageMF {
   // Values (slots dst..) and reference gradients (slots gdst + NC d + c): d/dX0 from the z-contracted intermediate with
   // G (G_x B_y B_z), d/dX1 and d/dX2 collocated from the values (Dc_y, Dc_z)
   template <int NC>
-  __device__ void interp_grad(const double (&u)[NC], int, int, int dst, int gdst) {
+  __device__ void interp_grad(const double (&u)[NC], int dst, int gdst) {
     const RowRot rr(qy);
     double       by[4], dy[4];
 #pragma unroll

@@ -6,7 +6,8 @@
 // It serves the velocity-gradient projection right-hand side (qfunctions/velocity_gradient_projection.h:9-36), the
 // anisotropy-tensor projection right-hand side (qfunctions/grid_anisotropy_tensor.h:34-54), Mass_N for any component
 // count (qfunctions/mass.h:19-26) and the SGS residual IFunction_NodalSgs (qfunctions/sgs_dd_model.h:215-241).
-// Each element owns Q^3 threads, one per quadrature point, and its basis passes are staged through LDS (basis3::Stage).
+// Each element owns Q^3 threads, one per quadrature point, and its basis passes are those of the
+// Newtonian volume kernels (basis3::LineStage, and basis3::StageMF for the 4 x 4 x 4 element).
 //
 // k_sgs_nodal evaluates ComputeSgsDDNodal (qfunctions/sgs_dd_model.h:65-96) once per node of the SGS field: every
 // element node of a mesh node sees the same nodal inputs, so the closure value is computed once and the element
@@ -29,16 +30,21 @@ template <int Q>
 constexpr int sgs_elems_per_block() {
   return (Q * Q * Q >= 64) ? 1 : 64 / (Q * Q * Q);
 }
+// Threads of a k_field block: its elements' points in whole waves
+template <int Q>
+constexpr int sgs_block_threads() {
+  return (sgs_elems_per_block<Q>() * Q * Q * Q + 63) / 64 * 64;
+}
 
 // ---- quadrature-point bodies ----
 // Op::NU: components of the active interpolated input (0: none), Op::GRAD: its reference gradient is used,
 // Op::NU2: components of the passive interpolated input, Op::NV: output components, Op::OUTG: the output is gradient
-// test weights out[d * NV + c] (else values out[c]), Op::NST: LDS slots per element.
+// test weights out[d * NV + c] (else values out[c]).
 
 template <int VAR>
 struct VelocityGradientRHS {  // v[j*3+k] = wdetJ du_j/dx_k
   using Ctx                       = CeedMiNewtonianContext;
-  static constexpr int  NU = 5, NU2 = 0, NV = 9, NST = 27;
+  static constexpr int  NU = 5, NU2 = 0, NV = 9;
   static constexpr bool GRAD = true, OUTV = true, OUTG = false;
   __device__ static void qf(const FieldArgs &, const Ctx &ctx, int, int, const double qd[10], bool ok, const double (&u)[5], const double (&gu)[3][5],
                             const double (&)[1], double (&out)[9]) {
@@ -60,7 +66,7 @@ struct VelocityGradientRHS {  // v[j*3+k] = wdetJ du_j/dx_k
 
 struct AnisotropyRHS {  // v = wdetJ [KM(A_ij), delta]
   using Ctx                       = CeedMiNewtonianContext;
-  static constexpr int  NU = 0, NU2 = 0, NV = 7, NST = 21;
+  static constexpr int  NU = 0, NU2 = 0, NV = 7;
   static constexpr bool GRAD = false, OUTV = true, OUTG = false;
   __device__ static void qf(const FieldArgs &, const Ctx &, int, int, const double qd[10], bool ok, const double (&)[1], const double (&)[3][1],
                             const double (&)[1], double (&out)[7]) {
@@ -76,7 +82,7 @@ struct AnisotropyRHS {  // v = wdetJ [KM(A_ij), delta]
 template <int NC>
 struct MassN {  // v = wdetJ u
   using Ctx                       = CeedMiNewtonianContext;
-  static constexpr int  NU = NC, NU2 = 0, NV = NC, NST = 3 * NC;
+  static constexpr int  NU = NC, NU2 = 0, NV = NC;
   static constexpr bool GRAD = false, OUTV = true, OUTG = false;
   __device__ static void qf(const FieldArgs &, const Ctx &, int, int, const double qd[10], bool ok, const double (&u)[NC], const double (&)[3][NC],
                             const double (&)[1], double (&out)[NC]) {
@@ -89,7 +95,7 @@ struct MassN {  // v = wdetJ u
 template <int VAR>
 struct NodalSgsResidual {  // Grad_v[k][j] = -wdetJ (dXdx[k] . F_sgs[j])
   using Ctx                       = CeedMiNewtonianContext;
-  static constexpr int  NU = 5, NU2 = 6, NV = 5, NST = 20;
+  static constexpr int  NU = 5, NU2 = 6, NV = 5;
   static constexpr bool GRAD = false, OUTV = false, OUTG = true;
   __device__ static void qf(const FieldArgs &, const Ctx &ctx, int, int, const double qd[10], bool ok, const double (&u)[5], const double (&)[3][5],
                             const double (&km)[6], double (&out)[15]) {
@@ -111,7 +117,7 @@ struct NodalSgsResidual {  // Grad_v[k][j] = -wdetJ (dXdx[k] . F_sgs[j])
 template <int VAR>
 struct DiffFilterRHS {  // v0 = wdetJ Y, v1 = wdetJ u_i u_j (XX YY ZZ YZ XZ XY): one 11-component output
   using Ctx                       = CeedMiDiffFilterContext;
-  static constexpr int  NU = 5, NU2 = 0, NV = 11, NST = 33;
+  static constexpr int  NU = 5, NU2 = 0, NV = 11;
   static constexpr bool GRAD = false, OUTV = true, OUTG = false;
   __device__ static void qf(const FieldArgs &, const Ctx &ctx, int, int, const double qd[10], bool ok, const double (&u)[5], const double (&)[3][5],
                             const double (&)[1], double (&out)[11]) {
@@ -185,7 +191,7 @@ __device__ __forceinline__ void filter_alpha(const FieldArgs &a, const CeedMiDif
 template <int N>
 struct DiffFilterLHS {  // v = wdetJ q, Grad_v[k] = wdetJ (alpha (dXdx grad_x q))[k], every component alike
   using Ctx                       = CeedMiDiffFilterContext;
-  static constexpr int  NU = N, NU2 = 0, NV = N, NST = 4 * N;
+  static constexpr int  NU = N, NU2 = 0, NV = N;
   static constexpr bool GRAD = true, OUTV = true, OUTG = true;
   template <int Q>
   __device__ static void qfq(const FieldArgs &a, const Ctx &ctx, int e, int t, const double qd[10], bool ok, const double (&u)[N],
@@ -207,9 +213,8 @@ struct DiffFilterLHS {  // v = wdetJ q, Grad_v[k] = wdetJ (alpha (dXdx grad_x q)
   }
 };
 
-// Slot map of the stage: active input u -> 0..NU-1 (interpolation scratch NU..3NU-1), its reference gradient ->
-// NU + NU d + c, passive input -> 5..10 (interpolation scratch 11..16 and 5..10; only with NU = 5 and no gradient).
-// Outputs: values -> 0..NV-1 (transpose scratch up to 3NV), gradient test weights -> NV + NV d + c.
+// Slot map of the stage: active input u -> 0..NU-1, its reference gradient -> NU + NU d + c, passive input (without a
+// gradient) -> NU + c.  Outputs: values -> 0..NV-1, gradient test weights -> NV + NV d + c.
 // Op::qf(a, ctx, e, t, ...) or, for bodies that depend on Q, Op::qfq<Q>(...)
 template <class Op, int Q, class = void>
 struct HasQfq {
@@ -221,59 +226,73 @@ struct HasQfq<Op, Q, decltype((void)&Op::template qfq<Q>)> {
 };
 
 template <int P, int Q, class Op>
-__global__ void __launch_bounds__(sgs_elems_per_block<Q>() * Q * Q * Q) k_field(FieldArgs a, const typename Op::Ctx ctx) {
+__global__ void __launch_bounds__(sgs_block_threads<Q>()) k_field(FieldArgs a, const typename Op::Ctx ctx) {
   using Dm          = Dims<P, Q>;
   constexpr int EPB = sgs_elems_per_block<Q>();
   constexpr int Q3  = Dm::Q3;
+  constexpr int NT  = sgs_block_threads<Q>();
   constexpr int NU = Op::NU, NU2 = Op::NU2, NV = Op::NV;
   constexpr int NUX = NU > 0 ? NU : 1, NU2X = NU2 > 0 ? NU2 : 1, NOUT = (Op::OUTV ? NV : 0) + (Op::OUTG ? 3 * NV : 0);
-  constexpr int G0  = Op::OUTV ? NV : 0;  // first gradient-weight entry of out[]
-  static_assert(NU2 == 0 || (NU == 5 && !Op::GRAD && NU2 == 6), "passive input slot map assumes a 5-component value input");
-  static_assert(Op::NST >= 3 * NU && Op::NST >= (Op::GRAD ? 4 * NU : 0) && Op::NST >= (NU2 ? 17 : 0), "stage too small for the inputs");
-  static_assert(Op::NST >= (Op::OUTG ? 4 * NV : 3 * NV), "stage too small for the output transpose");
+  constexpr int G0   = Op::OUTV ? NV : 0;  // first gradient-weight entry of out[]
+  constexpr int NIN  = NU * (Op::GRAD ? 4 : 1) + NU2, NST = std::max(NIN, NV * (Op::OUTG ? 4 : 1));
+  static_assert(NU2 == 0 || !Op::GRAD, "the passive input's slots follow the active input's values");
   static_assert(Op::OUTV || Op::OUTG, "no output");
   static_assert(Dm::P3 <= Q3, "P <= Q is required");
-  __shared__ double sB[Q * P], sDc[Q * Q];
-  __shared__ double sX[EPB][Op::NST][Q3];
-  for (int i = threadIdx.x; i < Q * P; i += blockDim.x) sB[i] = a.bt.B[i];
-  for (int i = threadIdx.x; i < Q * Q; i += blockDim.x) sDc[i] = a.bt.Dc[i];
-  const int       le = threadIdx.x / Q3, t = threadIdx.x % Q3;
-  const bool      nd = t < Dm::P3;
-  double(*X)[Q3]     = sX[le];
+  constexpr bool LINES = !(P == 4 && Q == 4);
+  using Lines          = basis3::LineStage<P, Q, EPB, NST>;
+  constexpr int SLOT   = LINES ? Lines::kSlot : Q3;
+  static_assert(!LINES || Lines::NT == NT, "block size");
+  __shared__ double sB[LINES ? 1 : Q * P], sDc[LINES ? 1 : Q * Q], sG[LINES ? 1 : Q * P];
+  __shared__ double sX[EPB][NST][SLOT];
+  if constexpr (!LINES) {
+    for (int i = threadIdx.x; i < Q * P; i += blockDim.x) sB[i] = a.bt.B[i];
+    for (int i = threadIdx.x; i < Q * Q; i += blockDim.x) sDc[i] = a.bt.Dc[i];
+    for (int i = threadIdx.x; i < Q * P; i += blockDim.x) {  // G = Dc B
+      double g = 0;
+      for (int m = 0; m < Q; m++) g += a.bt.Dc[i / P * Q + m] * a.bt.B[m * P + i % P];
+      sG[i] = g;
+    }
+    __syncthreads();
+  }
+  // threads past the elements' points only take part in the lines
+  const bool      act = NT == EPB * Q3 || threadIdx.x < EPB * Q3;
+  const int       le = act ? threadIdx.x / Q3 : 0, t = act ? threadIdx.x % Q3 : 0;
+  const bool      nd = act && t < Dm::P3;
+  double(*X)[SLOT]   = sX[le];
   const long long nbatch = ((long long)a.nelem + EPB - 1) / EPB;
 
   for (long long bt = blockIdx.x; bt < nbatch; bt += gridDim.x) {
     const long long e_    = bt * EPB + le;
-    const bool      ok    = e_ < a.nelem;
+    const bool      ok    = act && e_ < a.nelem;
     const int       e     = ok ? (int)e_ : 0;
     const long long enode = (long long)e * Dm::P3 + t;
-    basis3::Stage<P, Q> st(sB, sDc, nullptr, X, t);
+    double          un[NUX], kn[NU2X];
     if constexpr (NU > 0) {
-      double un[NUX];
-      if (ok && nd) {
-        const int off = a.in_offsets[enode];
+      const int off = ok && nd ? a.in_offsets[enode] : 0;
 #pragma unroll
-        for (int c = 0; c < NU; c++) un[c] = a.u[off + c * a.in_comp_stride];
-      } else {
-#pragma unroll
-        for (int c = 0; c < NU; c++) un[c] = 0.0;
-      }
-      st.template interp<NUX>(un, NU, 2 * NU, 0);
-      if constexpr (Op::GRAD) st.template grad<NUX>(0, NU);
-    } else {
-      __syncthreads();  // the previous batch's transpose may still read the stage
+      for (int c = 0; c < NU; c++) un[c] = ok && nd ? a.u[off + c * a.in_comp_stride] : 0.0;
     }
     if constexpr (NU2 > 0) {
-      double kn[NU2X];
-      if (ok && nd) {
-        const int off = a.in2_offsets[enode];
+      const int off = ok && nd ? a.in2_offsets[enode] : 0;
 #pragma unroll
-        for (int c = 0; c < NU2; c++) kn[c] = a.u2[off + c * a.in2_comp_stride];
-      } else {
+      for (int c = 0; c < NU2; c++) kn[c] = ok && nd ? a.u2[off + c * a.in2_comp_stride] : 0.0;
+    }
+    if constexpr (LINES) {
+      if (nd) {
+        const int at = Lines::node(t);
+        if constexpr (NU > 0)
 #pragma unroll
-        for (int c = 0; c < NU2; c++) kn[c] = 0.0;
+          for (int c = 0; c < NU; c++) X[c][at] = un[c];
+        if constexpr (NU2 > 0)
+#pragma unroll
+          for (int c = 0; c < NU2; c++) X[NU + c][at] = kn[c];
       }
-      st.template interp<NU2X>(kn, 11, 5, 5);
+      if constexpr (NU + NU2 > 0) Lines(a.bt.B, a.bt.Dc, sX, threadIdx.x).template interp_grad<NU + NU2, Op::GRAD>(0, NU);
+    } else {
+      basis3::StageMF st(sB, sDc, sG, X, t);
+      if constexpr (Op::GRAD) st.template interp_grad<NUX>(un, 0, NU);
+      else if constexpr (NU > 0) st.template interp<NUX>(un, 0);
+      if constexpr (NU2 > 0) st.template interp<NU2X>(kn, NU);
     }
     double qd[10];
 #pragma unroll
@@ -286,22 +305,31 @@ __global__ void __launch_bounds__(sgs_elems_per_block<Q>() * Q * Q * Q) k_field(
       for (int d = 0; d < 3; d++) gu[d][c] = Op::GRAD ? X[NU + NU * d + c][t] : 0.0;
     }
 #pragma unroll
-    for (int c = 0; c < NU2X; c++) u2[c] = NU2 > 0 ? X[5 + c][t] : 0.0;
+    for (int c = 0; c < NU2X; c++) u2[c] = NU2 > 0 ? X[NU + c][t] : 0.0;
     if constexpr (HasQfq<Op, Q>::value) Op::template qfq<Q>(a, ctx, e, t, qd, ok, u, gu, u2, out);
     else Op::qf(a, ctx, e, t, qd, ok, u, gu, u2, out);
-    __syncthreads();  // other threads' last interpolation pass may still read the stage
+    if (act) {
+      if constexpr (Op::OUTV) {
+#pragma unroll
+        for (int c = 0; c < NV; c++) X[c][t] = out[c];
+      }
+      if constexpr (Op::OUTG) {
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+#pragma unroll
+          for (int c = 0; c < NV; c++) X[NV + NV * d + c][t] = out[G0 + d * NV + c];
+      }
+    }
     double r[NV];
-    if constexpr (Op::OUTV) {
+    if constexpr (LINES) {
+      Lines(a.bt.B, a.bt.Dc, sX, threadIdx.x).template transpose<NV, Op::OUTV, Op::OUTG>(0, NV);
+      const int at = Lines::node(t);
 #pragma unroll
-      for (int c = 0; c < NV; c++) X[c][t] = out[c];
+      for (int c = 0; c < NV; c++) r[c] = X[c][at];
+      __syncthreads();  // without an input (NU = 0) the next batch's outputs go to slots that other threads still read
+    } else {
+      basis3::StageMF(sB, sDc, sG, X, t).template transpose<NV, Op::OUTV, Op::OUTG>(0, NV, r);
     }
-    if constexpr (Op::OUTG) {
-#pragma unroll
-      for (int d = 0; d < 3; d++)
-#pragma unroll
-        for (int c = 0; c < NV; c++) X[NV + NV * d + c][t] = out[G0 + d * NV + c];
-    }
-    st.template transpose<NV, Op::OUTV, Op::OUTG>(0, NV, r);
     if (ok && nd) {
       if (a.ev) {  // two-pass scatter: node-sorted element-node contributions, summed per node by launch_node_gather
         double *dst = a.ev + (long long)a.perm[enode] * NV;
@@ -545,7 +573,7 @@ template <int P, int Q, class Op>
 hipError_t launch_field_pq(const FieldArgs &a, const typename Op::Ctx &ctx, hipStream_t s) {
   if (a.nelem <= 0) return hipSuccess;
   constexpr int EPB   = sgs_elems_per_block<Q>();
-  constexpr int block = EPB * Q * Q * Q;
+  constexpr int block = sgs_block_threads<Q>();
   auto          kern  = k_field<P, Q, Op>;
   const int     grid  = grid_for_batches(kern, block, ((long long)a.nelem + EPB - 1) / EPB);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, s, a, ctx);

@@ -64,20 +64,11 @@ __device__ __forceinline__ void stage_coords_async(const VolumeArgs &a, long lon
   }
 }
 
-// The interpolated inputs of every quadrature point and the quadrature-point outputs are staged in LDS (X), one slot
-// per (field component, point).  The basis stages treat the five components of a field together (basis3::Stage), so
-// a 1D coefficient row is read once per pass and five independent contractions are in flight; the quadrature-point
-// body then runs with only its own registers live.
-//
-// Slot map of the stage: u -> 0..4, reference gradient of u -> 5 + 5 d + c (kGrad), u2 -> 20..24 (kGrad) or 5..9;
-// outputs: v -> 0..4, gradient test weights -> 5 + 5 d + c.  Interpolation scratch is chosen from the slots that are
-// not live at that point.
 // Asynchronous copy of the quadrature data of element batch bt (EPB consecutive elements, [elem][10][Q^3] and
 // contiguous) into sQD through the LDS-DMA path (global_load_lds_dwordx4, 16 bytes per lane): no registers are held
 // while the loads are in flight.  The caller waits with s_waitcnt vmcnt(0) and a barrier before reading sQD.
-template <int EPB, int Q3>
+template <int EPB, int Q3, int NT>
 __device__ __forceinline__ void stage_qdata_async(const VolumeArgs &a, long long bt, double (*sQD)[10][Q3]) {
-  constexpr int   NT   = EPB * Q3;                       // threads of the block
   constexpr int   NB   = EPB * 10 * Q3 * 8;              // bytes of a full batch
   constexpr int   NCH  = (NB + NT * 16 - 1) / (NT * 16);  // copy instructions per thread
   const long long e0   = bt * EPB;
@@ -97,13 +88,11 @@ __device__ __forceinline__ void stage_qdata_async(const VolumeArgs &a, long long
 }
 
 // The interpolated inputs of every quadrature point and the quadrature-point outputs are staged in LDS (X), one slot
-// per (field component, point).  The basis stages treat the five components of a field together (basis3::Stage), so
-// a 1D coefficient row is read once per pass and five independent contractions are in flight; the quadrature-point
-// body then runs with only its own registers live.
+// per (field component, point).  The basis stages treat the components of the fields together, so that independent
+// contractions are in flight; the quadrature-point body then runs with only its own registers live.
 //
 // Slot map of the stage: u -> 0..4, reference gradient of u -> 5 + 5 d + c (kGrad), u2 -> 20..24 (kGrad) or 5..9;
-// outputs: v -> 0..4, gradient test weights -> 5 + 5 d + c.  Interpolation scratch is chosen from the slots that are
-// not live at that point.
+// outputs: v -> 0..4, gradient test weights -> 5 + 5 d + c.
 //
 // Software pipeline over a block's element batches: the next batch's quadrature data is copied into sQD by LDS DMA
 // while the current batch's quadrature-point body runs, and its node values are loaded into registers while the
@@ -112,20 +101,22 @@ __device__ __forceinline__ void stage_qdata_async(const VolumeArgs &a, long long
 // With GEO the quadrature data is recomputed from the element's vertex coordinates (192 bytes per element, staged by
 // the same DMA path) instead of read (80 bytes per quadrature point).
 template <int P, int Q, class Op, bool GEO>
-__global__ void __launch_bounds__(elems_per_block<Q>() * Q * Q * Q, 2) k_volume(VolumeArgs a, const CeedMiNewtonianContext ctx) {
+__global__ void __launch_bounds__(block_threads<Q>(), 2) k_volume(VolumeArgs a, const CeedMiNewtonianContext ctx) {
   using Dm           = Dims<P, Q>;
   constexpr int EPB  = elems_per_block<Q>();
   constexpr int Q3   = Dm::Q3;
+  constexpr int NT   = block_threads<Q>();
   constexpr int NIN  = 5 + (Op::kGrad ? 15 : 0) + (Op::kIn2 ? 5 : 0);
-  constexpr int NOUT = Op::kScatter ? 20 : 1;
-  constexpr int NST0 = NIN > NOUT ? NIN : NOUT;
-  constexpr int NST  = NST0 > 15 ? NST0 : 15;            // interpolation scratch needs slots up to 14
+  constexpr int NOUT = Op::kScatter ? (Op::kOutG ? 20 : 5) : 1;
+  constexpr int NST  = NIN > NOUT ? NIN : NOUT;
   constexpr int U2   = Op::kGrad ? 20 : 5;               // slot of u2
-  constexpr int SU2  = Op::kGrad ? 0 : 10;               // scratch of the u2 interpolation
-  constexpr int SU   = (Op::kIn2 && !Op::kGrad) ? 10 : 5;  // scratch of the u interpolation
-  static_assert(!Op::kIn2 || Op::kGrad || NST >= 20, "stage too small for the u2 scratch");
-  __shared__ double                 sB[Q * P], sDc[Q * Q], sG[Q * P];
-  __shared__ double                 sX[EPB][NST][Q3];
+  // the 4 x 4 x 4 element has its own stages (whole wave per element); every other one a line per thread
+  constexpr bool LINES = !(P == 4 && Q == 4);
+  using Lines          = basis3::LineStage<P, Q, EPB, NST>;
+  constexpr int SLOT   = LINES ? Lines::kSlot : Q3;
+  static_assert(!LINES || Lines::NT == NT, "block size");
+  __shared__ double                 sB[LINES ? 1 : Q * P], sDc[LINES ? 1 : Q * Q], sG[LINES ? 1 : Q * P];
+  __shared__ double                 sX[EPB][NST][SLOT];
   // quadrature data staged through LDS by DMA (Op::kStageQData) or read from global memory at the point body
   constexpr bool                    SQ = Op::kStageQData && !GEO;
   __shared__ __align__(16) double   sQD[SQ ? EPB : 1][10][SQ ? Q3 : 1];
@@ -134,34 +125,32 @@ __global__ void __launch_bounds__(elems_per_block<Q>() * Q * Q * Q, 2) k_volume(
   if constexpr (GEO)
     for (int i = threadIdx.x; i < 5 * Q; i += blockDim.x) sGT[i] = a.gtab[i];
   static_assert(Dm::P3 <= Q3, "P <= Q is required");
-  using Stage = typename StageFor<P, Q, ZCross<Op>::value>::type;
-  load_tables<P, Q>(a.bt, sB, sDc, sG);
-  const int           le = threadIdx.x / Q3, t = threadIdx.x % Q3;
-  const bool          nd = t < Dm::P3;
-  double(*X)[Q3]         = sX[le];
-  const BatchRange br    = batch_range(((long long)a.nelem + EPB - 1) / EPB);
-  const int        cs    = a.comp_stride;
+  if constexpr (!LINES) load_tables<P, Q>(a.bt, sB, sDc, sG);
+  // threads past the elements' points (the block is whole waves) only take part in the lines and the copies
+  const bool           act = NT == EPB * Q3 || threadIdx.x < EPB * Q3;
+  const int            le = act ? threadIdx.x / Q3 : 0, t = act ? threadIdx.x % Q3 : 0;
+  const bool           nd = act && t < Dm::P3;
+  double(*X)[SLOT]        = sX[le];
+  const BatchRange br     = batch_range(((long long)a.nelem + EPB - 1) / EPB);
+  const int        cs     = a.comp_stride;
 
   // prologue: quadrature data and node values of the first batch
   int    off = 0;
   double un[5] = {0, 0, 0, 0, 0}, u2n[5] = {0, 0, 0, 0, 0};
   if (br.first < br.end) {
-    if constexpr (SQ) stage_qdata_async<EPB, Q3>(a, br.first, sQD);
+    if constexpr (SQ) stage_qdata_async<EPB, Q3, NT>(a, br.first, sQD);
     if constexpr (GEO) stage_coords_async<EPB>(a, br.first, sXE);
     const long long e_ = br.first * EPB + le;
     if (nd && e_ < a.nelem) {
       off = a.offsets[e_ * Dm::P3 + t];
-#pragma unroll
-      for (int c = 0; c < 5; c++) un[c] = a.u[off + c * cs];
-      if constexpr (Op::kIn2)
-#pragma unroll
-        for (int c = 0; c < 5; c++) u2n[c] = a.u2[off + c * cs];
+      load_node(a.u, off, cs, un);
+      if constexpr (Op::kIn2) load_node(a.u2, off, cs, u2n);
     }
   }
 
   for (long long bt = br.first; bt < br.end; bt += br.stride) {
     const long long e_   = bt * EPB + le;
-    const bool      ok   = e_ < a.nelem;
+    const bool      ok   = act && e_ < a.nelem;
     const int       e    = ok ? (int)e_ : 0;
     const long long btn  = bt + br.stride;
     const bool      more = btn < br.end;
@@ -172,12 +161,26 @@ __global__ void __launch_bounds__(elems_per_block<Q>() * Q * Q * Q, 2) k_volume(
     // The basis stages index LDS with per-thread addresses derived from t.  An opaque copy of t per phase keeps the
     // compiler from hoisting those addresses out of the loop, where they would stay live (or spill) across the
     // quadrature-point body.
-    int tb = t;
-    asm volatile("" : "+v"(tb));
-    Stage st(sB, sDc, sG, X, tb);
-    if constexpr (Op::kIn2) st.template interp<5>(u2n, SU2, SU2 + 5, U2);
-    if constexpr (Op::kGrad) st.template interp_grad<5>(un, SU, SU + 5, 0, 5);
-    else st.template interp<5>(un, SU, SU + 5, 0);
+    if constexpr (LINES) {
+      int tb = threadIdx.x;
+      asm volatile("" : "+v"(tb));
+      if (nd) {
+        const int at = Lines::node(t);
+#pragma unroll
+        for (int c = 0; c < 5; c++) {
+          X[c][at] = un[c];
+          if constexpr (Op::kIn2) X[U2 + c][at] = u2n[c];
+        }
+      }
+      Lines(a.bt.B, a.bt.Dc, sX, tb).template interp_grad<5, Op::kGrad, Op::kIn2 ? 5 : 0>(0, 5, U2);
+    } else {
+      int tb = t;
+      asm volatile("" : "+v"(tb));
+      typename StageFor<ZCross<Op>::value>::type st(sB, sDc, sG, X, tb);
+      if constexpr (Op::kIn2) st.template interp<5>(u2n, U2);
+      if constexpr (Op::kGrad) st.template interp_grad<5>(un, 0, 5);
+      else st.template interp<5>(un, 0);
+    }
     int off_next = 0;
     {
       double qd[10], u[5], gu[3][5], u2[5], v[5], gw[3][5];
@@ -187,7 +190,7 @@ __global__ void __launch_bounds__(elems_per_block<Q>() * Q * Q * Q, 2) k_volume(
 #pragma unroll
         for (int k = 0; k < 10; k++) qd[k] = sQD[le][k][t];
         __syncthreads();  // all of sQD has been read: the next batch's copy may overwrite it
-        if (more) stage_qdata_async<EPB, Q3>(a, btn, sQD);
+        if (more) stage_qdata_async<EPB, Q3, NT>(a, btn, sQD);
       } else if constexpr (GEO) {
         __builtin_amdgcn_s_waitcnt(0);  // this batch's vertex coordinates have landed in sXE
         __syncthreads();
@@ -208,13 +211,15 @@ __global__ void __launch_bounds__(elems_per_block<Q>() * Q * Q * Q, 2) k_volume(
       }
       Op::template qf<Q>(a, ctx, e, t, ok, qd, u, gu, u2, v, gw);
       if constexpr (Op::kScatter) {
-        __syncthreads();  // other threads' gradient passes read slots 0..4
+        if constexpr (!LINES) __syncthreads();  // other threads' gradient passes read slots 0..4
+        if (act) {
 #pragma unroll
-        for (int c = 0; c < 5; c++) {
-          if (Op::kOutV) X[c][t] = v[c];
-          if (Op::kOutG)
+          for (int c = 0; c < 5; c++) {
+            if (Op::kOutV) X[c][t] = v[c];
+            if (Op::kOutG)
 #pragma unroll
-            for (int d = 0; d < 3; d++) X[5 + 5 * d + c][t] = gw[d][c];
+              for (int d = 0; d < 3; d++) X[5 + 5 * d + c][t] = gw[d][c];
+          }
         }
       }
     }
@@ -225,29 +230,38 @@ __global__ void __launch_bounds__(elems_per_block<Q>() * Q * Q * Q, 2) k_volume(
     const int off_cur = off;
     const int slot    = (a.perm && ok && nd) ? a.perm[enode] : 0;
     if (more) {
-      const bool ld = nd && okn;
+      if (nd && okn) {
+        load_node(a.u, off_next, cs, un);
+        if constexpr (Op::kIn2) load_node(a.u2, off_next, cs, u2n);
+      } else {
 #pragma unroll
-      for (int c = 0; c < 5; c++) un[c] = ld ? a.u[off_next + c * cs] : 0.0;
-      if constexpr (Op::kIn2)
-#pragma unroll
-        for (int c = 0; c < 5; c++) u2n[c] = ld ? a.u2[off_next + c * cs] : 0.0;
+        for (int c = 0; c < 5; c++) un[c] = u2n[c] = 0.0;
+      }
       off = off_next;
     }
     if constexpr (Op::kScatter) {
-      int tt = t;
-      asm volatile("" : "+v"(tt));
-      Stage               sto(sB, sDc, sG, X, tt);
-      double              r[5];
-      sto.template transpose<5, Op::kOutV, Op::kOutG>(0, 5, r);
+      double r[5];
+      if constexpr (LINES) {
+        int tt = threadIdx.x;
+        asm volatile("" : "+v"(tt));
+        Lines(a.bt.B, a.bt.Dc, sX, tt).template transpose<5, Op::kOutV, Op::kOutG>(0, 5);
+        // read back by the thread that writes the next batch's node values there
+        const int at = Lines::node(t);
+#pragma unroll
+        for (int c = 0; c < 5; c++) r[c] = X[c][at];
+      } else {
+        int tt = t;
+        asm volatile("" : "+v"(tt));
+        typename StageFor<ZCross<Op>::value>::type sto(sB, sDc, sG, X, tt);
+        sto.template transpose<5, Op::kOutV, Op::kOutG>(0, 5, r);
+      }
       if (ok && nd) {
         if (a.ev32) {  // two-pass scatter in FP32: element order
           float *dst = a.ev32 + enode * 5;
 #pragma unroll
           for (int c = 0; c < 5; c++) dst[c] = (float)r[c];
         } else if (a.ev) {  // two-pass scatter: element-node contributions, summed per node by a second kernel
-          double *dst = a.ev + (a.perm ? (long long)slot : enode) * 5;
-#pragma unroll
-          for (int c = 0; c < 5; c++) dst[c] = r[c];
+          store_node5(a.ev + (a.perm ? (long long)slot : enode) * 5, r);
         } else {
 #pragma unroll
           for (int c = 0; c < 5; c++) atomicAdd(&a.v[off_cur + c * cs], r[c]);
@@ -276,7 +290,7 @@ struct RecomputeAt<nsop::IJacobian<VAR, double>, 4> : std::true_type {};
 template <int P, int Q, class Op>
 hipError_t launch_op(const VolumeArgs &a, const CeedMiNewtonianContext &ctx, hipStream_t stream) {
   constexpr int EPB   = elems_per_block<Q>();
-  const int     block = EPB * Q * Q * Q;
+  const int     block = block_threads<Q>();
   auto          k     = k_volume<P, Q, Op, false>;
   if constexpr (P == Q && RecomputeAt<Op, Q>::value)
     if (a.xe) k = k_volume<P, Q, Op, true>;

@@ -20,6 +20,12 @@ constexpr int elems_per_block() {
   return (Q * Q * Q >= 64) ? 1 : 64 / (Q * Q * Q);
 }
 
+// Threads of a block: the quadrature points of its elements, in whole waves
+template <int Q>
+constexpr int block_threads() {
+  return (elems_per_block<Q>() * Q * Q * Q + 63) / 64 * 64;
+}
+
 // Element-batch schedule of the persistent blocks.  The workgroups of a dispatch are distributed round-robin over
 // the 8 XCDs of an MI355X, each with its own L2 (block b runs on XCD b % 8).  Each XCD gets one contiguous range of
 // element batches, which its blocks sweep together, so the nodes that neighbouring elements share are fetched into
@@ -39,19 +45,19 @@ __device__ __forceinline__ BatchRange batch_range(long long nbatch) {
   return {lo + j, hi, G / kNumXcd};
 }
 
-// The basis stage of the fused kernel: for the 4 x 4 x 4 element the x and z passes run on the FP64 matrix cores and the
-// y passes across lanes (basis3::StageMF), except for ops with Op::kZCrossLane (the FP32 Jacobian, measured faster with
-// all passes across lanes); otherwise sum factorization through LDS (basis3::Stage, ZX: z passes across lanes)
-template <int P, int Q, bool ZX>
+// The basis stage of the fused kernel on the 4 x 4 x 4 element: the x and z passes on the FP64 matrix cores and the y passes
+// across lanes (basis3::StageMF), except for ops with Op::kZCrossLane (the FP32 Jacobian, measured faster with all passes
+// across lanes)
+template <bool ZX>
 struct StageFor {
-  using type = basis3::Stage<P, Q, ZX>;
-};
-template <>
-struct StageFor<4, 4, false> {
   using type = basis3::StageMF;
 };
+template <>
+struct StageFor<true> {
+  using type = basis3::StageX;
+};
 
-// Op::kZCrossLane selects the basis stage whose z passes also run across lanes (basis3::Stage's ZX); default off
+// Op::kZCrossLane selects the basis stage whose z passes also run across lanes; default off
 template <class Op, class = void>
 struct ZCross {
   static constexpr bool value = false;
@@ -60,6 +66,29 @@ template <class Op>
 struct ZCross<Op, std::void_t<decltype(Op::kZCrossLane)>> {
   static constexpr bool value = Op::kZCrossLane;
 };
+
+// The five components of a node of an interleaved vector as two 16-byte accesses and one of 8 bytes (a node starts on any
+// multiple of 8 bytes, which the global memory instructions allow): 3 accesses and one address instead of 5 and 5.
+// Measured: residual and Jacobian pair at 48^3 p=2 600.9 -> 590.2 us, at 32^3 p=3 341.0 -> 339.7 us.
+using double2a8 = double __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ void load_node5(const double *p, double (&v)[5]) {
+  const double2a8 a = *(const double2a8 *)p, b = *(const double2a8 *)(p + 2);
+  v[0] = a.x, v[1] = a.y, v[2] = b.x, v[3] = b.y, v[4] = p[4];
+}
+__device__ __forceinline__ void store_node5(double *p, const double (&v)[5]) {
+  *(double2a8 *)p       = double2a8{v[0], v[1]};
+  *(double2a8 *)(p + 2) = double2a8{v[2], v[3]};
+  p[4]                  = v[4];
+}
+// Node values of an L-vector at the offset of component 0
+__device__ __forceinline__ void load_node(const double *u, int off, int comp_stride, double (&v)[5]) {
+  if (comp_stride == 1) {
+    load_node5(u + off, v);
+  } else {
+#pragma unroll
+    for (int c = 0; c < 5; c++) v[c] = u[off + c * comp_stride];
+  }
+}
 
 template <int P, int Q>
 __device__ __forceinline__ void load_tables(const BasisTables &bt, double *sB, double *sDc) {
