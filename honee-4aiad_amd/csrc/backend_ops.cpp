@@ -853,6 +853,19 @@ bool op_plan_overwrites(CeedOperator op, CeedVector out) {
     case QfKind::MassNewtonian:
     case QfKind::Mass5:
       break;
+    case QfKind::VelocityGradientRHS:
+    case QfKind::AnisotropyRHS:
+    case QfKind::MassN:
+    case QfKind::NodalSgsResidual:
+    case QfKind::DiffFilterRHS:
+    case QfKind::DiffFilterLHS:
+    case QfKind::SgsNodal:
+    case QfKind::SgsTrainingNodal: {  // rows of consecutive components (the filter's 5 + 6 outputs are rows of 11)
+      const CeedElemRestriction r = p->r_out;
+      const int                 n = p->ncomp_out ? p->ncomp_out : r->num_comp;
+      if (rstr_transpose_map(r)) return false;
+      return r->comp_stride == 1 && r->t_stride == n && (CeedSize)r->t_nrows * n == r->l_size && out->length == r->l_size;
+    }
     default:
       return false;
   }
@@ -973,6 +986,7 @@ static int sgs_field_apply(CeedOperator op, OpPlan *p, CeedVector in, CeedVector
     a.index           = r->d_t_index;
     a.row_offset      = r->d_t_offset;
     a.out_comp_stride = r->comp_stride;
+    a.overwrite       = overwrite;
     MI_CALL(vec_device_write(out, &a.v, true));
     MI_CALL(rstr_device_offsets(p->r_aux, &a.q_offsets));
     MI_CALL(rstr_device_offsets(p->r_in2, &a.p_offsets));
@@ -1006,6 +1020,7 @@ static int sgs_field_apply(CeedOperator op, OpPlan *p, CeedVector in, CeedVector
     a.index      = r->d_t_index;
     a.row_offset = r->d_t_offset;
     a.out_comp_stride = r->comp_stride;
+    a.overwrite       = overwrite;
     MI_CALL(vec_device_write(out, &a.v, true));
     MI_CALL(rstr_device_offsets(p->r_aux, &a.q_offsets));
     MI_CALL(rstr_device_offsets(p->r_q, &a.g_offsets));

@@ -8,6 +8,8 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
+#include <cmath>
 #include <string>
 
 #include "ceed_impl.hpp"
@@ -250,6 +252,8 @@ extern "C" int CeedDestroy(Ceed *ceed) {
   for (hipEvent_t e : c->event_pool) (void)hipEventDestroy(e);
   if (c->d_scratch) (void)hipFree(c->d_scratch);
   if (c->h_scratch) (void)hipHostFree(c->h_scratch);
+  if (c->d_cg) (void)hipFree(c->d_cg);
+  if (c->h_cg) (void)hipHostFree(c->h_cg);
   if (c->d_work) (void)hipFree(c->d_work);
   delete c;
   *ceed = nullptr;
@@ -666,6 +670,73 @@ extern "C" int CeedMiVectorDot(CeedVector x, CeedVector y, double *result) {
   return CEED_ERROR_SUCCESS;
 }
 
+// Conjugate gradients with a Jacobi preconditioner.  The scalars stay on the device: every kernel of an iteration sums the
+// block partials that the one before left (in a fixed order), so that the host reads one value an iteration, r.z, which
+// the last kernel also stores into mapped host memory.  The next iteration's operator apply and p.Ap, which change nothing
+// that is returned, are launched before the host waits for that value.
+extern "C" int CeedMiJacobiCg(CeedOperator op, CeedVector dinv, CeedVector rhs, CeedVector x, CeedVector r, CeedVector p, CeedVector Ap,
+                              CeedScalar rtol, CeedScalar atol, CeedInt max_it, CeedInt *iterations) {
+  Ceed           ceed = op->ceed;
+  hipStream_t    s    = ceed->stream;
+  const CeedSize n    = rhs->length;
+  for (CeedVector v : {dinv, x, r, p, Ap})
+    if (v->length != n) return MI_ERR(ceed, CEED_ERROR_DIMENSION, "vector lengths differ");
+  if (!ceed->d_cg) {
+    MI_HIP(ceed, hipMalloc((void **)&ceed->d_cg, sizeof(double) * kCgScratch));
+    MI_HIP(ceed, hipHostMalloc((void **)&ceed->h_cg, sizeof(double) * 2, hipHostMallocMapped | hipHostMallocCoherent));
+    MI_HIP(ceed, hipHostGetDevicePointer((void **)&ceed->g_cg, ceed->h_cg, 0));
+  }
+  auto              *h_seq = reinterpret_cast<unsigned long long *>(ceed->h_cg + 1);
+  unsigned long long seq   = 0;
+  __atomic_store_n(h_seq, 0ull, __ATOMIC_RELEASE);
+  auto published = [&](double *value) -> int {  // poll for up to 2 ms, then wait on the stream
+    const auto t0 = std::chrono::steady_clock::now();
+    while (__atomic_load_n(h_seq, __ATOMIC_ACQUIRE) != seq)
+      if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+        MI_HIP(ceed, hipStreamSynchronize(s));
+        if (__atomic_load_n(h_seq, __ATOMIC_ACQUIRE) != seq) return MI_ERR(ceed, CEED_ERROR_BACKEND, "reduction result not published");
+        break;
+      }
+    *value = ceed->h_cg[0];
+    return 0;
+  };
+  CgArgs a{};
+  a.n = n;
+  MI_CALL(vec_device_read(dinv, &a.dinv));
+  MI_CALL(vec_device_read(rhs, &a.rhs));
+  MI_CALL(vec_device_write(x, &a.x, false));
+  MI_CALL(vec_device_write(r, &a.r, false));
+  MI_CALL(vec_device_write(p, &a.p, false));
+  a.scratch = ceed->d_cg;
+  a.h       = ceed->g_cg;
+  a.flag    = reinterpret_cast<unsigned long long *>(ceed->g_cg + 1);
+  a.seq     = ++seq;
+  MI_HIP(ceed, launch_cg_start(a, s));
+  double rz;
+  int    its = 0;
+  MI_CALL(published(&rz));
+  const double ttol    = std::max(rtol * std::sqrt(std::fabs(rz)), atol);
+  bool         applied = false;  // Ap and the partials of p.Ap belong to the present p
+  while (std::sqrt(std::fabs(rz)) > ttol && its < max_it) {
+    auto apply = [&]() -> int {
+      MI_CALL(CeedOperatorApply(op, p, Ap, CEED_REQUEST_IMMEDIATE));
+      MI_CALL(vec_device_read(Ap, &a.ap));
+      MI_HIP(ceed, launch_cg_dot(a, s));
+      return 0;
+    };
+    if (!applied) MI_CALL(apply());
+    a.seq = ++seq;
+    a.odd = its & 1;
+    MI_HIP(ceed, launch_cg_update(a, s));
+    its++;
+    applied = its < max_it;
+    if (applied) MI_CALL(apply());
+    MI_CALL(published(&rz));
+  }
+  *iterations = its;
+  return CEED_ERROR_SUCCESS;
+}
+
 extern "C" int CeedVectorScale(CeedVector x, CeedScalar alpha) {
   double *d;
   MI_CALL(vec_device_write(x, &d, true));
@@ -838,6 +909,9 @@ int rstr_transpose_map(CeedElemRestriction r) {
   for (size_t j = 0; j < n; j++) perm[index[j]] = (int)j;
   r->t_nrows      = (int)toff.size();
   r->t_covers_all = (CeedSize)r->t_nrows * r->num_comp == r->l_size;
+  r->t_stride     = toff.size() > 1 ? toff[1] : r->num_comp;
+  for (size_t k = 0; k < toff.size() && r->t_stride; k++)
+    if ((long long)toff[k] != (long long)k * r->t_stride) r->t_stride = 0;
   const size_t nr = std::max<size_t>(toff.size(), 1);
   MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_rowptr, sizeof(int) * (nr + 1)));
   MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_perm, sizeof(int) * std::max<size_t>(n, 1)));

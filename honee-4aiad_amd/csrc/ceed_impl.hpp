@@ -37,6 +37,8 @@ struct Ceed_private {
   double                                  *d_scratch = nullptr;  // reduction scratch (norms)
   double                                  *h_scratch = nullptr;
   int                                      scratch_len = 0;
+  double             *h_cg = nullptr, *g_cg = nullptr;  // mapped host memory of CeedMiJacobiCg (host and device address)
+  double             *d_cg = nullptr;                   // its block partials and scalars
   double *d_fixed = nullptr;  // this device's copy of the fixed E-vector scratch (CeedMiOperatorApplyNoAlloc), or null
 };
 
@@ -84,6 +86,7 @@ struct CeedElemRestriction_private {
   // slot t_perm[i]; the slots of L-vector row k (offset t_offset[k]) are t_rowptr[k]..t_rowptr[k+1]-1, ordered by i
   int                  t_nrows      = 0;
   bool                 t_covers_all = false;  // the rows cover every L-vector entry
+  int                  t_stride     = 0;      // row k's offset is k t_stride (0: no such stride)
   int                 *d_t_rowptr = nullptr, *d_t_perm = nullptr, *d_t_offset = nullptr;
   int                 *d_t_index = nullptr;  // element node of each slot (inverse of t_perm)
 };

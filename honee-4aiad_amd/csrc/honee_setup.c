@@ -77,8 +77,8 @@ struct HoneeMiProblem_ {
   int                   filter_enabled, filter_pc_ready, train_enabled, filter_its;
   double                filter_rtol, filter_atol;
   int                   filter_max_it;
-  CeedElemRestriction   elem_restr_filter[2], elem_restr_aniso_col, elem_restr_train;
-  CeedBasis             basis_filter[2];
+  CeedElemRestriction   elem_restr_filter[3], elem_restr_aniso_col, elem_restr_train;
+  CeedBasis             basis_filter[3];
   CeedVector            filter_rhs, filtered, filter_dinv, aniso_col, train_data, cg_work[3];
   CeedOperator          op_filter_rhs, op_filter_lhs, op_filtered_grad_velo_rhs, op_sgs_train;
   CeedQFunctionContext  diff_filter_qfctx, train_qfctx;
@@ -597,31 +597,9 @@ static int VelocityGradientProjectionSetup(HoneeMiProblem p) {
 // KSPCG with PCJACOBI (inverse diagonal dinv) and KSP_NORM_NATURAL from a zero initial guess: converged when
 // sqrt(r.z) <= max(rtol sqrt(r0.z0), atol), at most max_it iterations (KSPSolve_CG recurrences).  work holds three
 // vectors of the system size.
-static int CgJacobi(HoneeMiProblem p, CeedOperator op, CeedVector dinv, CeedVector R, CeedVector X, CeedVector work[3], CeedVector Ap, double rtol,
-                    double atol, int max_it, int *iterations) {
-  CeedVector r = work[0], z = work[1], pv = work[2];
-  double     rz, pAp, rz_new;
-  CHK(p, CeedVectorSetValue(X, 0.0));
-  CHK(p, CeedVectorCopy(R, r));
-  CHK(p, CeedVectorPointwiseMult(z, dinv, r));
-  CHK(p, CeedVectorCopy(z, pv));
-  CHK(p, CeedMiVectorDot(r, z, &rz));
-  const double ttol = fmax(rtol * sqrt(fabs(rz)), atol);
-  int          its  = 0;
-  while (sqrt(fabs(rz)) > ttol && its < max_it) {
-    CHK(p, CeedOperatorApply(op, pv, Ap, CEED_REQUEST_IMMEDIATE));
-    CHK(p, CeedMiVectorDot(pv, Ap, &pAp));
-    const double alpha = rz / pAp;
-    CHK(p, CeedVectorAXPY(X, alpha, pv));
-    CHK(p, CeedVectorAXPY(r, -alpha, Ap));
-    CHK(p, CeedVectorPointwiseMult(z, dinv, r));
-    CHK(p, CeedMiVectorDot(r, z, &rz_new));
-    const double beta = rz_new / rz;
-    CHK(p, CeedVectorAXPBY(pv, 1.0, beta, z));
-    rz = rz_new;
-    its++;
-  }
-  *iterations = its;
+static int CgJacobi(HoneeMiProblem p, CeedOperator op, CeedVector dinv, CeedVector R, CeedVector X, CeedVector work[3], double rtol, double atol,
+                    int max_it, int *iterations) {
+  CHK(p, CeedMiJacobiCg(op, dinv, R, X, work[0], work[1], work[2], rtol, atol, max_it, iterations));
   return 0;
 }
 
@@ -631,7 +609,7 @@ static int GridAnisotropyTensorProjection(HoneeMiProblem p) {
   if (p->grid_aniso) return 0;
   CeedQFunction qf;
   CeedOperator  op_rhs, op_mass;
-  CeedVector    R, dinv, Ap, work[3];
+  CeedVector    R, dinv, work[3];
   CHK(p, NodalField(p, 7, &p->elem_restr_grid_aniso, &p->basis_grid_aniso));
   CHK(p, CeedQFunctionCreateInterior(p->ceed, 1, HoneeMiQFunctionNotOnHost, "qfunctions/grid_anisotropy_tensor.h:AnisotropyTensorProjection", &qf));
   CHK(p, CeedQFunctionAddInput(qf, "qdata", 10, CEED_EVAL_NONE));
@@ -641,13 +619,13 @@ static int GridAnisotropyTensorProjection(HoneeMiProblem p) {
   CHK(p, CeedOperatorSetField(op_rhs, "v", p->elem_restr_grid_aniso, p->basis_grid_aniso, CEED_VECTOR_ACTIVE));
   CHK(p, CeedQFunctionDestroy(&qf));
   CHK(p, MassOperator(p, 7, p->elem_restr_grid_aniso, p->basis_grid_aniso, &op_mass));
-  CeedVector *vs[7] = {&R, &dinv, &Ap, &work[0], &work[1], &work[2], &p->grid_aniso};
-  for (int i = 0; i < 7; i++) CHK(p, CeedElemRestrictionCreateVector(p->elem_restr_grid_aniso, vs[i], NULL));
+  CeedVector *vs[6] = {&R, &dinv, &work[0], &work[1], &work[2], &p->grid_aniso};
+  for (int i = 0; i < 6; i++) CHK(p, CeedElemRestrictionCreateVector(p->elem_restr_grid_aniso, vs[i], NULL));
   CHK(p, CeedOperatorApply(op_rhs, CEED_VECTOR_NONE, R, CEED_REQUEST_IMMEDIATE));
   CHK(p, CeedOperatorLinearAssembleDiagonal(op_mass, dinv, CEED_REQUEST_IMMEDIATE));
   CHK(p, JacobiInverse(p, dinv));
-  CHK(p, CgJacobi(p, op_mass, dinv, R, p->grid_aniso, work, Ap, 1e-10, 1e-50, 10000, &p->grid_aniso_its));
-  for (int i = 0; i < 6; i++) CHK(p, CeedVectorDestroy(vs[i]));
+  CHK(p, CgJacobi(p, op_mass, dinv, R, p->grid_aniso, work, 1e-10, 1e-50, 10000, &p->grid_aniso_its));
+  for (int i = 0; i < 5; i++) CHK(p, CeedVectorDestroy(vs[i]));
   CHK(p, CeedOperatorDestroy(&op_rhs));
   CHK(p, CeedOperatorDestroy(&op_mass));
   return 0;
@@ -783,14 +761,14 @@ static const char *const kFilterRHSLoc[3] = {"qfunctions/differential_filter.h:D
                                              "qfunctions/differential_filter.h:DifferentialFilter_RHS_Entropy"};
 
 // DifferentialFilterSetup + DifferentialFilterCreateOperators: the filtered field holds per node the primitive state
-// (field 0, 5 components) then the velocity products (field 1, 6 components); the LHS is the composite of
-// DifferentialFilter_LHS_5 and _6 over those fields with the collocated grid anisotropy tensor; the solve is KSPCG +
-// PCJACOBI (diagonal), natural norm.
+// (field 0, 5 components) then the velocity products (field 1, 6 components); the LHS is DifferentialFilter_LHS_11 over
+// both (field 2) with the collocated grid anisotropy tensor, where the reference applies _5 and _6 in turn; the solve is
+// KSPCG + PCJACOBI (diagonal), natural norm.
 int HoneeMiProblemSetupDiffFilter(HoneeMiProblem p, const HoneeMiDiffFilterOptions *o) {
   if (p->filter_enabled) return CEED_ERROR_MINOR;
   const HoneeMiMesh *m = &p->mesh;
-  const int          P3 = m->P * m->P * m->P, ncomps[2] = {5, 6}, field_off[2] = {0, 5};
-  for (int f = 0; f < 2; f++) {
+  const int          P3 = m->P * m->P * m->P, ncomps[3] = {5, 6, 11}, field_off[3] = {0, 5, 0};
+  for (int f = 0; f < 3; f++) {
     CeedInt *off = malloc(sizeof(CeedInt) * (size_t)m->nelem * P3);
     for (size_t i = 0; i < (size_t)m->nelem * P3; i++) off[i] = 11 * m->offsets[i] + field_off[f];
     int ierr = CeedElemRestrictionCreate(p->ceed, m->nelem, P3, ncomps[f], 1, 11 * (CeedSize)m->nnodes, CEED_MEM_HOST, CEED_COPY_VALUES, off,
@@ -846,36 +824,28 @@ int HoneeMiProblemSetupDiffFilter(HoneeMiProblem p, const HoneeMiDiffFilterOptio
     CHK(p, CeedOperatorDestroy(&op));
     CHK(p, CeedQFunctionDestroy(&qf));
   }
-  {  // LHS composite
-    static const char *const kLHSLoc[2] = {"qfunctions/differential_filter.h:DifferentialFilter_LHS_5",
-                                           "qfunctions/differential_filter.h:DifferentialFilter_LHS_6"};
-    CHK(p, CeedOperatorCreateComposite(p->ceed, &p->op_filter_lhs));
-    for (int f = 0; f < 2; f++) {
-      CeedQFunction qf;
-      CeedOperator  sub;
-      const int     N = ncomps[f];
-      CHK(p, CeedQFunctionCreateInterior(p->ceed, 1, HoneeMiQFunctionNotOnHost, kLHSLoc[f], &qf));
-      CHK(p, CeedQFunctionSetContext(qf, p->diff_filter_qfctx));
-      CHK(p, CeedQFunctionSetUserFlopsEstimate(qf, 0));
-      CHK(p, CeedQFunctionAddInput(qf, "q", N, CEED_EVAL_INTERP));
-      CHK(p, CeedQFunctionAddInput(qf, "Grad_q", 3 * N, CEED_EVAL_GRAD));
-      CHK(p, CeedQFunctionAddInput(qf, "anisotropy tensor", 7, CEED_EVAL_NONE));
-      CHK(p, CeedQFunctionAddInput(qf, "x", 3, CEED_EVAL_INTERP));
-      CHK(p, CeedQFunctionAddInput(qf, "qdata", 10, CEED_EVAL_NONE));
-      CHK(p, CeedQFunctionAddOutput(qf, "v", N, CEED_EVAL_INTERP));
-      CHK(p, CeedQFunctionAddOutput(qf, "Grad_v", 3 * N, CEED_EVAL_GRAD));
-      CHK(p, CeedOperatorCreate(p->ceed, qf, NULL, NULL, &sub));
-      CHK(p, CeedOperatorSetField(sub, "q", p->elem_restr_filter[f], p->basis_filter[f], CEED_VECTOR_ACTIVE));
-      CHK(p, CeedOperatorSetField(sub, "Grad_q", p->elem_restr_filter[f], p->basis_filter[f], CEED_VECTOR_ACTIVE));
-      CHK(p, CeedOperatorSetField(sub, "anisotropy tensor", p->elem_restr_aniso_col, CEED_BASIS_NONE, p->aniso_col));
-      CHK(p, CeedOperatorSetField(sub, "x", p->elem_restr_x, p->basis_x, p->x_coord));
-      CHK(p, CeedOperatorSetField(sub, "qdata", p->elem_restr_qd, CEED_BASIS_NONE, p->q_data));
-      CHK(p, CeedOperatorSetField(sub, "v", p->elem_restr_filter[f], p->basis_filter[f], CEED_VECTOR_ACTIVE));
-      CHK(p, CeedOperatorSetField(sub, "Grad_v", p->elem_restr_filter[f], p->basis_filter[f], CEED_VECTOR_ACTIVE));
-      CHK(p, CeedOperatorCompositeAddSub(p->op_filter_lhs, sub));
-      CHK(p, CeedOperatorDestroy(&sub));
-      CHK(p, CeedQFunctionDestroy(&qf));
-    }
+  {  // LHS: DifferentialFilter_LHS_N acts on every component alike, so the two fields are one of 11 components to it
+    CeedQFunction qf;
+    const int     N = 11;
+    CHK(p, CeedQFunctionCreateInterior(p->ceed, 1, HoneeMiQFunctionNotOnHost, "qfunctions/differential_filter.h:DifferentialFilter_LHS_11", &qf));
+    CHK(p, CeedQFunctionSetContext(qf, p->diff_filter_qfctx));
+    CHK(p, CeedQFunctionSetUserFlopsEstimate(qf, 0));
+    CHK(p, CeedQFunctionAddInput(qf, "q", N, CEED_EVAL_INTERP));
+    CHK(p, CeedQFunctionAddInput(qf, "Grad_q", 3 * N, CEED_EVAL_GRAD));
+    CHK(p, CeedQFunctionAddInput(qf, "anisotropy tensor", 7, CEED_EVAL_NONE));
+    CHK(p, CeedQFunctionAddInput(qf, "x", 3, CEED_EVAL_INTERP));
+    CHK(p, CeedQFunctionAddInput(qf, "qdata", 10, CEED_EVAL_NONE));
+    CHK(p, CeedQFunctionAddOutput(qf, "v", N, CEED_EVAL_INTERP));
+    CHK(p, CeedQFunctionAddOutput(qf, "Grad_v", 3 * N, CEED_EVAL_GRAD));
+    CHK(p, CeedOperatorCreate(p->ceed, qf, NULL, NULL, &p->op_filter_lhs));
+    CHK(p, CeedOperatorSetField(p->op_filter_lhs, "q", p->elem_restr_filter[2], p->basis_filter[2], CEED_VECTOR_ACTIVE));
+    CHK(p, CeedOperatorSetField(p->op_filter_lhs, "Grad_q", p->elem_restr_filter[2], p->basis_filter[2], CEED_VECTOR_ACTIVE));
+    CHK(p, CeedOperatorSetField(p->op_filter_lhs, "anisotropy tensor", p->elem_restr_aniso_col, CEED_BASIS_NONE, p->aniso_col));
+    CHK(p, CeedOperatorSetField(p->op_filter_lhs, "x", p->elem_restr_x, p->basis_x, p->x_coord));
+    CHK(p, CeedOperatorSetField(p->op_filter_lhs, "qdata", p->elem_restr_qd, CEED_BASIS_NONE, p->q_data));
+    CHK(p, CeedOperatorSetField(p->op_filter_lhs, "v", p->elem_restr_filter[2], p->basis_filter[2], CEED_VECTOR_ACTIVE));
+    CHK(p, CeedOperatorSetField(p->op_filter_lhs, "Grad_v", p->elem_restr_filter[2], p->basis_filter[2], CEED_VECTOR_ACTIVE));
+    CHK(p, CeedQFunctionDestroy(&qf));
     CHK(p, CeedOperatorGetContextFieldLabel(p->op_filter_lhs, "filter width scaling", &p->filter_width_label));
   }
   CeedVector *vs[6] = {&p->filter_rhs, &p->filtered, &p->filter_dinv, &p->cg_work[0], &p->cg_work[1], &p->cg_work[2]};
@@ -897,12 +867,8 @@ static int DiffFilterApply(HoneeMiProblem p) {
     CHK(p, JacobiInverse(p, p->filter_dinv));
     p->filter_pc_ready = 1;
   }
-  CeedVector ApV;
-  CHK(p, CeedElemRestrictionCreateVector(p->elem_restr_filter[0], &ApV, NULL));
-  int ierr = CgJacobi(p, p->op_filter_lhs, p->filter_dinv, p->filter_rhs, p->filtered, p->cg_work, ApV, p->filter_rtol, p->filter_atol,
-                      p->filter_max_it, &p->filter_its);
-  CeedVectorDestroy(&ApV);
-  return ierr;
+  return CgJacobi(p, p->op_filter_lhs, p->filter_dinv, p->filter_rhs, p->filtered, p->cg_work, p->filter_rtol, p->filter_atol, p->filter_max_it,
+                  &p->filter_its);
 }
 
 int HoneeMiSetFilterWidthScaling(HoneeMiProblem p, const double scaling[3]) {
@@ -1414,7 +1380,7 @@ int HoneeMiProblemDestroy(HoneeMiProblem *problem) {
   CeedOperatorDestroy(&p->op_filter_lhs);
   CeedOperatorDestroy(&p->op_filtered_grad_velo_rhs);
   CeedOperatorDestroy(&p->op_sgs_train);
-  for (int i = 0; i < 2; i++) {
+  for (int i = 0; i < 3; i++) {
     CeedElemRestrictionDestroy(&p->elem_restr_filter[i]);
     CeedBasisDestroy(&p->basis_filter[i]);
   }

@@ -98,6 +98,7 @@ struct SgsNodalArgs {
   const double *model;  // b1[20], b2[6], W1[20][6], W2[6][20], bounds[6][2], alpha
   const int    *p_offsets;  // training pairs: filtered velocity products (offsets into the filtered field q)
   int           p_comp_stride;
+  bool          overwrite;  // write v instead of adding to it
 };
 
 hipError_t launch_gather_vertex_coords(int nelem, const int *xoffsets, const double *x, int xcs, double *xe, hipStream_t s);
@@ -154,6 +155,23 @@ hipError_t launch_node_gather_rows_f32(int nrows, int comp_stride, const int *t_
 hipError_t launch_node_gather_blocks(int nrows, const int *t_rowptr, const int *t_index, const int *t_offset, const double *ev, double *v,
                                      hipStream_t s);
 hipError_t launch_restriction_transpose(const int *offsets, int nelem, int elemsize, int ncomp, int comp_stride, const double *e, double *u, hipStream_t s);
+
+// Conjugate gradients with a Jacobi preconditioner (kernels_vector.hip).  scratch holds two sets of kCgBlocks block partials
+// (of r.z, then of p.Ap) and r.z of the last two iterations.  start: x = 0, r = rhs, p = dinv r, then r.z into scalar 0;
+// dot: the partials of p.Ap; update: alpha = r.z / p.Ap, x += alpha p, r -= alpha Ap, then beta and p = dinv r + beta p, with
+// the old r.z in scalar odd and the new one in the other.  start and update publish r.z to h, then seq to flag (mapped host
+// memory).
+constexpr int kCgBlocks = 512, kCgScratch = 2 * kCgBlocks + 2;
+struct CgArgs {
+  long long           n;
+  const double       *dinv, *rhs, *ap;
+  double             *x, *r, *p, *scratch, *h;
+  unsigned long long *flag, seq;
+  int                 odd;
+};
+hipError_t launch_cg_start(const CgArgs &a, hipStream_t s);
+hipError_t launch_cg_dot(const CgArgs &a, hipStream_t s);
+hipError_t launch_cg_update(const CgArgs &a, hipStream_t s);
 
 // SGS closure and projections (kernels_sgs.hip)
 bool       sgs_pq_supported(int P, int Q);

@@ -30,6 +30,10 @@ template <int Q>
 constexpr int sgs_elems_per_block() {
   return (Q * Q * Q >= 64) ? 1 : 64 / (Q * Q * Q);
 }
+// Most components of a k_filter_lhs chunk (11: 6 + 5).  With 4 + 4 + 3 the deconvolution pairs at 32^3 p=2 took 15.5 ms
+// against 14.6: more barriers and passes over the tensor outweigh the LDS saved.
+constexpr int kFilterChunk = 6;
+
 // Threads of a k_field block: its elements' points in whole waves
 template <int Q>
 constexpr int sgs_block_threads() {
@@ -188,43 +192,33 @@ __device__ __forceinline__ void filter_alpha(const FieldArgs &a, const CeedMiDif
     for (int j = 0; j < 3; j++) alpha[i][j] = (SD[i][0] * SD[0][j] + SD[i][1] * SD[1][j] + SD[i][2] * SD[2][j]) * f.kernel_scaling;
 }
 
-template <int N>
-struct DiffFilterLHS {  // v = wdetJ q, Grad_v[k] = wdetJ (alpha (dXdx grad_x q))[k], every component alike
-  using Ctx                       = CeedMiDiffFilterContext;
-  static constexpr int  NU = N, NU2 = 0, NV = N;
-  static constexpr bool GRAD = true, OUTV = true, OUTG = true;
-  template <int Q>
-  __device__ static void qfq(const FieldArgs &a, const Ctx &ctx, int e, int t, const double qd[10], bool ok, const double (&u)[N],
-                             const double (&gu)[3][N], const double (&)[1], double (&out)[4 * N]) {
-    double wdetJ, dXdx[3][3], alpha[3][3];
-    nsop::unpack_qdata(qd, ok, wdetJ, dXdx);
-    filter_alpha<Q>(a, ctx, e, t, ok, alpha);
+// K = wdetJ alpha dXdx dXdx^T: the filter's gradient coupling in the reference directions
+__device__ __forceinline__ void filter_tensor(double wdetJ, const double dXdx[3][3], const double alpha[3][3], double K[3][3]) {
+  double G[3][3];
 #pragma unroll
-    for (int j = 0; j < N; j++) {
-      out[j] = wdetJ * u[j];
-      double dq[3], dqX[3];
+  for (int i = 0; i < 3; i++)
 #pragma unroll
-      for (int k = 0; k < 3; k++) dq[k] = gu[0][j] * dXdx[0][k] + gu[1][j] * dXdx[1][k] + gu[2][j] * dXdx[2][k];
+    for (int d = 0; d < 3; d++) G[i][d] = dXdx[i][0] * dXdx[d][0] + dXdx[i][1] * dXdx[d][1] + dXdx[i][2] * dXdx[d][2];
 #pragma unroll
-      for (int k = 0; k < 3; k++) dqX[k] = dXdx[k][0] * dq[0] + dXdx[k][1] * dq[1] + dXdx[k][2] * dq[2];
+  for (int k = 0; k < 3; k++)
 #pragma unroll
-      for (int k = 0; k < 3; k++) out[N + k * N + j] = wdetJ * (alpha[k][0] * dqX[0] + alpha[k][1] * dqX[1] + alpha[k][2] * dqX[2]);
-    }
+    for (int d = 0; d < 3; d++) K[k][d] = wdetJ * (alpha[k][0] * G[0][d] + alpha[k][1] * G[1][d] + alpha[k][2] * G[2][d]);
+}
+
+// The 1D tables of the 4 x 4 x 4 element in LDS, with G = Dc B
+template <int P, int Q>
+__device__ __forceinline__ void stage_tables(const BasisTables &bt, double *sB, double *sDc, double *sG) {
+  for (int i = threadIdx.x; i < Q * P; i += blockDim.x) sB[i] = bt.B[i];
+  for (int i = threadIdx.x; i < Q * Q; i += blockDim.x) sDc[i] = bt.Dc[i];
+  for (int i = threadIdx.x; i < Q * P; i += blockDim.x) {
+    double g = 0;
+    for (int m = 0; m < Q; m++) g += bt.Dc[i / P * Q + m] * bt.B[m * P + i % P];
+    sG[i] = g;
   }
-};
+}
 
 // Slot map of the stage: active input u -> 0..NU-1, its reference gradient -> NU + NU d + c, passive input (without a
 // gradient) -> NU + c.  Outputs: values -> 0..NV-1, gradient test weights -> NV + NV d + c.
-// Op::qf(a, ctx, e, t, ...) or, for bodies that depend on Q, Op::qfq<Q>(...)
-template <class Op, int Q, class = void>
-struct HasQfq {
-  static constexpr bool value = false;
-};
-template <class Op, int Q>
-struct HasQfq<Op, Q, decltype((void)&Op::template qfq<Q>)> {
-  static constexpr bool value = true;
-};
-
 template <int P, int Q, class Op>
 __global__ void __launch_bounds__(sgs_block_threads<Q>()) k_field(FieldArgs a, const typename Op::Ctx ctx) {
   using Dm          = Dims<P, Q>;
@@ -245,13 +239,7 @@ __global__ void __launch_bounds__(sgs_block_threads<Q>()) k_field(FieldArgs a, c
   __shared__ double sB[LINES ? 1 : Q * P], sDc[LINES ? 1 : Q * Q], sG[LINES ? 1 : Q * P];
   __shared__ double sX[EPB][NST][SLOT];
   if constexpr (!LINES) {
-    for (int i = threadIdx.x; i < Q * P; i += blockDim.x) sB[i] = a.bt.B[i];
-    for (int i = threadIdx.x; i < Q * Q; i += blockDim.x) sDc[i] = a.bt.Dc[i];
-    for (int i = threadIdx.x; i < Q * P; i += blockDim.x) {  // G = Dc B
-      double g = 0;
-      for (int m = 0; m < Q; m++) g += a.bt.Dc[i / P * Q + m] * a.bt.B[m * P + i % P];
-      sG[i] = g;
-    }
+    stage_tables<P, Q>(a.bt, sB, sDc, sG);
     __syncthreads();
   }
   // threads past the elements' points only take part in the lines
@@ -306,8 +294,7 @@ __global__ void __launch_bounds__(sgs_block_threads<Q>()) k_field(FieldArgs a, c
     }
 #pragma unroll
     for (int c = 0; c < NU2X; c++) u2[c] = NU2 > 0 ? X[NU + c][t] : 0.0;
-    if constexpr (HasQfq<Op, Q>::value) Op::template qfq<Q>(a, ctx, e, t, qd, ok, u, gu, u2, out);
-    else Op::qf(a, ctx, e, t, qd, ok, u, gu, u2, out);
+    Op::qf(a, ctx, e, t, qd, ok, u, gu, u2, out);
     if (act) {
       if constexpr (Op::OUTV) {
 #pragma unroll
@@ -339,6 +326,100 @@ __global__ void __launch_bounds__(sgs_block_threads<Q>()) k_field(FieldArgs a, c
         const int off = a.out_offsets[enode];
 #pragma unroll
         for (int c = 0; c < NV; c++) atomicAdd(&a.v[off + c * a.out_comp_stride], r[c]);
+      }
+    }
+  }
+}
+
+// DifferentialFilter_LHS_N (qfunctions/differential_filter.h:91-125): v = wdetJ q, Grad_v[k] = wdetJ (alpha (dXdx grad_x q))[k]
+// for N components alike, which in the reference directions is the 3 x 3 matrix K = wdetJ alpha dXdx dXdx^T on the reference
+// gradient.  K and the node offsets are formed once per element and serve all components, NC of which go through the stage
+// at a time (11 components at once would leave one block of LDS to a SIMD).
+// Bound by LDS and instruction issue.  Measured at 32^3 p=2, 11 components: 139 us as two operators of 5 and 6 components
+// through k_field, each with its own copy of the point data -> 102 us.
+template <int P, int Q, int N>
+__global__ void __launch_bounds__(sgs_block_threads<Q>()) k_filter_lhs(FieldArgs a, const CeedMiDiffFilterContext ctx) {
+  using Dm          = Dims<P, Q>;
+  constexpr int EPB = sgs_elems_per_block<Q>();
+  constexpr int Q3  = Dm::Q3;
+  constexpr int NT  = sgs_block_threads<Q>();
+  constexpr int NCH = (N + kFilterChunk - 1) / kFilterChunk, NC = (N + NCH - 1) / NCH, NST = 4 * NC;
+  static_assert(Dm::P3 <= Q3, "P <= Q is required");
+  constexpr bool LINES = !(P == 4 && Q == 4);
+  using Lines          = basis3::LineStage<P, Q, EPB, NST>;
+  constexpr int SLOT   = LINES ? Lines::kSlot : Q3;
+  __shared__ double sB[LINES ? 1 : Q * P], sDc[LINES ? 1 : Q * Q], sG[LINES ? 1 : Q * P];
+  __shared__ double sX[EPB][NST][SLOT];
+  if constexpr (!LINES) {
+    stage_tables<P, Q>(a.bt, sB, sDc, sG);
+    __syncthreads();
+  }
+  const bool      act = NT == EPB * Q3 || threadIdx.x < EPB * Q3;
+  const int       le = act ? threadIdx.x / Q3 : 0, t = act ? threadIdx.x % Q3 : 0;
+  const bool      nd = act && t < Dm::P3;
+  double(*X)[SLOT]   = sX[le];
+  const long long nbatch = ((long long)a.nelem + EPB - 1) / EPB;
+  for (long long bt = blockIdx.x; bt < nbatch; bt += gridDim.x) {
+    const long long e_    = bt * EPB + le;
+    const bool      ok    = act && e_ < a.nelem;
+    const int       e     = ok ? (int)e_ : 0;
+    const long long enode = (long long)e * Dm::P3 + t;
+    const int       off = ok && nd ? a.in_offsets[enode] : 0, slot = a.ev && ok && nd ? a.perm[enode] : 0;
+    double          wdetJ, K[3][3];
+    {
+      double qd[10], dXdx[3][3], alpha[3][3];
+#pragma unroll
+      for (int k = 0; k < 10; k++) qd[k] = ok ? a.qdata[(long long)e * a.qd.se + k * Q3 + t] : 0.0;
+      nsop::unpack_qdata(qd, ok, wdetJ, dXdx);
+      filter_alpha<Q>(a, ctx, e, t, ok, alpha);
+      filter_tensor(wdetJ, dXdx, alpha, K);
+    }
+    // N components in NCH chunks of NC (the last one repeats components of the one before, which writes them twice alike,
+    // where N is no multiple of NC)
+#pragma unroll
+    for (int ch = 0; ch < NCH; ch++) {
+      const int c0 = ch < NCH - 1 ? ch * NC : N - NC;
+      double    r[NC];
+#pragma unroll
+      for (int c = 0; c < NC; c++) r[c] = ok && nd ? a.u[off + (c0 + c) * a.in_comp_stride] : 0.0;
+      if constexpr (LINES) {
+        if (nd) {
+          const int at = Lines::node(t);
+#pragma unroll
+          for (int c = 0; c < NC; c++) X[c][at] = r[c];
+        }
+        Lines(a.bt.B, a.bt.Dc, sX, threadIdx.x).template interp_grad<NC, true>(0, NC);
+      } else {
+        basis3::StageMF(sB, sDc, sG, X, t).template interp_grad<NC>(r, 0, NC);
+      }
+      if (act) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          const double g0 = X[NC + c][t], g1 = X[2 * NC + c][t], g2 = X[3 * NC + c][t];
+          X[c][t] *= wdetJ;
+#pragma unroll
+          for (int k = 0; k < 3; k++) X[NC + NC * k + c][t] = K[k][0] * g0 + K[k][1] * g1 + K[k][2] * g2;
+        }
+      }
+      if constexpr (LINES) {
+        Lines(a.bt.B, a.bt.Dc, sX, threadIdx.x).template transpose<NC, true, true>(0, NC);
+        const int at = Lines::node(t);
+#pragma unroll
+        for (int c = 0; c < NC; c++) r[c] = X[c][at];
+        __syncthreads();  // (P < Q) the values are read before the next node values go to these slots
+      } else {
+        basis3::StageMF(sB, sDc, sG, X, t).template transpose<NC, true, true>(0, NC, r);
+      }
+      if (ok && nd) {
+        if (a.ev) {
+          double *dst = a.ev + (long long)slot * N + c0;
+#pragma unroll
+          for (int c = 0; c < NC; c++) dst[c] = r[c];
+        } else {
+#pragma unroll
+          for (int c = 0; c < NC; c++)
+            if (c0 + c >= ch * NC) atomicAdd(&a.v[off + (c0 + c) * a.out_comp_stride], r[c]);
+        }
       }
     }
   }
@@ -432,9 +513,9 @@ __global__ void __launch_bounds__(kNodalBlock) k_sgs_nodal(SgsNodalArgs a, const
 #pragma unroll
       for (int c = 0; c < 6; c++) acc[c] += w * km[c];
     }
-    const int off = a.row_offset[k];
+    double *dst = a.v + a.row_offset[k];
 #pragma unroll
-    for (int c = 0; c < 6; c++) a.v[off + c * a.out_comp_stride] += acc[c];
+    for (int c = 0; c < 6; c++) dst[c * a.out_comp_stride] = a.overwrite ? acc[c] : dst[c * a.out_comp_stride] + acc[c];
   }
 }
 
@@ -463,17 +544,10 @@ __global__ void __launch_bounds__(sgs_elems_per_block<Q>() * Q * Q * Q) k_filter
     double          qd[10];
 #pragma unroll
     for (int k = 0; k < 10; k++) qd[k] = ok ? a.qdata[(long long)e * a.qd.se + k * Q3 + t] : 0.0;
-    double wdetJ, dXdx[3][3], alpha[3][3], G[3][3], K[3][3];
+    double wdetJ, dXdx[3][3], alpha[3][3], K[3][3];
     nsop::unpack_qdata(qd, ok, wdetJ, dXdx);
     filter_alpha<Q>(a, ctx, e, t, ok, alpha);
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int d = 0; d < 3; d++) G[i][d] = dXdx[i][0] * dXdx[d][0] + dXdx[i][1] * dXdx[d][1] + dXdx[i][2] * dXdx[d][2];
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-#pragma unroll
-      for (int d = 0; d < 3; d++) K[k][d] = wdetJ * (alpha[k][0] * G[0][d] + alpha[k][1] * G[1][d] + alpha[k][2] * G[2][d]);
+    filter_tensor(wdetJ, dXdx, alpha, K);
     basis3::Elem<P, Q> el(nullptr, nullptr, sS[le][0], sS[le][1], sS[le][2], t);
     double             r = el.contract_t(wdetJ, sBB, sBB, sBB);
     r += el.contract_t(K[0][0], sGG, sBB, sBB);
@@ -552,9 +626,9 @@ __global__ void __launch_bounds__(kNodalBlock) k_sgs_training_nodal(SgsNodalArgs
 #pragma unroll
     for (int c = 0; c < 12; c++) acc[c] += val[c] * w;
   }
-  const int off = a.row_offset[k];
+  double *dst = a.v + a.row_offset[k];
 #pragma unroll
-  for (int c = 0; c < 12; c++) a.v[off + c * a.out_comp_stride] += acc[c];
+  for (int c = 0; c < 12; c++) dst[c * a.out_comp_stride] = a.overwrite ? acc[c] : dst[c * a.out_comp_stride] + acc[c];
 }
 
 template <typename K>
@@ -588,6 +662,15 @@ hipError_t launch_mass_n_diagonal_pq(const FieldArgs &a, int ncomp, hipStream_t 
   auto          kern  = k_mass_n_diagonal<P, Q>;
   const int     grid  = grid_for_batches(kern, block, ((long long)a.nelem + EPB - 1) / EPB);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, s, a, ncomp);
+  return hipGetLastError();
+}
+
+template <int P, int Q, int N>
+hipError_t launch_filter_lhs_pq(const FieldArgs &a, const CeedMiDiffFilterContext &ctx, hipStream_t s) {
+  constexpr int EPB  = sgs_elems_per_block<Q>();
+  auto          kern = k_filter_lhs<P, Q, N>;
+  const int     grid = grid_for_batches(kern, sgs_block_threads<Q>(), ((long long)a.nelem + EPB - 1) / EPB);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(sgs_block_threads<Q>()), 0, s, a, ctx);
   return hipGetLastError();
 }
 
@@ -715,16 +798,18 @@ hipError_t launch_diff_filter_rhs(int P, int Q, int var, const FieldArgs &a, con
 bool diff_filter_ncomp_supported(int ncomp) { return ncomp == 1 || ncomp == 5 || ncomp == 6 || ncomp == 11; }
 
 hipError_t launch_diff_filter_lhs(int P, int Q, int ncomp, const FieldArgs &a, const CeedMiDiffFilterContext &ctx, hipStream_t s) {
-  switch (ncomp) {
-    case 1:
-      return dispatch_pq<RunField, DiffFilterLHS<1>>(P, Q, a, ctx, s);
-    case 5:
-      return dispatch_pq<RunField, DiffFilterLHS<5>>(P, Q, a, ctx, s);
-    case 6:
-      return dispatch_pq<RunField, DiffFilterLHS<6>>(P, Q, a, ctx, s);
-    case 11:
-      return dispatch_pq<RunField, DiffFilterLHS<11>>(P, Q, a, ctx, s);
+  if (a.nelem <= 0) return hipSuccess;
+#define FD_LHS(p, q)                                                  \
+  if (P == p && Q == q) {                                             \
+    switch (ncomp) {                                                  \
+      case 1: return launch_filter_lhs_pq<p, q, 1>(a, ctx, s);        \
+      case 5: return launch_filter_lhs_pq<p, q, 5>(a, ctx, s);        \
+      case 6: return launch_filter_lhs_pq<p, q, 6>(a, ctx, s);        \
+      case 11: return launch_filter_lhs_pq<p, q, 11>(a, ctx, s);      \
+    }                                                                 \
   }
+  SGS_PQ_LIST(FD_LHS)
+#undef FD_LHS
   return hipErrorInvalidValue;
 }
 

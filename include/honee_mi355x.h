@@ -129,6 +129,12 @@ int CeedMiVectorGetFp32ShadowRead(CeedVector vec, const float **d_array, CeedSiz
 // a fixed order (the same result for the same inputs on every call).
 int CeedMiVectorDot(CeedVector x, CeedVector y, double *result);
 
+// Solve op x = rhs by conjugate gradients from x = 0, preconditioned by the inverse diagonal dinv, in the natural norm:
+// converged when sqrt(r.z) <= max(rtol sqrt(r0.z0), atol), at most max_it iterations (the KSPCG + PCJACOBI recurrences).
+// r, p and Ap are work vectors of the same length.  Deterministic: every sum runs in a fixed order.
+int CeedMiJacobiCg(CeedOperator op, CeedVector dinv, CeedVector rhs, CeedVector x, CeedVector r, CeedVector p, CeedVector Ap,
+                   CeedScalar rtol, CeedScalar atol, CeedInt max_it, CeedInt *iterations);
+
 // Synchronize the backend stream.
 int CeedMiSynchronize(Ceed ceed);
 
