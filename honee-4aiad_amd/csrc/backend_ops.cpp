@@ -830,12 +830,10 @@ static int scatter_finish(OpPlan *p, Ceed ceed, const VolumeArgs &a, bool overwr
   CeedElemRestriction r = p->r_q;
   hipEvent_t          ev;
   MI_CALL(timing_begin(ceed, "scatter_node_gather", &ev));
-  if (a.ev32)
-    MI_HIP(ceed, launch_node_gather_rows_f32(r->t_nrows, r->comp_stride, r->d_t_rowptr, r->d_t_index, r->d_t_offset, a.ev32, a.v, overwrite,
-                                             ceed->stream));
+  if (a.perm)
+    MI_HIP(ceed, launch_node_gather(r->t_nrows, 5, r->comp_stride, r->d_t_rowptr, r->d_t_offset, a.ev, a.v, overwrite, ceed->stream));
   else
-    MI_HIP(ceed, launch_node_gather(r->t_nrows, 5, r->comp_stride, r->d_t_rowptr, a.perm ? nullptr : r->d_t_index, r->d_t_offset, a.ev, a.v,
-                                    overwrite, ceed->stream));
+    MI_HIP(ceed, launch_node_gather_tiles(rstr_gather_tiles(r), r->comp_stride, a.ev, a.ev32, a.v, overwrite, ceed->stream));
   MI_CALL(timing_end(ceed, "scatter_node_gather", ev));
   return 0;
 }
@@ -1097,7 +1095,7 @@ static int sgs_field_apply(CeedOperator op, OpPlan *p, CeedVector in, CeedVector
   MI_CALL(timing_end(ceed, p->kernel_name.c_str(), ev));
   if (a.ev) {
     MI_CALL(timing_begin(ceed, "scatter_node_gather", &ev));
-    MI_HIP(ceed, launch_node_gather(r->t_nrows, p->ncomp_out, r->comp_stride, r->d_t_rowptr, nullptr, r->d_t_offset, a.ev, a.v, overwrite, s));
+    MI_HIP(ceed, launch_node_gather(r->t_nrows, p->ncomp_out, r->comp_stride, r->d_t_rowptr, r->d_t_offset, a.ev, a.v, overwrite, s));
     MI_CALL(timing_end(ceed, "scatter_node_gather", ev));
   }
   return 0;
@@ -1347,7 +1345,7 @@ static int field_diag_evec_begin(Ceed ceed, OpPlan *p, CeedElemRestriction r, Fi
   return 0;
 }
 static int field_diag_evec_finish(Ceed ceed, OpPlan *p, CeedElemRestriction r, const FieldArgs &a) {
-  MI_HIP(ceed, launch_node_gather(r->t_nrows, p->ncomp_out, r->comp_stride, r->d_t_rowptr, nullptr, r->d_t_offset, a.ev, a.v, false, ceed->stream));
+  MI_HIP(ceed, launch_node_gather(r->t_nrows, p->ncomp_out, r->comp_stride, r->d_t_rowptr, r->d_t_offset, a.ev, a.v, false, ceed->stream));
   return 0;
 }
 

@@ -896,6 +896,30 @@ void group_by_offset(const std::vector<CeedInt> &offsets, std::vector<int> &rowp
   for (size_t i = 0; i < n; i++) index[start[offsets[i]]++] = (int)i;
 }
 
+// Tiles of consecutive rows with at most `target` slots each (a row with more is a tile by itself), the slots of each tile
+// sorted in place and the sorted position of every slot in the rows' order.  Few slots are split into smaller tiles, so that
+// more blocks share the latency.
+void gather_tiles(const std::vector<int> &rowptr, std::vector<int> &index, std::vector<int> &tile, std::vector<unsigned short> &pos) {
+  const int nrows = (int)rowptr.size() - 1, target = (int)std::clamp<size_t>(index.size() / 1024, 64, kGatherSlots);
+  tile.assign(1, 0);
+  pos.resize(index.size());
+  std::vector<int> order;
+  for (int r0 = 0; r0 < nrows;) {
+    int r1 = r0 + 1;
+    while (r1 < nrows && rowptr[r1 + 1] - rowptr[r0] <= target) r1++;
+    const int j0 = rowptr[r0], m = rowptr[r1] - j0;
+    if (m <= kGatherSlots) {
+      order.resize(m);
+      for (int i = 0; i < m; i++) order[i] = i;
+      std::sort(order.begin(), order.end(), [&](int x, int y) { return index[j0 + x] < index[j0 + y]; });
+      for (int i = 0; i < m; i++) pos[j0 + order[i]] = (unsigned short)i;
+      std::sort(index.begin() + j0, index.begin() + j0 + m);
+    }
+    tile.push_back(r1);
+    r0 = r1;
+  }
+}
+
 // Transpose of the offsets for the two-pass scatter: L-vector offsets in ascending order (rows), each with the
 // ascending list of element-node indices e * elem_size + j that gather from it; t_perm maps an element node to its
 // slot in that node-sorted order.  Built once per restriction on the host.
@@ -921,7 +945,29 @@ int rstr_transpose_map(CeedElemRestriction r) {
   if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_perm, perm.data(), sizeof(int) * n, hipMemcpyHostToDevice));
   if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_index, index.data(), sizeof(int) * n, hipMemcpyHostToDevice));
   if (!toff.empty()) MI_HIP(r->ceed, hipMemcpy(r->d_t_offset, toff.data(), sizeof(int) * toff.size(), hipMemcpyHostToDevice));
+  std::vector<int>            tile;
+  std::vector<unsigned short> pos;
+  gather_tiles(rowptr, index, tile, pos);
+  r->t_ntile = (int)tile.size() - 1;
+  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_tile, sizeof(int) * tile.size()));
+  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_slot, sizeof(int) * std::max<size_t>(n, 1)));
+  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_pos, sizeof(unsigned short) * std::max<size_t>(n, 1)));
+  MI_HIP(r->ceed, hipMemcpy(r->d_t_tile, tile.data(), sizeof(int) * tile.size(), hipMemcpyHostToDevice));
+  if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_slot, index.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+  if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_pos, pos.data(), sizeof(unsigned short) * n, hipMemcpyHostToDevice));
   return 0;
+}
+
+GatherTiles rstr_gather_tiles(CeedElemRestriction r) {
+  GatherTiles g{};
+  g.ntile    = r->t_ntile;
+  g.stride   = r->t_stride;
+  g.tile_row = r->d_t_tile;
+  g.rowptr   = r->d_t_rowptr;
+  g.slot     = r->d_t_slot;
+  g.toff     = r->d_t_offset;
+  g.pos      = r->d_t_pos;
+  return g;
 }
 
 // Device workspace of at least len doubles, owned by the Ceed and reused by every operator apply on its stream.
@@ -1029,6 +1075,9 @@ extern "C" int CeedElemRestrictionDestroy(CeedElemRestriction *rstr) {
   if (r->d_t_perm) (void)hipFree(r->d_t_perm);
   if (r->d_t_index) (void)hipFree(r->d_t_index);
   if (r->d_t_offset) (void)hipFree(r->d_t_offset);
+  if (r->d_t_tile) (void)hipFree(r->d_t_tile);
+  if (r->d_t_slot) (void)hipFree(r->d_t_slot);
+  if (r->d_t_pos) (void)hipFree(r->d_t_pos);
   Ceed c = r->ceed;
   delete r;
   CeedDestroy(&c);

@@ -89,6 +89,10 @@ struct CeedElemRestriction_private {
   int                  t_stride     = 0;      // row k's offset is k t_stride (0: no such stride)
   int                 *d_t_rowptr = nullptr, *d_t_perm = nullptr, *d_t_offset = nullptr;
   int                 *d_t_index = nullptr;  // element node of each slot (inverse of t_perm)
+  // tiles of rows for the gather of an element-ordered E-vector (GatherTiles)
+  int                  t_ntile = 0;
+  int                 *d_t_tile = nullptr, *d_t_slot = nullptr;
+  unsigned short      *d_t_pos = nullptr;
 };
 
 struct CeedBasis_private {
@@ -226,6 +230,7 @@ int  ceed_set_error(Ceed ceed, const char *file, int line, const char *func, int
 
 int vec_device_read(CeedVector v, const double **d);
 int rstr_transpose_map(CeedElemRestriction r);
+GatherTiles rstr_gather_tiles(CeedElemRestriction r);  // of a restriction with its transpose map
 // Element-node slots grouped by offset, in increasing offset order, each group listing its slots in increasing order:
 // rows r = 0..toff.size()-1 hold slots index[rowptr[r] .. rowptr[r+1]) of offset toff[r].  O(n + max offset).
 void group_by_offset(const std::vector<CeedInt> &offsets, std::vector<int> &rowptr, std::vector<int> &index, std::vector<int> &toff);

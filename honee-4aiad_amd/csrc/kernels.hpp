@@ -143,15 +143,22 @@ hipError_t launch_reciprocal(double *x, long long n, hipStream_t s);
 hipError_t launch_norm(const double *x, long long n, int type, double *d_partial, int npartial, hipStream_t s);
 hipError_t launch_multiplicity(const int *offsets, long long n_offsets, int ncomp, int comp_stride, double *mult, hipStream_t s);
 hipError_t launch_restriction_notranspose(const int *offsets, int nelem, int elemsize, int ncomp, int comp_stride, const double *u, double *e, hipStream_t s);
-// Second pass of the deterministic scatter: v[t_offset[k] + c * comp_stride] (+)= sum over j in
-// [t_rowptr[k], t_rowptr[k+1]) of ev[slot(j) * ncomp + c] in ascending j, with slot(j) = t_index[j] for an
-// element-ordered E-vector or slot(j) = j for a node-sorted one (t_index null).
-hipError_t launch_node_gather(int nrows, int ncomp, int comp_stride, const int *t_rowptr, const int *t_index, const int *t_offset,
-                              const double *ev, double *v, bool overwrite, hipStream_t s);
+// Second pass of the deterministic scatter of a node-sorted E-vector: v[t_offset[k] + c * comp_stride] (+)= sum over j in
+// [t_rowptr[k], t_rowptr[k+1]) of ev[j * ncomp + c] in ascending j.
+hipError_t launch_node_gather(int nrows, int ncomp, int comp_stride, const int *t_rowptr, const int *t_offset, const double *ev, double *v,
+                              bool overwrite, hipStream_t s);
+// The same for an element-ordered E-vector [elem node][5], FP64 (ev) or FP32 (ev32, summed in FP64).  Tile t holds the rows
+// tile_row[t] .. tile_row[t+1]-1; slot[j], j over the rows' range of t_rowptr, are the tile's element nodes in ascending
+// order, and pos[j] is the place in that order of the j-th one in row order.  Row k's offset is k stride, or toff[k].
+constexpr int kGatherSlots = 512;
+struct GatherTiles {
+  int                   ntile, stride;
+  const int            *tile_row, *rowptr, *slot, *toff;
+  const unsigned short *pos;
+};
+hipError_t launch_node_gather_tiles(const GatherTiles &g, int comp_stride, const double *ev, const float *ev32, double *v, bool overwrite,
+                                    hipStream_t s);
 // The same for 5 x 5 point blocks: v[25 (t_offset[k] / 5) + i] += sum over the node's slots of ev[t_index[j] * 25 + i]
-// Two-pass scatter with an FP32 element-ordered E-vector [elem node][5]: sums per node in FP64, in slot order
-hipError_t launch_node_gather_rows_f32(int nrows, int comp_stride, const int *t_rowptr, const int *t_index, const int *t_offset, const float *ev,
-                                      double *v, bool overwrite, hipStream_t s);
 hipError_t launch_node_gather_blocks(int nrows, const int *t_rowptr, const int *t_index, const int *t_offset, const double *ev, double *v,
                                      hipStream_t s);
 hipError_t launch_restriction_transpose(const int *offsets, int nelem, int elemsize, int ncomp, int comp_stride, const double *e, double *u, hipStream_t s);

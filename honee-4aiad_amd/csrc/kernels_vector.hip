@@ -75,14 +75,12 @@ __global__ void k_rstr_t(const int *off, int nelem, int esize, int ncomp, int cs
 }
 
 // Deterministic second scatter pass: one thread per (L-vector node, component) item.  Row k's contributions are the
-// E-vector slots t_rowptr[k] .. t_rowptr[k+1]-1 (node-sorted E-vector) or the slots index[] of that range
-// (element-ordered E-vector); they are summed in ascending order.  Each thread handles NPT items a grid stride apart
+// E-vector slots t_rowptr[k] .. t_rowptr[k+1]-1 (node-sorted E-vector); they are summed in ascending order.  Each thread handles NPT items a grid stride apart
 // and issues all their row-pointer loads, then all their contribution loads (up to 8 per row, the most a hexahedral
 // mesh node has), so a thread waits on two memory round trips for NPT items.
-template <bool INDEXED, int NPT>
-__global__ void __launch_bounds__(256) k_node_gather(int nrows, int ncomp, int cs, const int *__restrict__ rowptr, const int *__restrict__ index,
-                                                     const int *__restrict__ toff, const double *__restrict__ ev, double *__restrict__ v,
-                                                     bool overwrite) {
+template <int NPT>
+__global__ void __launch_bounds__(256) k_node_gather(int nrows, int ncomp, int cs, const int *__restrict__ rowptr, const int *__restrict__ toff,
+                                                     const double *__restrict__ ev, double *__restrict__ v, bool overwrite) {
   const long long n      = (long long)nrows * ncomp;
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += stride * NPT) {
@@ -108,7 +106,7 @@ __global__ void __launch_bounds__(256) k_node_gather(int nrows, int ncomp, int c
 #pragma unroll
         for (int k = 0; k < 8; k++) {
           x[j][k] = 0;
-          if (k < m[j]) x[j][k] = ev[(INDEXED ? (long long)index[b[j] + k] : (long long)(b[j] + k)) * ncomp + c[j]];
+          if (k < m[j]) x[j][k] = ev[(long long)(b[j] + k) * ncomp + c[j]];
         }
 #pragma unroll
       for (int j = 0; j < NPT; j++)
@@ -118,7 +116,7 @@ __global__ void __launch_bounds__(256) k_node_gather(int nrows, int ncomp, int c
     } else {
 #pragma unroll
       for (int j = 0; j < NPT; j++)
-        for (int k = 0; k < m[j]; k++) acc[j] += ev[(INDEXED ? (long long)index[b[j] + k] : (long long)(b[j] + k)) * ncomp + c[j]];
+        for (int k = 0; k < m[j]; k++) acc[j] += ev[(long long)(b[j] + k) * ncomp + c[j]];
     }
 #pragma unroll
     for (int j = 0; j < NPT; j++) {
@@ -130,53 +128,61 @@ __global__ void __launch_bounds__(256) k_node_gather(int nrows, int ncomp, int c
   }
 }
 
-// The same sum for the element-ordered E-vector, one thread per L-vector node: each contribution is the node's NC
-// consecutive values in its element's block (40 contiguous bytes for 5 components), read whole; the sums run over the
-// slots in ascending order, as in k_node_gather (identical results).  Measured at 32^3 p=3: 50 us against 49-57 us for
-// one thread per (node, component) in node or in element order.
-// The rows are split into 8 contiguous ranges, one per XCD (block b runs on XCD b % 8; the grid is a multiple of 8):
-// the nodes of one range belong to a contiguous range of elements, whose E-vector lines are then fetched into one XCD's
-// L2 instead of into several.
+// The same sum for the element-ordered E-vector of 5 components, a tile of consecutive rows per block.  The block loads the
+// tile's slots in ascending address order, lanes along the 40 bytes of a slot and on to the next, so that each line is asked
+// for by one or two wave loads; it then sums each (row, component) from LDS over the row's slots in ascending order, as in
+// k_node_gather (identical results).  A thread per row that reads its slots straight from memory asks for each line 5 to 10
+// times and spends the time on requests that wait for a line already on its way (measured: 0.9 of the cycles, and L2 to L1
+// traffic of 4.7 times the E-vector at p=2).
+// Tiles hold at most kGatherSlots slots (20 KB of LDS: 7 blocks a CU) and as many rows; a row with more slots is a tile by
+// itself, summed straight from memory.  The tiles are split into 8 contiguous ranges, one per XCD (block b runs on XCD
+// b % 8; the grid is a multiple of 8), so that a range's E-vector lines go to one L2.
+// Measured against a thread per row: 64^3 p=2 177 -> 122 us (3.4 TB/s), 40^3 p=4 196 -> 158 us, 32^3 p=3 50 -> 44 us.
 // E is the E-vector's type: double, or float for the FP32 Jacobian's contributions (summed in FP64 here).
-template <int NC, typename E>
-__global__ void __launch_bounds__(512) k_node_gather_rows(int nrows, int cs, const int *__restrict__ rowptr, const int *__restrict__ index,
-                                                          const int *__restrict__ toff, const E *__restrict__ ev, double *__restrict__ v,
-                                                          bool overwrite) {
-  const long long per = ((long long)nrows + 7) / 8;
-  const long long x = blockIdx.x % 8, j = blockIdx.x / 8, nb = gridDim.x / 8;
-  const long long lo = x * per, hi = (x + 1) * per < nrows ? (x + 1) * per : nrows;
-  for (long long row = lo + j * blockDim.x + threadIdx.x; row < hi; row += nb * blockDim.x) {
-    const int b = rowptr[row], m = rowptr[row + 1] - b;
-    double    acc[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = 0;
-    if (m <= 8) {  // at most 8 contributions (a hexahedral mesh node): all slot indices, then all values
-      int slot[8];
-#pragma unroll
-      for (int k = 0; k < 8; k++) slot[k] = k < m ? index[b + k] : 0;
-      double x[8][NC];
-#pragma unroll
-      for (int k = 0; k < 8; k++)
-#pragma unroll
-        for (int c = 0; c < NC; c++) x[k][c] = k < m ? (double)ev[(long long)slot[k] * NC + c] : 0.0;
-#pragma unroll
-      for (int k = 0; k < 8; k++)
-        if (k < m)
-#pragma unroll
-          for (int c = 0; c < NC; c++) acc[c] += x[k][c];
-    } else {
-      for (int k = 0; k < m; k++) {
-        const long long sl = index[b + k];
-#pragma unroll
-        for (int c = 0; c < NC; c++) acc[c] += (double)ev[sl * NC + c];
-      }
+template <typename E>
+__global__ void __launch_bounds__(256) k_node_gather_tiles(GatherTiles g, int cs, const E *__restrict__ ev, double *__restrict__ v, bool overwrite) {
+  constexpr int NC = 5, NT = 256, NL = kGatherSlots * NC / NT;
+  __shared__ E              buf[kGatherSlots * NC];
+  __shared__ unsigned short pos[kGatherSlots];
+  __shared__ int            first[kGatherSlots + 1];
+  const int per = (g.ntile + 7) / 8, tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if ((int)(blockIdx.x / 8) >= per || tile >= g.ntile) return;
+  const int r0 = g.tile_row[tile], nr = g.tile_row[tile + 1] - r0, j0 = g.rowptr[r0], m = g.rowptr[r0 + nr] - j0, tid = threadIdx.x;
+  auto store = [&](int row, int c, double acc) {
+    const long long o = (g.stride ? (long long)row * g.stride : (long long)g.toff[row]) + (long long)c * cs;
+    v[o]              = overwrite ? acc : v[o] + acc;
+  };
+  if (m > kGatherSlots) {  // one row
+    if (tid < NC) {
+      double acc = 0;
+      for (int k = 0; k < m; k++) acc += (double)ev[(long long)g.slot[j0 + k] * NC + tid];
+      store(r0, tid, acc);
     }
-    const long long o = toff[row];
+    return;
+  }
+  int s[NL];
+  E   x[NL];
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-      double *dst = &v[o + (long long)c * cs];
-      *dst        = overwrite ? acc[c] : *dst + acc[c];
-    }
+  for (int u = 0; u < NL; u++) {
+    const int i = tid + u * NT;
+    s[u]        = i < m * NC ? g.slot[j0 + i / NC] : 0;
+  }
+#pragma unroll
+  for (int u = 0; u < NL; u++) {
+    const int i = tid + u * NT;
+    x[u]        = i < m * NC ? ev[(long long)s[u] * NC + i % NC] : (E)0;
+  }
+  for (int i = tid; i <= nr; i += NT) first[i] = g.rowptr[r0 + i] - j0;
+  for (int i = tid; i < m; i += NT) pos[i] = (unsigned short)(g.pos[j0 + i] * NC);
+#pragma unroll
+  for (int u = 0; u < NL; u++)
+    if (tid + u * NT < m * NC) buf[tid + u * NT] = x[u];
+  __syncthreads();
+  for (int i = tid; i < nr * NC; i += NT) {
+    const int row = i / NC, c = i % NC, end = first[row + 1];
+    double    acc = 0;
+    for (int k = first[row]; k < end; k++) acc += (double)buf[pos[k] + c];
+    store(r0 + row, c, acc);
   }
 }
 
@@ -322,34 +328,24 @@ hipError_t launch_cg_update(const CgArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_node_gather(int nrows, int ncomp, int comp_stride, const int *t_rowptr, const int *t_index, const int *t_offset,
-                              const double *ev, double *v, bool overwrite, hipStream_t s) {
+hipError_t launch_node_gather(int nrows, int ncomp, int comp_stride, const int *t_rowptr, const int *t_offset, const double *ev, double *v,
+                              bool overwrite, hipStream_t s) {
   constexpr int   NPT = 2;  // measured: 2 items per thread 31.8 us against 39.1 us (1) and 39.0 us (4) at 884,736 rows
   const long long n   = (long long)nrows * ncomp;
   if (n <= 0) return hipSuccess;
-  if (t_index && ncomp == 5) {  // element-ordered E-vector: one thread per node, 8 row ranges (one per XCD)
-    // 512-thread blocks: 49.4 us against 50.6 us (256) and 50.3 us (128) at 884,736 rows, two A/B pairs
-    constexpr int kRowsBlock = 512;
-    const int     grid       = (int)(((nrows + kRowsBlock - 1) / kRowsBlock + 7) / 8 * 8);
-    hipLaunchKernelGGL((k_node_gather_rows<5, double>), dim3(grid), dim3(kRowsBlock), 0, s, nrows, comp_stride, t_rowptr, t_index, t_offset, ev, v,
-                       overwrite);
-    return hipGetLastError();
-  }
   const int grid = grid_for((n + NPT - 1) / NPT);
-  if (t_index)
-    hipLaunchKernelGGL((k_node_gather<true, NPT>), dim3(grid), dim3(kBlock), 0, s, nrows, ncomp, comp_stride, t_rowptr, t_index, t_offset, ev, v,
-                       overwrite);
-  else
-    hipLaunchKernelGGL((k_node_gather<false, NPT>), dim3(grid), dim3(kBlock), 0, s, nrows, ncomp, comp_stride, t_rowptr, t_index, t_offset, ev,
-                       v, overwrite);
+  hipLaunchKernelGGL((k_node_gather<NPT>), dim3(grid), dim3(kBlock), 0, s, nrows, ncomp, comp_stride, t_rowptr, t_offset, ev, v, overwrite);
   return hipGetLastError();
 }
 
-hipError_t launch_node_gather_rows_f32(int nrows, int comp_stride, const int *t_rowptr, const int *t_index, const int *t_offset, const float *ev,
-                                      double *v, bool overwrite, hipStream_t s) {
-  if (nrows <= 0) return hipSuccess;
-  const int grid = (grid_for(nrows) + 7) / 8 * 8;
-  hipLaunchKernelGGL((k_node_gather_rows<5, float>), dim3(grid), dim3(kBlock), 0, s, nrows, comp_stride, t_rowptr, t_index, t_offset, ev, v, overwrite);
+hipError_t launch_node_gather_tiles(const GatherTiles &g, int comp_stride, const double *ev, const float *ev32, double *v, bool overwrite,
+                                    hipStream_t s) {
+  if (g.ntile <= 0) return hipSuccess;
+  const dim3 grid((g.ntile + 7) / 8 * 8);
+  if (ev32)
+    hipLaunchKernelGGL((k_node_gather_tiles<float>), grid, dim3(256), 0, s, g, comp_stride, ev32, v, overwrite);
+  else
+    hipLaunchKernelGGL((k_node_gather_tiles<double>), grid, dim3(256), 0, s, g, comp_stride, ev, v, overwrite);
   return hipGetLastError();
 }
 
