@@ -240,9 +240,11 @@ int lincomb(HoneeMiTS ts, double *y, double a, const std::vector<double> &c, con
   return 0;
 }
 
-// Left-preconditioned GMRES(restart), zero initial guess (see the file header); apply(x, y) computes y = A x.
+// Left-preconditioned GMRES(restart), zero initial guess (see the file header); apply(x, y) computes y = A x and counts itself
+// in *applies.  ahead: apply only launches, so that the next one can be launched before the host has read the present step.
 template <class Apply, class Prec>
-int gmres(HoneeMiTS ts, Apply apply, Prec prec, const double *b, double *x, double rtol, double atol, int restart, int maxit, int *its_out) {
+int gmres(HoneeMiTS ts, Apply apply, long long *applies, bool ahead, Prec prec, const double *b, double *x, double rtol, double atol, int restart,
+          int maxit, int *its_out) {
   const long long     n = ts->n;
   const int           K = restart;
   std::vector<double> H((size_t)(K + 1) * (K + 1), 0.0), cc(K + 1, 0.0), ss(K + 1, 0.0), grs(K + 2, 0.0), nrs(K + 1, 0.0);
@@ -260,24 +262,29 @@ int gmres(HoneeMiTS ts, Apply apply, Prec prec, const double *b, double *x, doub
     }
     // ||V_0||, with V_0 normalized on the device while the host reads the norm
     const Publish pub = next_publish(ts, 1);
-    TS_HIP(ts, launch_dot(V, V, n, 0, ts->partial, ts->d_red, ts->s, pub));
-    TS_HIP(ts, launch_normalize(V, ts->d_red, n, ts->s));
+    TS_HIP(ts, launch_dot_partial(V, V, n, 0, ts->partial, ts->s));
+    TS_HIP(ts, launch_normalize(V, ts->partial, 0, ts->d_red, n, ts->s, pub));
     TS_CALL(wait_published(ts, pub));
     double res = std::sqrt(ts->h_red[0]);
     if (its == 0) ttol = std::fmax(rtol * res, atol);
     if (res <= ttol) break;
     grs[0] = res;
-    int it = 0;
+    int  it      = 0;
+    bool applied = false;  // w = A V_it is already on its way
     while (it < K && its < maxit) {
       double *v_new = V + (size_t)(it + 1) * n;
-      TS_CALL(apply(V + (size_t)it * n, ts->w));
+      if (!applied) TS_CALL(apply(V + (size_t)it * n, ts->w));
       TS_CALL(prec(v_new, ts->w, nullptr));
       // classical Gram-Schmidt: all dots first, then one projection pass that also forms ||v_new||^2; v_new is
       // normalized on the device while the host reads (h_0..h_it, ||v_new||^2)
-      TS_HIP(ts, launch_mdot(v_new, V, n, it + 1, n, ts->partial, ts->d_red, ts->s));
+      TS_HIP(ts, launch_mdot(v_new, V, n, it + 1, n, ts->partial, ts->s));
       const Publish pub = next_publish(ts, it + 2);
-      TS_HIP(ts, launch_project_out(v_new, V, n, it + 1, ts->d_red, n, it + 1, ts->partial, ts->d_red, ts->s, pub));
-      TS_HIP(ts, launch_normalize(v_new, ts->d_red + it + 1, n, ts->s));
+      TS_HIP(ts, launch_project_out(v_new, V, n, it + 1, n, it + 1, ts->partial, ts->d_red, ts->s));
+      TS_HIP(ts, launch_normalize(v_new, ts->partial, it + 1, ts->d_red, n, ts->s, pub));
+      // the next operator apply needs nothing from the host and changes nothing that is returned: it runs while the host
+      // reads.  Where this step converges it is in vain and not counted.
+      applied = ahead && it + 1 < K && its + 1 < maxit;
+      if (applied) TS_CALL(apply(v_new, ts->w));
       TS_CALL(wait_published(ts, pub));
       for (int j = 0; j <= it; j++) HH(j, it) = ts->h_red[j];
       HH(it + 1, it) = std::sqrt(ts->h_red[it + 1]);
@@ -297,6 +304,7 @@ int gmres(HoneeMiTS ts, Apply apply, Prec prec, const double *b, double *x, doub
       its++;
       if (res <= ttol) {
         converged = 1;
+        if (applied) --*applies;
         break;
       }
     }
@@ -374,7 +382,7 @@ int mass_solve(HoneeMiTS ts, const double *state, const double *r, double *k) {
     return 0;
   };
   int its = 0;
-  TS_CALL(gmres(ts, apply, prec, r, k, ts->o.mass_rtol, 1e-50, ts->o.mass_restart, ts->o.mass_max_it, &its));
+  TS_CALL(gmres(ts, apply, &ts->st.mass_applies, true, prec, r, k, ts->o.mass_rtol, 1e-50, ts->o.mass_restart, ts->o.mass_max_it, &its));
   ts->st.mass_krylov_its += its;
   return 0;
 }
@@ -498,7 +506,9 @@ int newton_solve(HoneeMiTS ts, double tnew) {
     }
     int kits = 0;
     if (o.snes_mf_operator) TS_CALL(norm2(ts, ts->x, &xnorm_mf));
-    TS_CALL(gmres(ts, apply, Precond{ts, ts->dinv, block}, ts->F, ts->dx, o.ksp_rtol, o.ksp_atol, o.ksp_restart, o.ksp_max_it, &kits));
+    // a finite-difference product reads a norm on the host: it cannot run ahead of the one that the step waits for
+    TS_CALL(gmres(ts, apply, &ts->st.jacobian_applies, !o.snes_mf_operator, Precond{ts, ts->dinv, block}, ts->F, ts->dx, o.ksp_rtol, o.ksp_atol,
+                  o.ksp_restart, o.ksp_max_it, &kits));
     ts->st.krylov_its += kits;
     ts->st.last_krylov_its += kits;
     // SNESLINESEARCHBT (cubic order, alpha 1e-4, minlambda 1e-12, 40 steps) along -dx, as SNESLineSearchApply_BT:

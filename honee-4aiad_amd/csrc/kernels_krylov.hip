@@ -1,111 +1,215 @@
 // Vector kernels of the time integrator and its Krylov solvers (GMRES with point-Jacobi, Newton, explicit RK).
 //
 // Reductions are deterministic: a grid of fixed size (a function of the length only) reduces contiguous grid-stride
-// slices per block in a fixed tree order into partials[slot][block] (slot-major, so that the second pass reads each
-// slot's partials contiguously), and a second kernel sums each slot over the blocks in a fixed order.  The same inputs
-// give bitwise identical results from run to run.
+// slices per block in a fixed tree order into partials[slot][block] (slot-major, so that a consumer reads each slot's
+// partials contiguously).  The kernel that needs a sum adds the at most 256 partials itself, every block alike and in the
+// same order (2 KB per sum out of L2), which costs no launch between; a sum that only the host needs has a last kernel.  The
+// same inputs give bitwise identical results from run to run.
 //
-// Multi-dot: the dots of w with up to kMaxDots basis vectors are taken in groups of 8 (w is read once per group).
-// Projection update: w -= sum_j h_j V_j with the h_j read from device memory (the reduced dots), fused with the
-// partial sums of ||w||^2, so that one Arnoldi step needs a single host read of (h_0..h_k, ||w||^2), which the final
-// reduction kernel stores into mapped host memory (Publish).
+// One Arnoldi step is three launches: the dots of w with all basis vectors, w -= sum_j h_j V_j with the partial sums of
+// ||w||^2, and w /= ||w||, whose first block also stores (h_0..h_k, ||w||^2) into mapped host memory (Publish) for the
+// step's single host read.
 #include <hip/hip_runtime.h>
 
 #include "krylov.hpp"
 
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = 256, kRed = 512;  // threads of an elementwise kernel's block, of a reduction's
 
-__device__ __forceinline__ double block_sum(double v, double *s) {
-  s[threadIdx.x] = v;
-  __syncthreads();
+__device__ __forceinline__ double wave_sum(double v) {  // to all lanes
 #pragma unroll
-  for (int w = kThreads / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  const double r = s[0];
+  for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w);
+  return v;
+}
+// Sum over the block in thread 0; s holds a value per wave
+__device__ __forceinline__ double block_sum(double v, double *s) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
   __syncthreads();
+  double r = 0;
+  if (threadIdx.x == 0)
+    for (int i = 0; i < (int)blockDim.x / 64; i++) r += s[i];
   return r;
 }
-
-// partial[j0 + j][block] = sum over this block's slice of w[i] V[(j0 + j) ldv + i], j < nj <= 8
-__global__ void __launch_bounds__(kThreads) k_mdot8(const double *__restrict__ w, const double *__restrict__ V, long long ldv, int j0, int nj,
-                                                    long long n, double *__restrict__ partial) {
-  __shared__ double s[kThreads];
-  double            acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  const long long   stride = (long long)gridDim.x * kThreads;
-  for (long long i = (long long)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
-    const double wi = w[i];
+// A slot's total, in every wave that asks alike
+__device__ __forceinline__ double slot_total(const double *__restrict__ partial, int slot, int nb) {
+  double x[kMaxReductionBlocks / 64];
 #pragma unroll
-    for (int j = 0; j < 8; j++)
-      if (j < nj) acc[j] += wi * V[(long long)(j0 + j) * ldv + i];
+  for (int i = 0; i < kMaxReductionBlocks / 64; i++) {
+    const int b = i * 64 + (int)(threadIdx.x & 63);
+    x[i]        = b < nb ? partial[(long long)slot * kMaxReductionBlocks + b] : 0.0;
   }
+  double v = 0;
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    if (j >= nj) break;
-    const double r = block_sum(acc[j], s);
-    if (threadIdx.x == 0) partial[(long long)(j0 + j) * kMaxReductionBlocks + blockIdx.x] = r;
+  for (int i = 0; i < kMaxReductionBlocks / 64; i++) v += x[i];
+  return wave_sum(v);
+}
+// The 8 sums over the wave of a[0..7]: lane l returns that of a[l >> 3].  At each of the first three steps a lane keeps half of
+// its sums and gives the others away: 10 exchanges instead of 48.
+__device__ __forceinline__ double wave_sum8(const double (&a)[8]) {
+  const bool b5 = threadIdx.x & 32, b4 = threadIdx.x & 16, b3 = threadIdx.x & 8;
+  double     x[4], y[2];
+#pragma unroll
+  for (int j = 0; j < 4; j++) x[j] = (b5 ? a[j + 4] : a[j]) + __shfl_xor(b5 ? a[j] : a[j + 4], 32);
+#pragma unroll
+  for (int j = 0; j < 2; j++) y[j] = (b4 ? x[j + 2] : x[j]) + __shfl_xor(b4 ? x[j] : x[j + 2], 16);
+  double z = (b3 ? y[1] : y[0]) + __shfl_xor(b3 ? y[0] : y[1], 8);
+#pragma unroll
+  for (int w = 4; w > 0; w >>= 1) z += __shfl_xor(z, w);
+  return z;
+}
+// Store out[0 .. count) into mapped host memory, slot's value being r, then the sequence number; one block of >= count threads
+__device__ __forceinline__ void publish(const Publish &pub, const double *out, int slot, double r) {
+  const int i = threadIdx.x;
+  if (i < pub.count) pub.h[i] = i == slot ? r : out[i];  // the other slots come from earlier launches
+  __threadfence_system();  // each thread's value reaches host memory before the sequence number
+  __syncthreads();
+  if (i == 0) __hip_atomic_store(pub.flag, pub.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// partial[j][block] = sum over this block's slice of w[i] V[j ldv + i], j < k, 8 vectors to a row of blocks (w is read once per
+// row, 1/8 of the bytes, and the rows share the latency).
+// Bound by the basis vectors' bytes (L2 and the memory-side cache hold those of a small problem).  Measured at 553 k entries,
+// 10.5 vectors on average: 12.6 us; with a launch for every 8 vectors, a tree of barriers for every sum and a kernel that adds
+// the partials, 26 us.
+__global__ void __launch_bounds__(kRed) k_mdot(const double *__restrict__ w, const double *__restrict__ V, long long ldv, int k, long long n,
+                                               double *__restrict__ partial) {
+  __shared__ double s[8][kRed / 64];
+  const int         j0 = 8 * blockIdx.y, nj = k - j0 < 8 ? k - j0 : 8;
+  const long long   stride = (long long)gridDim.x * kRed, i0 = (long long)blockIdx.x * kRed + threadIdx.x;
+  double            acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  V += (long long)j0 * ldv;
+  if (nj == 8) {
+#pragma unroll 2
+    for (long long i = i0; i < n; i += stride) {
+      const double wi = w[i];
+#pragma unroll
+      for (int j = 0; j < 8; j++) acc[j] += wi * V[(long long)j * ldv + i];
+    }
+  } else {
+#pragma unroll 2
+    for (long long i = i0; i < n; i += stride) {
+      const double wi = w[i];
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if (j < nj) acc[j] += wi * V[(long long)j * ldv + i];
+    }
+  }
+  const double r = wave_sum8(acc);
+  if ((threadIdx.x & 7) == 0) s[(threadIdx.x >> 3) % 8][threadIdx.x >> 6] = r;
+  __syncthreads();
+  if ((int)threadIdx.x < nj) {
+    double t = 0;
+#pragma unroll
+    for (int i = 0; i < kRed / 64; i++) t += s[threadIdx.x][i];
+    partial[(long long)(j0 + threadIdx.x) * kMaxReductionBlocks + blockIdx.x] = t;
   }
 }
 
 // partial[slot][block] = sum over this block's slice of x[i] y[i]
-__global__ void __launch_bounds__(kThreads) k_dot(const double *__restrict__ x, const double *__restrict__ y, long long n, int slot,
-                                                  double *__restrict__ partial) {
-  __shared__ double s[kThreads];
+__global__ void __launch_bounds__(kRed) k_dot(const double *__restrict__ x, const double *__restrict__ y, long long n, int slot,
+                                              double *__restrict__ partial) {
+  __shared__ double s[kRed / 64];
   double            acc    = 0;
-  const long long   stride = (long long)gridDim.x * kThreads;
-  for (long long i = (long long)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) acc += x[i] * y[i];
+  const long long   stride = (long long)gridDim.x * kRed;
+#pragma unroll 4
+  for (long long i = (long long)blockIdx.x * kRed + threadIdx.x; i < n; i += stride) acc += x[i] * y[i];
   const double r = block_sum(acc, s);
   if (threadIdx.x == 0) partial[(long long)slot * kMaxReductionBlocks + blockIdx.x] = r;
 }
 
-// w[i] -= sum_{j < k} h[j] V[j ldv + i] (in order j = 0, 1, ...); partial[slot][block] = sum of the new w[i]^2
-__global__ void __launch_bounds__(kThreads) k_project_out(double *__restrict__ w, const double *__restrict__ V, long long ldv, int k,
-                                                          const double *__restrict__ h, long long n, int slot, double *__restrict__ partial) {
-  __shared__ double s[kThreads];
+// acc[u] + SIGN sum_{j < k} c[j] V[j ldv + i + u stride] in the order j = 0, 1, ..., the loads of 8 vectors in flight
+template <int SIGN, int U>
+__device__ __forceinline__ void basis_sum(double (&acc)[U], const double *c, const double *__restrict__ V, long long ldv, int k, long long i,
+                                          long long stride) {
+  int j = 0;
+  for (; j + 8 <= k; j += 8) {
+    double v[U][8];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int l = 0; l < 8; l++) v[u][l] = V[(long long)(j + l) * ldv + i + u * stride];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int l = 0; l < 8; l++) acc[u] += SIGN * c[j + l] * v[u][l];
+  }
+  double v[U][8];
+#pragma unroll
+  for (int u = 0; u < U; u++)
+#pragma unroll
+    for (int l = 0; l < 8; l++) v[u][l] = j + l < k ? V[(long long)(j + l) * ldv + i + u * stride] : 0.0;
+#pragma unroll
+  for (int u = 0; u < U; u++)
+#pragma unroll
+    for (int l = 0; l < 8; l++)
+      if (j + l < k) acc[u] += SIGN * c[j + l] * v[u][l];
+}
+
+// out[j] = sum of partial[j][0 .. nb), j < k; w[i] -= sum_{j < k} out[j] V[j ldv + i] (in order j = 0, 1, ...);
+// partial[slot][block] = sum of the new w[i]^2.  slot >= k: a block may overwrite no partials that another one still reads.
+// Bound as k_mdot; measured there 12.3 us and 6.0 us for k_normalize, 11.4 + 3.6 us with a kernel of 4.1 us between them.
+__global__ void __launch_bounds__(kRed) k_project_out(double *__restrict__ w, const double *__restrict__ V, long long ldv, int k, long long n,
+                                                          int slot, double *__restrict__ partial, int nb, double *__restrict__ out) {
+  __shared__ double s[kRed / 64];
   __shared__ double c[kMaxDots];
-  if ((int)threadIdx.x < k) c[threadIdx.x] = h[threadIdx.x];
+  for (int j = threadIdx.x >> 6; j < k; j += kRed / 64) {
+    const double h = slot_total(partial, j, nb);
+    if ((threadIdx.x & 63) == 0) {
+      c[j] = h;
+      if (blockIdx.x == 0) out[j] = h;
+    }
+  }
   __syncthreads();
   double          ss     = 0;
-  const long long stride = (long long)gridDim.x * kThreads;
-  for (long long i = (long long)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
-    double acc = w[i];
-    for (int j = 0; j < k; j++) acc -= c[j] * V[(long long)j * ldv + i];
-    w[i] = acc;
-    ss += acc * acc;
+  const long long stride = (long long)gridDim.x * kRed;
+  long long       i      = (long long)blockIdx.x * kRed + threadIdx.x;
+  for (; i + stride < n; i += 2 * stride) {
+    double acc[2] = {w[i], w[i + stride]};
+    basis_sum<-1>(acc, c, V, ldv, k, i, stride);
+    w[i]          = acc[0];
+    w[i + stride] = acc[1];
+    ss += acc[0] * acc[0] + acc[1] * acc[1];
+  }
+  if (i < n) {
+    double acc[1] = {w[i]};
+    basis_sum<-1>(acc, c, V, ldv, k, i, stride);
+    w[i] = acc[0];
+    ss += acc[0] * acc[0];
   }
   const double r = block_sum(ss, s);
   if (threadIdx.x == 0) partial[(long long)slot * kMaxReductionBlocks + blockIdx.x] = r;
 }
 
-// out[slot] = sum over blocks b (in order) of partial[slot][b], for slots [s0, s0 + gridDim.x).  A single-block launch
-// with pub.h set then stores out[0 .. pub.count) into mapped host memory and pub.seq into *pub.flag (Publish).
-__global__ void __launch_bounds__(kThreads) k_reduce_partials(const double *__restrict__ partial, int nblocks, int s0, double *__restrict__ out,
-                                                              Publish pub) {
-  __shared__ double s[kThreads];
-  const int         slot = s0 + blockIdx.x;
-  double            acc  = 0;
-  for (int b = threadIdx.x; b < nblocks; b += kThreads) acc += partial[(long long)slot * kMaxReductionBlocks + b];
-  const double r = block_sum(acc, s);
+// out[slot] = sum over blocks b (in order) of partial[slot][b] (one wave); with pub.h set out[0 .. pub.count) is then published
+__global__ void __launch_bounds__(64) k_reduce_partials(const double *__restrict__ partial, int nb, int slot, double *__restrict__ out, Publish pub) {
+  const double r = slot_total(partial, slot, nb);
   if (threadIdx.x == 0) out[slot] = r;
-  if (pub.h) {
-    const int i = threadIdx.x;
-    if (i < pub.count) pub.h[i] = i == slot ? r : out[i];  // the other slots come from earlier launches
-    __threadfence_system();  // each thread's value reaches host memory before the sequence number
-    __syncthreads();
-    if (i == 0) __hip_atomic_store(pub.flag, pub.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+  if (pub.h) publish(pub, out, slot, r);
 }
 
-// y = y / sqrt(*hsq) unless *hsq is zero (a Krylov vector normalized by its squared norm in device memory)
-__global__ void __launch_bounds__(kThreads) k_normalize(double *__restrict__ y, const double *__restrict__ hsq, long long n) {
-  const double h = *hsq;
+// out[slot] = sum of partial[slot][0 .. nb), published with out[0 .. pub.count); y = y / sqrt(out[slot]) unless that is zero
+// (a Krylov vector normalized by its squared norm)
+constexpr int kNormalize = 4;  // entries a thread
+__global__ void __launch_bounds__(kThreads) k_normalize(double *__restrict__ y, const double *__restrict__ partial, int nb, int slot,
+                                                        double *__restrict__ out, long long n, Publish pub) {
+  // the first entries are on their way while the partials come
+  const long long stride = (long long)gridDim.x * kThreads, i0 = (long long)blockIdx.x * kThreads + threadIdx.x;
+  double          x[kNormalize];
+#pragma unroll
+  for (int u = 0; u < kNormalize; u++) x[u] = i0 + u * stride < n ? y[i0 + u * stride] : 0.0;
+  const double h = slot_total(partial, slot, nb);
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) out[slot] = h;
+    if (pub.h) publish(pub, out, slot, h);
+  }
   if (h == 0) return;
-  const double    a      = 1.0 / sqrt(h);
-  const long long stride = (long long)gridDim.x * kThreads;
-  for (long long i = (long long)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) y[i] = a * y[i];
+  const double a = 1.0 / sqrt(h);
+#pragma unroll
+  for (int u = 0; u < kNormalize; u++)
+    if (i0 + u * stride < n) y[i0 + u * stride] = a * x[u];
+  for (long long i = i0 + kNormalize * stride; i < n; i += stride) y[i] = a * y[i];
 }
 
 // y[i] = a y[i] + sum_{j < m} c_j X_j[i]
@@ -122,9 +226,9 @@ __global__ void __launch_bounds__(kThreads) k_lincomb(double *__restrict__ y, do
 __global__ void __launch_bounds__(kThreads) k_basis_comb(double *__restrict__ y, const double *__restrict__ V, long long ldv, Coefs cf, long long n) {
   const long long stride = (long long)gridDim.x * kThreads;
   for (long long i = (long long)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
-    double acc = y[i];
-    for (int j = 0; j < cf.k; j++) acc += cf.c[j] * V[(long long)j * ldv + i];
-    y[i] = acc;
+    double acc[1] = {y[i]};
+    basis_sum<1>(acc, cf.c, V, ldv, cf.k, i, stride);
+    y[i] = acc[0];
   }
 }
 
@@ -147,11 +251,12 @@ __global__ void __launch_bounds__(kThreads) k_set(double *__restrict__ x, double
 }
 
 // partial[slot][block] = number of non-finite entries in the block's slice (as a double)
-__global__ void __launch_bounds__(kThreads) k_count_nonfinite(const double *__restrict__ x, long long n, int slot, double *__restrict__ partial) {
-  __shared__ double s[kThreads];
+__global__ void __launch_bounds__(kRed) k_count_nonfinite(const double *__restrict__ x, long long n, int slot, double *__restrict__ partial) {
+  __shared__ double s[kRed / 64];
   double            cnt    = 0;
-  const long long   stride = (long long)gridDim.x * kThreads;
-  for (long long i = (long long)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) cnt += isfinite(x[i]) ? 0.0 : 1.0;
+  const long long   stride = (long long)gridDim.x * kRed;
+#pragma unroll 4
+  for (long long i = (long long)blockIdx.x * kRed + threadIdx.x; i < n; i += stride) cnt += isfinite(x[i]) ? 0.0 : 1.0;
   const double r = block_sum(cnt, s);
   if (threadIdx.x == 0) partial[(long long)slot * kMaxReductionBlocks + blockIdx.x] = r;
 }
@@ -160,7 +265,7 @@ __global__ void __launch_bounds__(kThreads) k_count_nonfinite(const double *__re
 // pivoting on [A | I]; every index is a compile-time constant so the blocks stay in registers.
 // partial[slot][block] counts the singular blocks of the block's slice.
 __global__ void __launch_bounds__(kThreads) k_pb_invert(double *__restrict__ pb, long long nn, int slot, double *__restrict__ partial) {
-  __shared__ double s[kThreads];
+  __shared__ double s[kThreads / 64];
   double            bad    = 0;
   const long long   stride = (long long)gridDim.x * kThreads;
   for (long long node = (long long)blockIdx.x * kThreads + threadIdx.x; node < nn; node += stride) {
@@ -247,41 +352,41 @@ int elementwise_grid(long long n) {
 }  // namespace
 
 int krylov_reduction_blocks(long long n) {
-  long long g = (n + kThreads - 1) / kThreads;
+  long long g = (n + kRed - 1) / kRed;
   if (g > kMaxReductionBlocks) g = kMaxReductionBlocks;
   return g < 1 ? 1 : (int)g;
 }
 
-hipError_t launch_mdot(const double *w, const double *V, long long ldv, int k, long long n, double *partial, double *out, hipStream_t s) {
+hipError_t launch_mdot(const double *w, const double *V, long long ldv, int k, long long n, double *partial, hipStream_t s) {
   if (k < 1 || k > kMaxDots) return hipErrorInvalidValue;
-  const int nb = krylov_reduction_blocks(n);
-  for (int j0 = 0; j0 < k; j0 += 8) {
-    const int nj = k - j0 < 8 ? k - j0 : 8;
-    hipLaunchKernelGGL(k_mdot8, dim3(nb), dim3(kThreads), 0, s, w, V, ldv, j0, nj, n, partial);
-  }
-  hipLaunchKernelGGL(k_reduce_partials, dim3(k), dim3(kThreads), 0, s, partial, nb, 0, out, Publish{});
+  hipLaunchKernelGGL(k_mdot, dim3(krylov_reduction_blocks(n), (k + 7) / 8), dim3(kRed), 0, s, w, V, ldv, k, n, partial);
+  return hipGetLastError();
+}
+
+hipError_t launch_dot_partial(const double *x, const double *y, long long n, int slot, double *partial, hipStream_t s) {
+  if (slot < 0 || slot >= kMaxDots) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_dot, dim3(krylov_reduction_blocks(n)), dim3(kRed), 0, s, x, y, n, slot, partial);
   return hipGetLastError();
 }
 
 hipError_t launch_dot(const double *x, const double *y, long long n, int slot, double *partial, double *out, hipStream_t s, const Publish &pub) {
+  if (slot < 0 || slot >= kMaxDots || pub.count > 64) return hipErrorInvalidValue;
+  const int nb = krylov_reduction_blocks(n);
+  hipLaunchKernelGGL(k_dot, dim3(nb), dim3(kRed), 0, s, x, y, n, slot, partial);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(64), 0, s, partial, nb, slot, out, pub);
+  return hipGetLastError();
+}
+
+hipError_t launch_project_out(double *w, const double *V, long long ldv, int k, long long n, int slot, double *partial, double *out, hipStream_t s) {
+  if (k < 0 || k > kMaxDots || slot < k || slot >= kMaxDots) return hipErrorInvalidValue;
+  const int nb = krylov_reduction_blocks(n);
+  hipLaunchKernelGGL(k_project_out, dim3(nb), dim3(kRed), 0, s, w, V, ldv, k, n, slot, partial, nb, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_normalize(double *y, const double *partial, int slot, double *out, long long n, hipStream_t s, const Publish &pub) {
   if (slot < 0 || slot >= kMaxDots || pub.count > kThreads) return hipErrorInvalidValue;
-  const int nb = krylov_reduction_blocks(n);
-  hipLaunchKernelGGL(k_dot, dim3(nb), dim3(kThreads), 0, s, x, y, n, slot, partial);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kThreads), 0, s, partial, nb, slot, out, pub);
-  return hipGetLastError();
-}
-
-hipError_t launch_project_out(double *w, const double *V, long long ldv, int k, const double *h, long long n, int slot, double *partial, double *out,
-                              hipStream_t s, const Publish &pub) {
-  if (k < 0 || k > kMaxDots || slot < 0 || slot >= kMaxDots || pub.count > kThreads) return hipErrorInvalidValue;
-  const int nb = krylov_reduction_blocks(n);
-  hipLaunchKernelGGL(k_project_out, dim3(nb), dim3(kThreads), 0, s, w, V, ldv, k, h, n, slot, partial);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kThreads), 0, s, partial, nb, slot, out, pub);
-  return hipGetLastError();
-}
-
-hipError_t launch_normalize(double *y, const double *hsq, long long n, hipStream_t s) {
-  hipLaunchKernelGGL(k_normalize, dim3(elementwise_grid(n)), dim3(kThreads), 0, s, y, hsq, n);
+  hipLaunchKernelGGL(k_normalize, dim3(elementwise_grid((n + kNormalize - 1) / kNormalize)), dim3(kThreads), 0, s, y, partial, krylov_reduction_blocks(n), slot, out, n, pub);
   return hipGetLastError();
 }
 
@@ -313,18 +418,18 @@ hipError_t launch_set(double *x, double v, long long n, hipStream_t s) {
 }
 
 hipError_t launch_count_nonfinite(const double *x, long long n, int slot, double *partial, double *out, hipStream_t s, const Publish &pub) {
-  if (slot < 0 || slot >= kMaxDots || pub.count > kThreads) return hipErrorInvalidValue;
+  if (slot < 0 || slot >= kMaxDots || pub.count > 64) return hipErrorInvalidValue;
   const int nb = krylov_reduction_blocks(n);
-  hipLaunchKernelGGL(k_count_nonfinite, dim3(nb), dim3(kThreads), 0, s, x, n, slot, partial);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kThreads), 0, s, partial, nb, slot, out, pub);
+  hipLaunchKernelGGL(k_count_nonfinite, dim3(nb), dim3(kRed), 0, s, x, n, slot, partial);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(64), 0, s, partial, nb, slot, out, pub);
   return hipGetLastError();
 }
 
 hipError_t launch_pb_invert(double *pb, long long nnodes, int slot, double *partial, double *out, hipStream_t s, const Publish &pub) {
-  if (slot < 0 || slot >= kMaxDots || pub.count > kThreads) return hipErrorInvalidValue;
+  if (slot < 0 || slot >= kMaxDots || pub.count > 64) return hipErrorInvalidValue;
   const int nb = krylov_reduction_blocks(nnodes);
   hipLaunchKernelGGL(k_pb_invert, dim3(nb), dim3(kThreads), 0, s, pb, nnodes, slot, partial);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kThreads), 0, s, partial, nb, slot, out, pub);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(64), 0, s, partial, nb, slot, out, pub);
   return hipGetLastError();
 }
 

@@ -4,8 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
-constexpr int kMaxDots            = 32;    // GMRES restart + 1 must not exceed this
-constexpr int kMaxReductionBlocks = 1024;  // partial buffers hold kMaxDots x kMaxReductionBlocks doubles, slot-major
+constexpr int kMaxDots            = 32;   // GMRES restart + 1 must not exceed this
+constexpr int kMaxReductionBlocks = 256;  // one per CU; partial buffers hold kMaxDots x kMaxReductionBlocks doubles, slot-major
 constexpr int kMaxLinComb         = 8;
 
 struct LinComb {  // sum_j c[j] x[j], passed by value
@@ -14,7 +14,7 @@ struct LinComb {  // sum_j c[j] x[j], passed by value
   const double *x[kMaxLinComb];
 };
 
-// Host read of reduction results without a copy: the final (single-block) reduction kernel of a launch stores
+// Host read of reduction results without a copy: the first block of the kernel that forms the last one stores
 // out[0 .. count) into h and then seq into *flag with system-scope release ordering.  h and flag are device addresses
 // of mapped, coherent host memory; h == nullptr publishes nothing.
 struct Publish {
@@ -30,16 +30,17 @@ struct Coefs {  // basis coefficients, passed by value
 };
 
 int krylov_reduction_blocks(long long n);
-// out[j] = <w, V_j>, j < k (V_j = V + j ldv)
-hipError_t launch_mdot(const double *w, const double *V, long long ldv, int k, long long n, double *partial, double *out, hipStream_t s);
+// Partial sums of <w, V_j>, j < k (V_j = V + j ldv), into slots 0 .. k-1
+hipError_t launch_mdot(const double *w, const double *V, long long ldv, int k, long long n, double *partial, hipStream_t s);
+// Partial sums of <x, y> into slot
+hipError_t launch_dot_partial(const double *x, const double *y, long long n, int slot, double *partial, hipStream_t s);
 // out[slot] = <x, y>
 hipError_t launch_dot(const double *x, const double *y, long long n, int slot, double *partial, double *out, hipStream_t s,
                       const Publish &pub = Publish{});
-// w -= sum_{j<k} h[j] V_j (h in device memory), then out[slot] = <w, w>
-hipError_t launch_project_out(double *w, const double *V, long long ldv, int k, const double *h, long long n, int slot, double *partial, double *out,
-                              hipStream_t s, const Publish &pub = Publish{});
-// y /= sqrt(*hsq) unless *hsq == 0 (hsq in device memory)
-hipError_t launch_normalize(double *y, const double *hsq, long long n, hipStream_t s);
+// out[j] = sum of the partials of slot j, j < k; w -= sum_{j<k} out[j] V_j, then partial sums of <w, w> into slot >= k
+hipError_t launch_project_out(double *w, const double *V, long long ldv, int k, long long n, int slot, double *partial, double *out, hipStream_t s);
+// out[slot] = sum of the slot's partials; out[0 .. pub.count) is published; y /= sqrt(out[slot]) unless that is 0
+hipError_t launch_normalize(double *y, const double *partial, int slot, double *out, long long n, hipStream_t s, const Publish &pub);
 // y = a y + sum_j lc.c[j] lc.x[j]  (a == 0 does not read y)
 hipError_t launch_lincomb(double *y, double a, const LinComb &lc, long long n, hipStream_t s);
 // y += sum_{j<cf.k} cf.c[j] V_j
