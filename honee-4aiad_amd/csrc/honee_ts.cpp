@@ -349,20 +349,23 @@ int invert_diagonal(HoneeMiTS ts, double *d, bool block, const char *what) {
   return 0;
 }
 
-int check_finite(HoneeMiTS ts, const double *x, const char *what) {
-  const Publish pub = next_publish(ts, 1);
-  TS_HIP(ts, launch_count_nonfinite(x, ts->n, 0, ts->partial, ts->d_red, ts->s, pub));
+// pub: the count of x that the caller has launched, if it has
+int check_finite(HoneeMiTS ts, const double *x, const char *what, Publish pub = Publish{}) {
+  if (!pub.h) {
+    pub = next_publish(ts, 1);
+    TS_HIP(ts, launch_count_nonfinite(x, ts->n, 0, ts->partial, ts->d_red, ts->s, pub));
+  }
   TS_CALL(wait_published(ts, pub));
   if (ts->h_red[0] != 0) return fail(ts, -3, "%s has %.0f non-finite entries at step %d (t = %g)", what, ts->h_red[0], ts->st.steps, ts->t);
   return 0;
 }
 
 // ---- explicit Runge-Kutta ----
-int mass_solve(HoneeMiTS ts, const double *state, const double *r, double *k) {
+// PCSetUp of the mass KSP at its first solve
+int mass_setup(HoneeMiTS ts, const double *state) {
   HoneeMiProblem p = ts->p;
   const bool block = ts->o.mass_pc == 1;
-  if (!ts->mass_pc_ready) {  // PCSetUp of the mass KSP at its first solve
-    if (block) {
+  if (!ts->mass_pc_ready) {    if (block) {
       TS_OP(ts, HoneeMiMassPointBlockDiagonal(p, kMemDevice, state, ts->mass_dinv));
     } else if (ts->o.mass_jacobi_rowsum) {
       TS_HIP(ts, launch_set(ts->w, 1.0, ts->n, ts->s));
@@ -374,6 +377,13 @@ int mass_solve(HoneeMiTS ts, const double *state, const double *r, double *k) {
     TS_CALL(invert_diagonal(ts, ts->mass_dinv, block, "mass preconditioner"));
     ts->mass_pc_ready = true;
   }
+  return 0;
+}
+
+int mass_solve(HoneeMiTS ts, const double *state, const double *r, double *k) {
+  HoneeMiProblem p = ts->p;
+  const bool block = ts->o.mass_pc == 1;
+  TS_CALL(mass_setup(ts, state));
   const Precond prec{ts, ts->mass_dinv, block};
   if (!ts->o.mass_gmres) return prec(k, r, nullptr);
   auto apply = [&](const double *xin, double *yout) -> int {
@@ -387,28 +397,64 @@ int mass_solve(HoneeMiTS ts, const double *state, const double *r, double *k) {
   return 0;
 }
 
-int rk_step(HoneeMiTS ts) {
-  const Tableau &T = ts->tab;
-  const double   h = ts->o.dt;
+// With a point-diagonal mass and at most kMaxLinComb stages, a stage is its right-hand side and one kernel for the mass solve,
+// the next stage's state or the result, and the result's check (the host waits for *checked); otherwise *checked stays empty.
+// A stage of one mass solve, one copy or combination and, behind the last, a count took SSP33 24 vector passes a step
+// against 17.
+int rk_step(HoneeMiTS ts, Publish *checked) {
+  const Tableau &T     = ts->tab;
+  const double   h     = ts->o.dt;
+  const bool     fused = !ts->o.mass_gmres && ts->o.mass_pc != 1 && T.s <= kMaxLinComb;
   for (int i = 0; i < T.s; i++) {
-    std::vector<double>         c{1.0};
-    std::vector<const double *> xs{ts->q};
-    for (int j = 0; j < i; j++) {
-      c.push_back(h * T.A[(size_t)i * T.s + j]);
-      xs.push_back(ts->K[j]);
+    const double *state = ts->q;
+    if (i > 0) {
+      state = ts->Y;
+      if (!fused) {
+        std::vector<double>         c{1.0};
+        std::vector<const double *> xs{ts->q};
+        for (int j = 0; j < i; j++) {
+          c.push_back(h * T.A[(size_t)i * T.s + j]);
+          xs.push_back(ts->K[j]);
+        }
+        TS_CALL(lincomb(ts, ts->Y, 0.0, c, xs));
+      }
     }
-    TS_CALL(lincomb(ts, ts->Y, 0.0, c, xs));
-    TS_OP(ts, HoneeMiApplyRHS(ts->p, kMemDevice, ts->t + T.c[i] * h, h, ts->Y, ts->R));
+    TS_OP(ts, HoneeMiApplyRHS(ts->p, kMemDevice, ts->t + T.c[i] * h, h, state, ts->R));
     ts->st.rhs_evals++;
-    TS_CALL(mass_solve(ts, ts->Y, ts->R, ts->K[i]));
+    if (!fused) {
+      TS_CALL(mass_solve(ts, state, ts->R, ts->K[i]));
+      continue;
+    }
+    TS_CALL(mass_setup(ts, state));
+    const bool last = i + 1 == T.s;
+    auto       coef = [&](int stage, int j) { return h * (stage == T.s ? T.b[j] : T.A[(size_t)stage * T.s + j]); };
+    RkStage    a{};
+    a.d = ts->mass_dinv, a.r = ts->R, a.q = ts->q, a.y = last ? ts->q : ts->Y;
+    a.ck = coef(i + 1, i);
+    for (int j = 0; j < i; j++) {
+      const double c = coef(i + 1, j);
+      if (c == 0) continue;
+      a.lc.c[a.lc.m]   = c;
+      a.lc.x[a.lc.m++] = ts->K[j];
+    }
+    for (int stage = i + 2; stage <= T.s; stage++)
+      if (coef(stage, i) != 0) a.k = ts->K[i];
+    if (last) {
+      *checked = next_publish(ts, 1);
+      TS_HIP(ts, launch_rk_last(a, ts->n, 0, ts->partial, ts->d_red, ts->s, *checked));
+    } else {
+      TS_HIP(ts, launch_rk_stage(a, ts->n, ts->s));
+    }
   }
-  std::vector<double>         c;
-  std::vector<const double *> xs;
-  for (int i = 0; i < T.s; i++) {
-    c.push_back(h * T.b[i]);
-    xs.push_back(ts->K[i]);
+  if (!fused) {
+    std::vector<double>         c;
+    std::vector<const double *> xs;
+    for (int i = 0; i < T.s; i++) {
+      c.push_back(h * T.b[i]);
+      xs.push_back(ts->K[i]);
+    }
+    TS_CALL(lincomb(ts, ts->q, 1.0, c, xs));
   }
-  TS_CALL(lincomb(ts, ts->q, 1.0, c, xs));
   ts->t += h;
   return 0;
 }
@@ -848,15 +894,16 @@ const double *HoneeMiTSGetSolutionDevice(HoneeMiTS ts) { return ts->q; }
 
 int HoneeMiTSStep(HoneeMiTS ts, int nsteps) {
   for (int i = 0; i < nsteps; i++) {
+    Publish checked;
     switch (ts->o.type) {
-      case HONEE_MI_TS_RK: TS_CALL(rk_step(ts)); break;
+      case HONEE_MI_TS_RK: TS_CALL(rk_step(ts, &checked)); break;
       case HONEE_MI_TS_ALPHA: TS_CALL(alpha_step(ts)); break;
       case HONEE_MI_TS_BEULER: TS_CALL(beuler_step(ts)); break;
       default: TS_CALL(bdf_step(ts));
     }
     ts->st.steps++;
     ts->st.time = ts->t;
-    TS_CALL(check_finite(ts, ts->q, "solution"));
+    TS_CALL(check_finite(ts, ts->q, "solution", checked));
   }
   return 0;
 }

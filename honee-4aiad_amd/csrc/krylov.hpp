@@ -14,6 +14,13 @@ struct LinComb {  // sum_j c[j] x[j], passed by value
   const double *x[kMaxLinComb];
 };
 
+struct RkStage {  // k = d r, y = q + sum_j lc.c[j] lc.x[j] + ck k; y may be q; k null: not stored
+  const double *d, *r, *q;
+  double       *k, *y;
+  double        ck;
+  LinComb       lc;
+};
+
 // Host read of reduction results without a copy: the first block of the kernel that forms the last one stores
 // out[0 .. count) into h and then seq into *flag with system-scope release ordering.  h and flag are device addresses
 // of mapped, coherent host memory; h == nullptr publishes nothing.
@@ -47,6 +54,9 @@ hipError_t launch_lincomb(double *y, double a, const LinComb &lc, long long n, h
 hipError_t launch_basis_comb(double *y, const double *V, long long ldv, const Coefs &cf, long long n, hipStream_t s);
 // z = d (x - y), or z = d x when y is null
 hipError_t launch_dscale_diff(double *z, const double *d, const double *x, const double *y, long long n, hipStream_t s);
+// A Runge-Kutta stage with the mass solve k = d r; the last one also sets out[slot] = number of NaN/Inf entries of y
+hipError_t launch_rk_stage(const RkStage &a, long long n, hipStream_t s);
+hipError_t launch_rk_last(const RkStage &a, long long n, int slot, double *partial, double *out, hipStream_t s, const Publish &pub);
 // d = 1/d with 1 for zero entries
 hipError_t launch_jacobi_invert(double *d, long long n, hipStream_t s);
 hipError_t launch_set(double *x, double v, long long n, hipStream_t s);
