@@ -903,17 +903,19 @@ void gather_tiles(const std::vector<int> &rowptr, std::vector<int> &index, std::
   const int nrows = (int)rowptr.size() - 1, target = (int)std::clamp<size_t>(index.size() / 1024, 64, kGatherSlots);
   tile.assign(1, 0);
   pos.resize(index.size());
-  std::vector<int> order;
+  std::vector<uint64_t> order;  // (slot, place among the tile's rows)
   for (int r0 = 0; r0 < nrows;) {
     int r1 = r0 + 1;
     while (r1 < nrows && rowptr[r1 + 1] - rowptr[r0] <= target) r1++;
     const int j0 = rowptr[r0], m = rowptr[r1] - j0;
     if (m <= kGatherSlots) {
       order.resize(m);
-      for (int i = 0; i < m; i++) order[i] = i;
-      std::sort(order.begin(), order.end(), [&](int x, int y) { return index[j0 + x] < index[j0 + y]; });
-      for (int i = 0; i < m; i++) pos[j0 + order[i]] = (unsigned short)i;
-      std::sort(index.begin() + j0, index.begin() + j0 + m);
+      for (int i = 0; i < m; i++) order[i] = (uint64_t)index[j0 + i] << 16 | (uint64_t)i;
+      std::sort(order.begin(), order.end());
+      for (int i = 0; i < m; i++) {
+        pos[j0 + (order[i] & 0xffff)] = (unsigned short)i;
+        index[j0 + i]                 = (int)(order[i] >> 16);
+      }
     }
     tile.push_back(r1);
     r0 = r1;
@@ -945,6 +947,7 @@ int rstr_transpose_map(CeedElemRestriction r) {
   if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_perm, perm.data(), sizeof(int) * n, hipMemcpyHostToDevice));
   if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_index, index.data(), sizeof(int) * n, hipMemcpyHostToDevice));
   if (!toff.empty()) MI_HIP(r->ceed, hipMemcpy(r->d_t_offset, toff.data(), sizeof(int) * toff.size(), hipMemcpyHostToDevice));
+  if (r->num_comp != 5) return 0;  // the operators with an element-ordered E-vector have 5 components
   std::vector<int>            tile;
   std::vector<unsigned short> pos;
   gather_tiles(rowptr, index, tile, pos);

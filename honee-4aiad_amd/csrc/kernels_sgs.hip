@@ -335,8 +335,8 @@ __global__ void __launch_bounds__(sgs_block_threads<Q>()) k_field(FieldArgs a, c
 // for N components alike, which in the reference directions is the 3 x 3 matrix K = wdetJ alpha dXdx dXdx^T on the reference
 // gradient.  K and the node offsets are formed once per element and serve all components, NC of which go through the stage
 // at a time (11 components at once would leave one block of LDS to a SIMD).
-// Bound by LDS and instruction issue.  Measured at 32^3 p=2, 11 components: 139 us as two operators of 5 and 6 components
-// through k_field, each with its own copy of the point data -> 102 us.
+// Bound by LDS and instruction issue.  Measured at 32^3 p=2, 11 components (now k_filter_lhs_lanes): 139 us as two operators of
+// 5 and 6 components through k_field, each with its own copy of the point data -> 102 us.
 template <int P, int Q, int N>
 __global__ void __launch_bounds__(sgs_block_threads<Q>()) k_filter_lhs(FieldArgs a, const CeedMiDiffFilterContext ctx) {
   using Dm          = Dims<P, Q>;
@@ -422,6 +422,114 @@ __global__ void __launch_bounds__(sgs_block_threads<Q>()) k_filter_lhs(FieldArgs
         }
       }
     }
+  }
+}
+
+// The same operator for small elements, a wave per group of elements and a lane per (element, component): the lane holds its
+// component's values in registers from the nodes to the points and back, and only the point's K and wdetJ (formed once per
+// element, read by all of its lanes alike) come through LDS.  Q = 4 would take 256 registers for the values alone.
+// Bound by latency at 2 waves a SIMD (226 registers; 168 spill).  Measured at 32^3 p=2, 11 components: 71 us (2.4 TB/s of the
+// E-vector, the point data and the field) against 102 us through the line stage, whose passes wait on LDS.
+template <int P, int Q, int N>
+struct FilterLanes {
+  static constexpr bool use = Q <= 3 && N >= 10;  // fewer components leave lanes idle
+  static constexpr int  EPB = 64 / N < 5 ? 64 / N : 5;  // elements of a wave (2.2 KB of K each at Q = 3)
+};
+template <int P, int Q, int N>
+__global__ void __launch_bounds__(64) k_filter_lhs_lanes(FieldArgs a, const CeedMiDiffFilterContext ctx) {
+  constexpr int EPB = FilterLanes<P, Q, N>::EPB, P3 = P * P * P, Q3 = Q * Q * Q;
+  static_assert(P == Q && N <= 64, "registers hold nodes or points");
+  using Table = const __attribute__((address_space(4))) double *;
+  const Table B = (Table)(unsigned long long)a.bt.B, D = (Table)(unsigned long long)a.bt.Dc;
+  __shared__ double sK[EPB * Q3][10];
+  __shared__ int    sOff[EPB * P3], sSlot[EPB * P3];
+  const int         lane = threadIdx.x, le = lane / N, c = lane % N;
+  const long long   nbatch = ((long long)a.nelem + EPB - 1) / EPB;
+  for (long long bt = blockIdx.x; bt < nbatch; bt += gridDim.x) {
+    const int  e0 = (int)(bt * EPB), ne = a.nelem - e0 < EPB ? a.nelem - e0 : EPB;
+    const bool ok = le < ne;
+    for (int i = lane; i < ne * P3; i += 64) {
+      sOff[i]  = a.in_offsets[(long long)e0 * P3 + i];
+      sSlot[i] = a.ev ? a.perm[(long long)e0 * P3 + i] : a.out_offsets[(long long)e0 * P3 + i];
+    }
+    __syncthreads();
+    double u[Q3], r[Q3];
+#pragma unroll
+    for (int n = 0; n < P3; n++) u[n] = ok ? a.u[(long long)sOff[le * P3 + n] + c * a.in_comp_stride] : 0.0;
+#pragma unroll
+    for (int i0 = 0; i0 < EPB * Q3; i0 += 64) {
+      const int i = i0 + lane;
+      if (i < ne * Q3) {
+        const int e = e0 + i / Q3, t = i % Q3;
+        double    qd[10], wdetJ, dXdx[3][3], alpha[3][3], K[3][3];
+#pragma unroll
+        for (int k = 0; k < 10; k++) qd[k] = a.qdata[(long long)e * a.qd.se + k * Q3 + t];
+        nsop::unpack_qdata(qd, true, wdetJ, dXdx);
+        filter_alpha<Q>(a, ctx, e, t, true, alpha);
+        filter_tensor(wdetJ, dXdx, alpha, K);
+        sK[i][0] = wdetJ;
+#pragma unroll
+        for (int k = 0; k < 9; k++) sK[i][1 + k] = K[k / 3][k % 3];
+      }
+    }
+    // x, y and z lines from nodes to points
+    auto line = [&](int at, int stride, bool transpose) {
+      double w[Q];
+#pragma unroll
+      for (int i = 0; i < Q; i++) {
+        w[i] = 0;
+#pragma unroll
+        for (int j = 0; j < Q; j++) w[i] += (transpose ? B[j * Q + i] : B[i * Q + j]) * u[at + j * stride];
+      }
+#pragma unroll
+      for (int i = 0; i < Q; i++) u[at + i * stride] = w[i];
+    };
+#pragma unroll
+    for (int l = 0; l < Q * Q; l++) line(l * Q, 1, false);
+#pragma unroll
+    for (int l = 0; l < Q * Q; l++) line(l % Q + l / Q * Q * Q, Q, false);
+#pragma unroll
+    for (int l = 0; l < Q * Q; l++) line(l, Q * Q, false);
+#pragma unroll
+    for (int t = 0; t < Q3; t++) r[t] = 0;
+    __syncthreads();
+    // the point's gradient along its three lines, times K, onto the lines' points
+#pragma unroll
+    for (int t = 0; t < Q3; t++) {
+      const int     q[3] = {t % Q, t / Q % Q, t / (Q * Q)}, stride[3] = {1, Q, Q * Q};
+      const double *k    = sK[(ok ? le : 0) * Q3 + t];
+      double        g[3];
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        g[d] = 0;
+#pragma unroll
+        for (int j = 0; j < Q; j++) g[d] += D[q[d] * Q + j] * u[t + (j - q[d]) * stride[d]];
+      }
+      r[t] += k[0] * u[t];
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const double f = k[1 + 3 * d] * g[0] + k[2 + 3 * d] * g[1] + k[3 + 3 * d] * g[2];
+#pragma unroll
+        for (int j = 0; j < Q; j++) r[t + (j - q[d]) * stride[d]] += D[q[d] * Q + j] * f;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < Q3; t++) u[t] = r[t];
+#pragma unroll
+    for (int l = 0; l < Q * Q; l++) line(l, Q * Q, true);
+#pragma unroll
+    for (int l = 0; l < Q * Q; l++) line(l % Q + l / Q * Q * Q, Q, true);
+#pragma unroll
+    for (int l = 0; l < Q * Q; l++) line(l * Q, 1, true);
+    if (ok) {
+#pragma unroll
+      for (int n = 0; n < P3; n++) {
+        const int slot = sSlot[le * P3 + n];
+        if (a.ev) a.ev[(long long)slot * N + c] = u[n];
+        else atomicAdd(&a.v[slot + c * a.out_comp_stride], u[n]);
+      }
+    }
+    __syncthreads();  // the next elements' offsets and K go to the same places
   }
 }
 
@@ -667,10 +775,18 @@ hipError_t launch_mass_n_diagonal_pq(const FieldArgs &a, int ncomp, hipStream_t 
 
 template <int P, int Q, int N>
 hipError_t launch_filter_lhs_pq(const FieldArgs &a, const CeedMiDiffFilterContext &ctx, hipStream_t s) {
-  constexpr int EPB  = sgs_elems_per_block<Q>();
-  auto          kern = k_filter_lhs<P, Q, N>;
-  const int     grid = grid_for_batches(kern, sgs_block_threads<Q>(), ((long long)a.nelem + EPB - 1) / EPB);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(sgs_block_threads<Q>()), 0, s, a, ctx);
+  if (a.nelem <= 0) return hipSuccess;
+  if constexpr (FilterLanes<P, Q, N>::use) {
+    constexpr int EPB  = FilterLanes<P, Q, N>::EPB;
+    auto          kern = k_filter_lhs_lanes<P, Q, N>;
+    const int     grid = grid_for_batches(kern, 64, ((long long)a.nelem + EPB - 1) / EPB);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, s, a, ctx);
+  } else {
+    constexpr int EPB  = sgs_elems_per_block<Q>();
+    auto          kern = k_filter_lhs<P, Q, N>;
+    const int     grid = grid_for_batches(kern, sgs_block_threads<Q>(), ((long long)a.nelem + EPB - 1) / EPB);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(sgs_block_threads<Q>()), 0, s, a, ctx);
+  }
   return hipGetLastError();
 }
 
