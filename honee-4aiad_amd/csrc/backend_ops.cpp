@@ -1318,21 +1318,33 @@ int op_plan_apply(CeedOperator op, CeedVector in, CeedVector out, bool overwrite
   }
 }
 
-// The point blocks go through the element-ordered E-vector (25 doubles per element node of workspace) and a per-node
-// gather that adds them to the output in a fixed order: deterministic, and measured 2.4 -> 1.0 ms at 32^3 p=3 against
-// 25 FP64 atomics per element node.  The Jacobi diagonal of the volume operators (5 atomics per element node) adds
-// atomically (measured 0.62 ms atomic, 0.68 ms two-pass).
+// The diagonals of the volume operators go through the element-ordered E-vector and a per-node gather in a fixed order:
+// point blocks (25 doubles per element node of workspace; 2.4 -> 1.0 ms at 32^3 p=3 against 25 FP64 atomics per element node)
+// always, the Jacobi diagonal (5 doubles; 24x16x20 p=3 101 -> 75 + 12 us against 5 atomics per element node) where the scatter
+// does so and allocation is not ruled out; else it adds atomically.
 static int diag_evec_begin(Ceed ceed, OpPlan *p, VolumeArgs &a, bool point_block) {
   a.ev = nullptr;
-  if (!point_block) return 0;
+  if (!point_block && (ceed->scatter != 1 || g_no_alloc)) return 0;
   MI_CALL(rstr_transpose_map(p->r_q));
-  return ceed_workspace(ceed, (size_t)p->nelem * p->r_q->elem_size * 25, &a.ev);
+  return ceed_workspace(ceed, (size_t)p->nelem * p->r_q->elem_size * (point_block ? 25 : 5), &a.ev);
 }
-static int diag_evec_finish(Ceed ceed, OpPlan *p, const VolumeArgs &a) {
+static int diag_evec_finish(Ceed ceed, OpPlan *p, const VolumeArgs &a, bool point_block, bool overwrite) {
   if (!a.ev) return 0;
   const CeedElemRestriction r = p->r_q;
-  MI_HIP(ceed, launch_node_gather_blocks(r->t_nrows, r->d_t_rowptr, r->d_t_index, r->d_t_offset, a.ev, a.v, ceed->stream));
+  if (point_block)
+    MI_HIP(ceed, launch_node_gather_blocks(r->t_nrows, r->d_t_rowptr, r->d_t_index, r->d_t_offset, a.ev, a.v, overwrite, ceed->stream));
+  else MI_HIP(ceed, launch_node_gather_tiles(rstr_gather_tiles(r), r->comp_stride, a.ev, nullptr, a.v, overwrite, ceed->stream));
   return 0;
+}
+// The gather writes every entry: no clear before it
+bool op_diagonal_overwrites(CeedOperator op, CeedVector diag, bool point_block) {
+  if (op->composite || op->ceed->scatter != 1 || g_no_alloc) return false;
+  if (!op->plan && plan_bind(op)) return false;
+  const OpPlan *p = op->plan;
+  if (p->kind != QfKind::IJacobian && p->kind != QfKind::MassNewtonian && p->kind != QfKind::Mass5) return false;
+  if (rstr_transpose_map(p->r_q)) return false;
+  if (!p->r_q->t_covers_all || diag->length != (point_block ? 5 : 1) * p->r_q->l_size) return false;
+  return !point_block || (p->r_q->comp_stride == 1 && p->r_q->t_stride == 5);
 }
 
 // The diagonals of the projection and filter operators (Mass_N, the filter LHS) through the node-sorted E-vector and
@@ -1352,7 +1364,7 @@ static int field_diag_evec_finish(Ceed ceed, OpPlan *p, CeedElemRestriction r, c
 // Point-Jacobi diagonal (MatGetDiagonal_Ceed -> CeedOperatorLinearAssembleDiagonal, src/mat-ceed.c:1603-1630) or, with
 // point_block, the [node][c_out][c_in] point-block diagonal (PCVPBJACOBI's MatInvertVariableBlockDiagonal input,
 // CeedOperatorLinearAssemblePointBlockDiagonal) of an interleaved (comp_stride 1) 5-component operator.
-int op_plan_diagonal(CeedOperator op, CeedVector diag, bool point_block) {
+int op_plan_diagonal(CeedOperator op, CeedVector diag, bool point_block, bool overwrite) {
   if (!op->plan) MI_CALL(plan_bind(op));
   OpPlan *p    = op->plan;
   Ceed    ceed = op->ceed;
@@ -1421,7 +1433,7 @@ int op_plan_diagonal(CeedOperator op, CeedVector diag, bool point_block) {
     MI_CALL(diag_evec_begin(ceed, p, a, point_block));
     if (point_block) MI_HIP(ceed, launch_mass_point_block_diagonal(p->P, p->Q, p->kind == QfKind::MassNewtonian, a, ctx, ceed->stream));
     else MI_HIP(ceed, launch_mass_diagonal(p->P, p->Q, p->kind == QfKind::MassNewtonian, a, ctx, ceed->stream));
-    MI_CALL(diag_evec_finish(ceed, p, a));
+    MI_CALL(diag_evec_finish(ceed, p, a, point_block, overwrite));
     MI_CALL(timing_end(ceed, "mass_diagonal", ev));
     return 0;
   }
@@ -1487,7 +1499,7 @@ int op_plan_diagonal(CeedOperator op, CeedVector diag, bool point_block) {
   MI_CALL(diag_evec_begin(ceed, p, a, point_block));
   if (point_block) MI_HIP(ceed, launch_ijacobian_point_block_diagonal(p->P, p->Q, p->var, ceed->jac_fp32, a, ctx, ceed->stream));
   else MI_HIP(ceed, launch_ijacobian_diagonal(p->P, p->Q, p->var, ceed->jac_fp32, a, ctx, ceed->stream));
-  MI_CALL(diag_evec_finish(ceed, p, a));
+  MI_CALL(diag_evec_finish(ceed, p, a, point_block, overwrite));
   MI_CALL(timing_end(ceed, "ijacobian_diagonal", ev));
   return 0;
 }

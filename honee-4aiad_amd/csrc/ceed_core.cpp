@@ -926,7 +926,7 @@ void gather_tiles(const std::vector<int> &rowptr, std::vector<int> &index, std::
 // ascending list of element-node indices e * elem_size + j that gather from it; t_perm maps an element node to its
 // slot in that node-sorted order.  Built once per restriction on the host.
 int rstr_transpose_map(CeedElemRestriction r) {
-  if (r->d_t_rowptr) return 0;
+  if (r->t_ready) return 0;
   if (r->strided) return MI_ERR(r->ceed, CEED_ERROR_BACKEND, "strided restriction has no transpose map");
   if (g_no_alloc) return MI_ERR(r->ceed, CEED_ERROR_UNSUPPORTED, "allocation-free apply: the scatter's transpose map is not built yet");
   const size_t     n = r->h_offsets.size();
@@ -938,26 +938,26 @@ int rstr_transpose_map(CeedElemRestriction r) {
   r->t_stride     = toff.size() > 1 ? toff[1] : r->num_comp;
   for (size_t k = 0; k < toff.size() && r->t_stride; k++)
     if ((long long)toff[k] != (long long)k * r->t_stride) r->t_stride = 0;
-  const size_t nr = std::max<size_t>(toff.size(), 1);
-  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_rowptr, sizeof(int) * (nr + 1)));
-  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_perm, sizeof(int) * std::max<size_t>(n, 1)));
-  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_offset, sizeof(int) * nr));
-  MI_HIP(r->ceed, hipMemcpy(r->d_t_rowptr, rowptr.data(), sizeof(int) * rowptr.size(), hipMemcpyHostToDevice));
-  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_index, sizeof(int) * std::max<size_t>(n, 1)));
-  if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_perm, perm.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_index, index.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  if (!toff.empty()) MI_HIP(r->ceed, hipMemcpy(r->d_t_offset, toff.data(), sizeof(int) * toff.size(), hipMemcpyHostToDevice));
-  if (r->num_comp != 5) return 0;  // the operators with an element-ordered E-vector have 5 components
-  std::vector<int>            tile;
-  std::vector<unsigned short> pos;
-  gather_tiles(rowptr, index, tile, pos);
-  r->t_ntile = (int)tile.size() - 1;
-  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_tile, sizeof(int) * tile.size()));
-  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_slot, sizeof(int) * std::max<size_t>(n, 1)));
-  MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_pos, sizeof(unsigned short) * std::max<size_t>(n, 1)));
-  MI_HIP(r->ceed, hipMemcpy(r->d_t_tile, tile.data(), sizeof(int) * tile.size(), hipMemcpyHostToDevice));
-  if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_slot, index.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_pos, pos.data(), sizeof(unsigned short) * n, hipMemcpyHostToDevice));
+  auto upload = [&](auto **d, const auto &h) -> int {
+    const size_t bytes = sizeof(**d) * h.size();
+    if (!*d) MI_HIP(r->ceed, hipMalloc((void **)d, std::max(bytes, sizeof(**d))));
+    if (bytes) MI_HIP(r->ceed, hipMemcpy(*d, h.data(), bytes, hipMemcpyHostToDevice));
+    return 0;
+  };
+  MI_CALL(upload(&r->d_t_rowptr, rowptr));
+  MI_CALL(upload(&r->d_t_perm, perm));
+  MI_CALL(upload(&r->d_t_offset, toff));
+  MI_CALL(upload(&r->d_t_index, index));
+  if (r->num_comp == 5) {  // of the operators with an element-ordered E-vector
+    std::vector<int>            tile;
+    std::vector<unsigned short> pos;
+    gather_tiles(rowptr, index, tile, pos);
+    MI_CALL(upload(&r->d_t_tile, tile));
+    MI_CALL(upload(&r->d_t_slot, index));
+    MI_CALL(upload(&r->d_t_pos, pos));
+    r->t_ntile = (int)tile.size() - 1;
+  }
+  r->t_ready = true;
   return 0;
 }
 
@@ -1853,35 +1853,44 @@ extern "C" int CeedMiOperatorApplyNoAlloc(CeedOperator op, CeedVector in, CeedVe
   return ierr;
 }
 
-extern "C" int CeedOperatorLinearAssembleAddDiagonal(CeedOperator op, CeedVector assembled, CeedRequest *request) {
+// Add the diagonals of op's leaves to assembled, the first of them overwriting it where *overwrite is set
+static int add_diagonals(CeedOperator op, CeedVector assembled, bool point_block, bool *overwrite) {
   if (op->composite) {
-    for (CeedOperator s : op->subs) MI_CALL(CeedOperatorLinearAssembleAddDiagonal(s, assembled, request));
+    for (CeedOperator s : op->subs) MI_CALL(add_diagonals(s, assembled, point_block, overwrite));
     return CEED_ERROR_SUCCESS;
   }
-  return op_plan_diagonal(op, assembled, false);
+  MI_CALL(op_plan_diagonal(op, assembled, point_block, *overwrite));
+  *overwrite = false;
+  return CEED_ERROR_SUCCESS;
+}
+static int assemble_diagonals(CeedOperator op, CeedVector assembled, bool point_block) {
+  double      *d;
+  CeedOperator first = op;
+  while (first->composite && !first->subs.empty()) first = first->subs[0];
+  MI_CALL(vec_device_write(assembled, &d, false));
+  bool overwrite = op_diagonal_overwrites(first, assembled, point_block);
+  if (!overwrite) MI_HIP(op->ceed, launch_fill(d, 0.0, assembled->length, op->ceed->stream));
+  return add_diagonals(op, assembled, point_block, &overwrite);
+}
+
+extern "C" int CeedOperatorLinearAssembleAddDiagonal(CeedOperator op, CeedVector assembled, CeedRequest *request) {
+  bool overwrite = false;
+  return add_diagonals(op, assembled, false, &overwrite);
 }
 
 extern "C" int CeedOperatorLinearAssembleAddPointBlockDiagonal(CeedOperator op, CeedVector assembled, CeedRequest *request) {
-  if (op->composite) {
-    for (CeedOperator s : op->subs) MI_CALL(CeedOperatorLinearAssembleAddPointBlockDiagonal(s, assembled, request));
-    return CEED_ERROR_SUCCESS;
-  }
-  return op_plan_diagonal(op, assembled, true);
+  bool overwrite = false;
+  return add_diagonals(op, assembled, true, &overwrite);
 }
 
 extern "C" int CeedOperatorLinearAssembleDiagonal(CeedOperator op, CeedVector assembled, CeedRequest *request) {
-  double *d;
-  MI_CALL(vec_device_write(assembled, &d, false));
-  MI_HIP(op->ceed, launch_fill(d, 0.0, assembled->length, op->ceed->stream));
-  return CeedOperatorLinearAssembleAddDiagonal(op, assembled, request);
+  return assemble_diagonals(op, assembled, false);
 }
 
 extern "C" int CeedOperatorLinearAssemblePointBlockDiagonal(CeedOperator op, CeedVector assembled, CeedRequest *request) {
-  double *d;
-  MI_CALL(vec_device_write(assembled, &d, false));
-  MI_HIP(op->ceed, launch_fill(d, 0.0, assembled->length, op->ceed->stream));
-  return CeedOperatorLinearAssembleAddPointBlockDiagonal(op, assembled, request);
+  return assemble_diagonals(op, assembled, true);
 }
+
 // COO pattern of the point-block diagonal values (MatCeedAssemblePointBlockDiagonalCOO, src/mat-ceed.c:76-141): entry
 // 25 n + 5 c_out + c_in sits at row 5 n + c_out, column 5 n + c_in of the interleaved 5-component L-vector space.  The
 // arrays are allocated with malloc (the caller frees them with free).

@@ -84,6 +84,7 @@ struct CeedElemRestriction_private {
   int                 *d_offsets = nullptr;
   // node-sorted E-vector map of the two-pass scatter: element node i = e * elem_size + j writes its contribution to
   // slot t_perm[i]; the slots of L-vector row k (offset t_offset[k]) are t_rowptr[k]..t_rowptr[k+1]-1, ordered by i
+  bool                 t_ready      = false;
   int                  t_nrows      = 0;
   bool                 t_covers_all = false;  // the rows cover every L-vector entry
   int                  t_stride     = 0;      // row k's offset is k t_stride (0: no such stride)
@@ -241,7 +242,8 @@ int rstr_device_offsets(CeedElemRestriction r, const int **d);
 int basis_device_tables(CeedBasis b);
 int op_plan_apply(CeedOperator op, CeedVector in, CeedVector out, bool overwrite);
 bool op_plan_overwrites(CeedOperator op, CeedVector out);
-int op_plan_diagonal(CeedOperator op, CeedVector diag, bool point_block);
+int  op_plan_diagonal(CeedOperator op, CeedVector diag, bool point_block, bool overwrite);
+bool op_diagonal_overwrites(CeedOperator op, CeedVector diag, bool point_block);  // whether overwrite may be set
 void op_plan_destroy(OpPlan *plan);
 int timing_begin(Ceed ceed, const char *name, hipEvent_t *start);
 int timing_end(Ceed ceed, const char *name, hipEvent_t start);

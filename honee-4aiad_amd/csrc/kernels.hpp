@@ -160,7 +160,7 @@ hipError_t launch_node_gather_tiles(const GatherTiles &g, int comp_stride, const
                                     hipStream_t s);
 // The same for 5 x 5 point blocks: v[25 (t_offset[k] / 5) + i] += sum over the node's slots of ev[t_index[j] * 25 + i]
 hipError_t launch_node_gather_blocks(int nrows, const int *t_rowptr, const int *t_index, const int *t_offset, const double *ev, double *v,
-                                     hipStream_t s);
+                                     bool overwrite, hipStream_t s);
 hipError_t launch_restriction_transpose(const int *offsets, int nelem, int elemsize, int ncomp, int comp_stride, const double *e, double *u, hipStream_t s);
 
 // Conjugate gradients with a Jacobi preconditioner (kernels_vector.hip).  scratch holds two sets of kCgBlocks block partials

@@ -104,7 +104,10 @@ __global__ void __launch_bounds__(elems_per_block<Q>() * Q * Q * Q, 2) k_diagona
       Wd[7][0][t] = M[1][2] + M[2][1], Wd[8][0][t] = M[1][3] + M[3][1], Wd[9][0][t] = M[2][3] + M[3][2];
       double r[1] = {0};
       basis3::ContractPairs<P, Q, 1>{tc}.add(Wd, sBB, sGB, sGG, r);
-      if (ok && t < Dm::P3) atomicAdd(&a.v[off + c * a.comp_stride], r[0]);
+      if (ok && t < Dm::P3) {
+        if (a.ev) a.ev[((long long)e * Dm::P3 + t) * 5 + c] = r[0];
+        else atomicAdd(&a.v[off + c * a.comp_stride], r[0]);
+      }
     }
   }
 }

@@ -189,9 +189,10 @@ __global__ void __launch_bounds__(256) k_node_gather_tiles(GatherTiles g, int cs
 // The point-block form of the element-ordered gather: the E-vector holds a 5 x 5 block [c_out][c_in] per element node
 // (25 consecutive values), the output a block per node at 25 * (offset / 5) (the L-vector offsets of an interleaved
 // 5-component field are 5 * node).  One thread per (node, c_out) row of the block sums its 5 values over the node's
-// contributions in ascending slot order and adds them to the output.
+// contributions in ascending slot order and writes them to the output, or adds them.
 __global__ void __launch_bounds__(256) k_node_gather_blocks(int nrows, const int *__restrict__ rowptr, const int *__restrict__ index,
-                                                            const int *__restrict__ toff, const double *__restrict__ ev, double *__restrict__ v) {
+                                                            const int *__restrict__ toff, const double *__restrict__ ev, double *__restrict__ v,
+                                                            bool overwrite) {
   const long long n = (long long)nrows * 5;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
     const int row = (int)(i / 5), co = (int)(i % 5);
@@ -204,7 +205,7 @@ __global__ void __launch_bounds__(256) k_node_gather_blocks(int nrows, const int
     }
     double *dst = v + (long long)toff[row] * 5 + co * 5;
 #pragma unroll
-    for (int c = 0; c < 5; c++) dst[c] += acc[c];
+    for (int c = 0; c < 5; c++) dst[c] = overwrite ? acc[c] : dst[c] + acc[c];
   }
 }
 
@@ -350,10 +351,10 @@ hipError_t launch_node_gather_tiles(const GatherTiles &g, int comp_stride, const
 }
 
 hipError_t launch_node_gather_blocks(int nrows, const int *t_rowptr, const int *t_index, const int *t_offset, const double *ev, double *v,
-                                     hipStream_t s) {
+                                     bool overwrite, hipStream_t s) {
   const long long n = (long long)nrows * 5;
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_node_gather_blocks, dim3(grid_for(n)), dim3(kBlock), 0, s, nrows, t_rowptr, t_index, t_offset, ev, v);
+  hipLaunchKernelGGL(k_node_gather_blocks, dim3(grid_for(n)), dim3(kBlock), 0, s, nrows, t_rowptr, t_index, t_offset, ev, v, overwrite);
   return hipGetLastError();
 }
 
