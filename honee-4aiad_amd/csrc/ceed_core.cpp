@@ -896,29 +896,28 @@ void group_by_offset(const std::vector<CeedInt> &offsets, std::vector<int> &rowp
   for (size_t i = 0; i < n; i++) index[start[offsets[i]]++] = (int)i;
 }
 
-// Tiles of consecutive rows with at most `target` slots each (a row with more is a tile by itself), the slots of each tile
-// sorted in place and the sorted position of every slot in the rows' order.  Few slots are split into smaller tiles, so that
-// more blocks share the latency.
-void gather_tiles(const std::vector<int> &rowptr, std::vector<int> &index, std::vector<int> &tile, std::vector<unsigned short> &pos) {
-  const int nrows = (int)rowptr.size() - 1, target = (int)std::clamp<size_t>(index.size() / 1024, 64, kGatherSlots);
+// Tiles of consecutive rows with at most `target` slots each (a row with more is a tile by itself): the slots of each tile in
+// ascending order, and the place there of every slot in the rows' order (perm: of element node i in the rows' order).  Few slots
+// are split into smaller tiles, so that more blocks share the latency.
+void gather_tiles(const std::vector<int> &rowptr, const std::vector<int> &perm, std::vector<int> &tile, std::vector<int> &slot,
+                  std::vector<unsigned short> &pos) {
+  const int        nrows = (int)rowptr.size() - 1, target = (int)std::clamp<size_t>(perm.size() / 1024, 64, kGatherSlots);
+  std::vector<int> tile_of(perm.size()), next;  // tile of the rows' slots; the next free place of each tile
   tile.assign(1, 0);
-  pos.resize(index.size());
-  std::vector<uint64_t> order;  // (slot, place among the tile's rows)
   for (int r0 = 0; r0 < nrows;) {
     int r1 = r0 + 1;
     while (r1 < nrows && rowptr[r1 + 1] - rowptr[r0] <= target) r1++;
-    const int j0 = rowptr[r0], m = rowptr[r1] - j0;
-    if (m <= kGatherSlots) {
-      order.resize(m);
-      for (int i = 0; i < m; i++) order[i] = (uint64_t)index[j0 + i] << 16 | (uint64_t)i;
-      std::sort(order.begin(), order.end());
-      for (int i = 0; i < m; i++) {
-        pos[j0 + (order[i] & 0xffff)] = (unsigned short)i;
-        index[j0 + i]                 = (int)(order[i] >> 16);
-      }
-    }
+    std::fill(tile_of.begin() + rowptr[r0], tile_of.begin() + rowptr[r1], (int)next.size());
+    next.push_back(rowptr[r0]);
     tile.push_back(r1);
     r0 = r1;
+  }
+  slot.resize(perm.size());
+  pos.resize(perm.size());
+  for (size_t i = 0; i < perm.size(); i++) {  // ascending: every tile's slots come in order
+    const int t = tile_of[perm[i]], k = next[t]++;
+    slot[k]      = (int)i;
+    pos[perm[i]] = (unsigned short)(k - rowptr[tile[t]]);  // not read in a tile of one row above kGatherSlots
   }
 }
 
@@ -949,11 +948,11 @@ int rstr_transpose_map(CeedElemRestriction r) {
   MI_CALL(upload(&r->d_t_offset, toff));
   MI_CALL(upload(&r->d_t_index, index));
   if (r->num_comp == 5) {  // of the operators with an element-ordered E-vector
-    std::vector<int>            tile;
+    std::vector<int>            tile, slot;
     std::vector<unsigned short> pos;
-    gather_tiles(rowptr, index, tile, pos);
+    gather_tiles(rowptr, perm, tile, slot, pos);
     MI_CALL(upload(&r->d_t_tile, tile));
-    MI_CALL(upload(&r->d_t_slot, index));
+    MI_CALL(upload(&r->d_t_slot, slot));
     MI_CALL(upload(&r->d_t_pos, pos));
     r->t_ntile = (int)tile.size() - 1;
   }
