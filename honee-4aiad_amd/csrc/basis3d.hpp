@@ -550,10 +550,10 @@ struct LineStage {
   __device__ LineStage(const double *B_, const double *Dc_, double (*X_)[NST][kSlot], int tid_)
       : B((Table)(unsigned long long)B_), Dc((Table)(unsigned long long)Dc_), X(&X_[0][0][0]), tid(tid_) {}
 
-  // Point of node t of an element
-  __device__ static int node(int t) {
-    if constexpr (P == Q) return t;
-    return t % P + Q * ((t / P) % P + Q * (t / (P * P)));
+  // Point of node t of an element; 0 for the threads t of an element's points that own no node (P < Q), whose values go unused
+  static constexpr __device__ int node(int t) {
+    if (P == Q) return t;
+    return t < P * P * P ? t % P + Q * ((t / P) % P + Q * (t / (P * P))) : 0;
   }
 
   // The thread's lines among the LA x LB lines at a SA + b SB of NC components of every element: line r of the thread starts

@@ -246,9 +246,11 @@ __global__ void __launch_bounds__(block_threads<Q>(), 2) k_volume(VolumeArgs a, 
         asm volatile("" : "+v"(tt));
         Lines(a.bt.B, a.bt.Dc, sX, tt).template transpose<5, Op::kOutV, Op::kOutG>(0, 5);
         // read back by the thread that writes the next batch's node values there
-        const int at = Lines::node(t);
+        if (nd) {
+          const int at = Lines::node(t);
 #pragma unroll
-        for (int c = 0; c < 5; c++) r[c] = X[c][at];
+          for (int c = 0; c < 5; c++) r[c] = X[c][at];
+        }
       } else {
         int tt = t;
         asm volatile("" : "+v"(tt));
