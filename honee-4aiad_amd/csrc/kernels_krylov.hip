@@ -68,11 +68,25 @@ __device__ __forceinline__ void publish(const Publish &pub, const double *out, i
   if (i == 0) __hip_atomic_store(pub.flag, pub.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// acc[j] += w[i] V[j ldv + i] over the thread's slice, j < NJ: the loads of several entries in flight (a count of vectors that is
+// known only at run time has every product wait for its own load)
+template <int NJ>
+__device__ __forceinline__ void dots(const double *__restrict__ w, const double *__restrict__ V, long long ldv, long long n, long long i0,
+                                     long long stride, double (&acc)[8]) {
+#pragma unroll(NJ <= 2 ? 4 : 2)
+  for (long long i = i0; i < n; i += stride) {
+    const double wi = w[i];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) acc[j] += wi * V[(long long)j * ldv + i];
+  }
+}
+
 // partial[j][block] = sum over this block's slice of w[i] V[j ldv + i], j < k, 8 vectors to a row of blocks (w is read once per
 // row, 1/8 of the bytes, and the rows share the latency).
-// Bound by the basis vectors' bytes (L2 and the memory-side cache hold those of a small problem).  Measured at 553 k entries,
-// 10.5 vectors on average: 12.6 us; with a launch for every 8 vectors, a tree of barriers for every sum and a kernel that adds
-// the partials, 26 us.
+// Bound by the basis vectors' bytes (L2 and the memory-side cache hold those of a small problem).  Measured at 553 k entries: 6.1 us
+// for 7 vectors, 11.2 us for 12; with a launch for every 8 vectors, a tree of barriers for every sum and a kernel that adds the
+// partials, 15.3 and 27.7 us.  At 10.6 M entries 117 and 202 us (5.8 TB/s), with that 166 and 287 us, and 271 and 279 us where the
+// vectors of a row that is not full were counted at run time.
 __global__ void __launch_bounds__(kRed) k_mdot(const double *__restrict__ w, const double *__restrict__ V, long long ldv, int k, long long n,
                                                double *__restrict__ partial) {
   __shared__ double s[8][kRed / 64];
@@ -80,21 +94,15 @@ __global__ void __launch_bounds__(kRed) k_mdot(const double *__restrict__ w, con
   const long long   stride = (long long)gridDim.x * kRed, i0 = (long long)blockIdx.x * kRed + threadIdx.x;
   double            acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   V += (long long)j0 * ldv;
-  if (nj == 8) {
-#pragma unroll 2
-    for (long long i = i0; i < n; i += stride) {
-      const double wi = w[i];
-#pragma unroll
-      for (int j = 0; j < 8; j++) acc[j] += wi * V[(long long)j * ldv + i];
-    }
-  } else {
-#pragma unroll 2
-    for (long long i = i0; i < n; i += stride) {
-      const double wi = w[i];
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        if (j < nj) acc[j] += wi * V[(long long)j * ldv + i];
-    }
+  switch (nj) {
+    case 1: dots<1>(w, V, ldv, n, i0, stride, acc); break;
+    case 2: dots<2>(w, V, ldv, n, i0, stride, acc); break;
+    case 3: dots<3>(w, V, ldv, n, i0, stride, acc); break;
+    case 4: dots<4>(w, V, ldv, n, i0, stride, acc); break;
+    case 5: dots<5>(w, V, ldv, n, i0, stride, acc); break;
+    case 6: dots<6>(w, V, ldv, n, i0, stride, acc); break;
+    case 7: dots<7>(w, V, ldv, n, i0, stride, acc); break;
+    default: dots<8>(w, V, ldv, n, i0, stride, acc);
   }
   const double r = wave_sum8(acc);
   if ((threadIdx.x & 7) == 0) s[(threadIdx.x >> 3) % 8][threadIdx.x >> 6] = r;
