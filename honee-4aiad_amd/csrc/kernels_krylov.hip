@@ -401,11 +401,12 @@ int elementwise_grid(long long n) {
 
 }  // namespace
 
-int krylov_reduction_blocks(long long n) {
-  long long g = (n + kRed - 1) / kRed;
+static int krylov_reduction_blocks(long long n, int threads) {
+  long long g = (n + threads - 1) / threads;
   if (g > kMaxReductionBlocks) g = kMaxReductionBlocks;
   return g < 1 ? 1 : (int)g;
 }
+int krylov_reduction_blocks(long long n) { return krylov_reduction_blocks(n, kRed); }
 
 hipError_t launch_mdot(const double *w, const double *V, long long ldv, int k, long long n, double *partial, hipStream_t s) {
   if (k < 1 || k > kMaxDots) return hipErrorInvalidValue;
@@ -491,7 +492,7 @@ hipError_t launch_count_nonfinite(const double *x, long long n, int slot, double
 
 hipError_t launch_pb_invert(double *pb, long long nnodes, int slot, double *partial, double *out, hipStream_t s, const Publish &pub) {
   if (slot < 0 || slot >= kMaxDots || pub.count > 64) return hipErrorInvalidValue;
-  const int nb = krylov_reduction_blocks(nnodes);
+  const int nb = krylov_reduction_blocks(nnodes, kThreads);  // a node a thread as long as the grid allows it
   hipLaunchKernelGGL(k_pb_invert, dim3(nb), dim3(kThreads), 0, s, pb, nnodes, slot, partial);
   hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(64), 0, s, partial, nb, slot, out, pub);
   return hipGetLastError();

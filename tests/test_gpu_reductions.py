@@ -38,6 +38,7 @@ PROJECT = "_Z18launch_project_outPdPKdxixiS_S_P12ihipStream_t"
 NORMALIZE = "_Z16launch_normalizePdPKdiS_xP12ihipStream_tRK7Publish"
 COUNT = "_Z22launch_count_nonfinitePKdxiPdS1_P12ihipStream_tRK7Publish"
 RK_LAST = "_Z14launch_rk_lastRK7RkStagexiPdS2_P12ihipStream_tRK7Publish"
+PB_INVERT = "_Z16launch_pb_invertPdxiS_S_P12ihipStream_tRK7Publish"
 
 
 class Launcher:
@@ -113,6 +114,23 @@ def test_dot_and_nonfinite_count(n):
             L(RK_LAST, a, n, ct.c_int(1), L.partial, L.out, None, Publish())
             assert L.result(1) == 1, (at, bad)
             assert np.array_equal(res.cpu().numpy(), z + 2 * y, equal_nan=True)
+
+
+@pytest.mark.parametrize("nodes", [1, 255, 257, BLOCKS * 256 - 1, BLOCKS * 256 + 300])
+def test_block_inverse(nodes):
+    _say(f"reductions pb_invert nodes={nodes}")
+    L, rng = Launcher(), np.random.default_rng(nodes)
+    A = rng.uniform(-1, 1, (nodes, 5, 5)) + 6 * np.eye(5)  # diagonally dominant: condition below 20
+    ref = np.linalg.inv(A)
+    dA = L.put(A)
+    L(PB_INVERT, dA, nodes, ct.c_int(0), L.partial, L.out, None, Publish())
+    assert L.result(0) == 0
+    assert np.abs(dA.cpu().numpy() - ref).max() < 100 * EPS * np.abs(ref).max()
+    for at in {0, nodes - 1, min(nodes - 1, BLOCKS * 256)}:
+        B = A.copy()
+        B[at, :, 2] = 0
+        L(PB_INVERT, L.put(B), nodes, ct.c_int(0), L.partial, L.out, None, Publish())
+        assert L.result(0) == 1, at
 
 
 @pytest.mark.parametrize("gmres", [0, 1])
