@@ -66,6 +66,8 @@ typedef struct {
   int    snes_linesearch_type;
 } HoneeMiTSOptions;
 
+// jacobian_applies and mass_applies count the products that a solve used: one that was launched ahead of the convergence test
+// and then not needed is not among them.
 typedef struct {
   int       steps;
   double    time;
