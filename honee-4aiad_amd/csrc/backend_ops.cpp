@@ -813,15 +813,16 @@ static int scatter_prepare(OpPlan *p, Ceed ceed, VolumeArgs &a, bool fp32 = fals
   a.ev32 = nullptr;
   a.perm = nullptr;
   if (ceed->scatter != 1) return 0;
-  MI_CALL(rstr_transpose_map(p->r_q));
+  GatherTiles tiles;
+  if (kSortedEvec) MI_CALL(rstr_sorted_slots(p->r_q, &a.perm));
+  else MI_CALL(rstr_gather_tiles(p->r_q, &tiles));
   double *ws;
   MI_CALL(ceed_workspace(ceed, (size_t)p->nelem * p->r_q->elem_size * 5, &ws));
   if (fp32 && !kSortedEvec) {
     a.ev32 = (float *)ws;
     return 0;
   }
-  a.ev   = ws;
-  a.perm = kSortedEvec ? p->r_q->d_t_perm : nullptr;
+  a.ev = ws;
   return 0;
 }
 
@@ -830,10 +831,13 @@ static int scatter_finish(OpPlan *p, Ceed ceed, const VolumeArgs &a, bool overwr
   CeedElemRestriction r = p->r_q;
   hipEvent_t          ev;
   MI_CALL(timing_begin(ceed, "scatter_node_gather", &ev));
-  if (a.perm)
+  if (a.perm) {
     MI_HIP(ceed, launch_node_gather(r->t_nrows, 5, r->comp_stride, r->d_t_rowptr, r->d_t_offset, a.ev, a.v, overwrite, ceed->stream));
-  else
-    MI_HIP(ceed, launch_node_gather_tiles(rstr_gather_tiles(r), r->comp_stride, a.ev, a.ev32, a.v, overwrite, ceed->stream));
+  } else {
+    GatherTiles tiles;
+    MI_CALL(rstr_gather_tiles(r, &tiles));
+    MI_HIP(ceed, launch_node_gather_tiles(tiles, r->comp_stride, a.ev, a.ev32, a.v, overwrite, ceed->stream));
+  }
   MI_CALL(timing_end(ceed, "scatter_node_gather", ev));
   return 0;
 }
@@ -1062,9 +1066,8 @@ static int sgs_field_apply(CeedOperator op, OpPlan *p, CeedVector in, CeedVector
   a.out_comp_stride = r->comp_stride;
   MI_CALL(vec_device_write(out, &a.v, true));
   if (ceed->scatter == 1) {
-    MI_CALL(rstr_transpose_map(r));
+    MI_CALL(rstr_sorted_slots(r, &a.perm));
     MI_CALL(ceed_workspace(ceed, (size_t)p->nelem * r->elem_size * p->ncomp_out, &a.ev));
-    a.perm = r->d_t_perm;
   }
   MI_CALL(vec_device_read(p->v_qdata, &a.qdata));
   a.qd         = p->qd;
@@ -1325,15 +1328,21 @@ int op_plan_apply(CeedOperator op, CeedVector in, CeedVector out, bool overwrite
 static int diag_evec_begin(Ceed ceed, OpPlan *p, VolumeArgs &a, bool point_block) {
   a.ev = nullptr;
   if (!point_block && (ceed->scatter != 1 || g_no_alloc)) return 0;
-  MI_CALL(rstr_transpose_map(p->r_q));
+  GatherTiles tiles;
+  if (point_block) MI_CALL(rstr_transpose_map(p->r_q));
+  else MI_CALL(rstr_gather_tiles(p->r_q, &tiles));
   return ceed_workspace(ceed, (size_t)p->nelem * p->r_q->elem_size * (point_block ? 25 : 5), &a.ev);
 }
 static int diag_evec_finish(Ceed ceed, OpPlan *p, const VolumeArgs &a, bool point_block, bool overwrite) {
   if (!a.ev) return 0;
   const CeedElemRestriction r = p->r_q;
-  if (point_block)
+  if (point_block) {
     MI_HIP(ceed, launch_node_gather_blocks(r->t_nrows, r->d_t_rowptr, r->d_t_index, r->d_t_offset, a.ev, a.v, overwrite, ceed->stream));
-  else MI_HIP(ceed, launch_node_gather_tiles(rstr_gather_tiles(r), r->comp_stride, a.ev, nullptr, a.v, overwrite, ceed->stream));
+    return 0;
+  }
+  GatherTiles tiles;
+  MI_CALL(rstr_gather_tiles(r, &tiles));
+  MI_HIP(ceed, launch_node_gather_tiles(tiles, r->comp_stride, a.ev, nullptr, a.v, overwrite, ceed->stream));
   return 0;
 }
 // The gather writes every entry: no clear before it
@@ -1351,9 +1360,8 @@ bool op_diagonal_overwrites(CeedOperator op, CeedVector diag, bool point_block) 
 // the fixed-order node gather, as their applies do: the Jacobi preconditioners of those CG solves are then bitwise
 // reproducible, and so are the solves.
 static int field_diag_evec_begin(Ceed ceed, OpPlan *p, CeedElemRestriction r, FieldArgs &a) {
-  MI_CALL(rstr_transpose_map(r));
+  MI_CALL(rstr_sorted_slots(r, &a.perm));
   MI_CALL(ceed_workspace(ceed, (size_t)p->nelem * r->elem_size * p->ncomp_out, &a.ev));
-  a.perm = r->d_t_perm;
   return 0;
 }
 static int field_diag_evec_finish(Ceed ceed, OpPlan *p, CeedElemRestriction r, const FieldArgs &a) {

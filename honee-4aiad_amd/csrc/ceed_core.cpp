@@ -901,80 +901,117 @@ void group_by_offset(const std::vector<CeedInt> &offsets, std::vector<int> &rowp
   for (size_t i = 0; i < n; i++) index[start[offsets[i]]++] = (int)i;
 }
 
-// Tiles of consecutive rows with at most `target` slots each (a row with more is a tile by itself): the slots of each tile in
-// ascending order, and the place there of every slot in the rows' order (perm: of element node i in the rows' order).  Few slots
-// are split into smaller tiles, so that more blocks share the latency.
-void gather_tiles(const std::vector<int> &rowptr, const std::vector<int> &perm, std::vector<int> &tile, std::vector<int> &slot,
-                  std::vector<unsigned short> &pos) {
-  const int        nrows = (int)rowptr.size() - 1, target = (int)std::clamp<size_t>(perm.size() / 1024, 64, kGatherSlots);
-  std::vector<int> tile_of(perm.size()), next;  // tile of the rows' slots; the next free place of each tile
-  tile.assign(1, 0);
-  for (int r0 = 0; r0 < nrows;) {
-    int r1 = r0 + 1;
-    while (r1 < nrows && rowptr[r1 + 1] - rowptr[r0] <= target) r1++;
-    std::fill(tile_of.begin() + rowptr[r0], tile_of.begin() + rowptr[r1], (int)next.size());
-    next.push_back(rowptr[r0]);
-    tile.push_back(r1);
-    r0 = r1;
-  }
-  slot.resize(perm.size());
-  pos.resize(perm.size());
-  for (size_t i = 0; i < perm.size(); i++) {  // ascending: every tile's slots come in order
-    const int t = tile_of[perm[i]], k = next[t]++;
-    slot[k]      = (int)i;
-    pos[perm[i]] = (unsigned short)(k - rowptr[tile[t]]);  // not read in a tile of one row above kGatherSlots
-  }
-}
+// Up to this many element nodes the scatter's tables are laid out on the host and uploaded at once, above by the device.  The
+// device's launches and waits cost as much as a few thousand nodes do on the host: first apply of a residual on 18 elements of
+// degree 1 (144 nodes) 174 us, by the device 250 us, by the host with an upload for every table 193-213 us.
+constexpr size_t kHostLayout = 8192;
 
 // Transpose of the offsets for the two-pass scatter: L-vector offsets in ascending order (rows), each with the
-// ascending list of element-node indices e * elem_size + j that gather from it; t_perm maps an element node to its
-// slot in that node-sorted order.  Built once per restriction on the host.
+// ascending list of element-node indices e * elem_size + j that gather from it.  Built once per restriction on the host.
 int rstr_transpose_map(CeedElemRestriction r) {
   if (r->t_ready) return 0;
   if (r->strided) return MI_ERR(r->ceed, CEED_ERROR_BACKEND, "strided restriction has no transpose map");
   if (g_no_alloc) return MI_ERR(r->ceed, CEED_ERROR_UNSUPPORTED, "allocation-free apply: the scatter's transpose map is not built yet");
   const size_t     n = r->h_offsets.size();
-  std::vector<int> rowptr, perm(n), index, toff;
-  group_by_offset(r->h_offsets, rowptr, index, toff);
-  for (size_t j = 0; j < n; j++) perm[index[j]] = (int)j;
-  r->t_nrows      = (int)toff.size();
-  r->t_covers_all = (CeedSize)r->t_nrows * r->num_comp == r->l_size;
-  r->t_stride     = toff.size() > 1 ? toff[1] : r->num_comp;
-  for (size_t k = 0; k < toff.size() && r->t_stride; k++)
+  std::vector<int> toff;
+  group_by_offset(r->h_offsets, r->h_t_rowptr, r->h_t_index, toff);
+  const size_t nr = toff.size();
+  r->t_nrows      = (int)nr;
+  r->t_covers_all = (CeedSize)nr * r->num_comp == r->l_size;
+  r->t_stride     = nr > 1 ? toff[1] : r->num_comp;
+  for (size_t k = 0; k < nr && r->t_stride; k++)
     if ((long long)toff[k] != (long long)k * r->t_stride) r->t_stride = 0;
-  auto upload = [&](auto **d, const auto &h) -> int {
-    const size_t bytes = sizeof(**d) * h.size();
-    if (!*d) MI_HIP(r->ceed, hipMalloc((void **)d, std::max(bytes, sizeof(**d))));
-    if (bytes) MI_HIP(r->ceed, hipMemcpy(*d, h.data(), bytes, hipMemcpyHostToDevice));
-    return 0;
-  };
-  MI_CALL(upload(&r->d_t_rowptr, rowptr));
-  MI_CALL(upload(&r->d_t_perm, perm));
-  MI_CALL(upload(&r->d_t_offset, toff));
-  MI_CALL(upload(&r->d_t_index, index));
-  if (r->num_comp == 5) {  // of the operators with an element-ordered E-vector
-    std::vector<int>            tile, slot;
-    std::vector<unsigned short> pos;
-    gather_tiles(rowptr, perm, tile, slot, pos);
-    MI_CALL(upload(&r->d_t_tile, tile));
-    MI_CALL(upload(&r->d_t_slot, slot));
-    MI_CALL(upload(&r->d_t_pos, pos));
-    r->t_ntile = (int)tile.size() - 1;
+  if (!r->d_t_rowptr) MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_rowptr, sizeof(int) * (2 * nr + 1 + n)));
+  r->d_t_offset = r->d_t_rowptr + nr + 1;
+  r->d_t_index  = r->d_t_offset + nr;
+  if (n <= kHostLayout) {
+    std::vector<int> all(r->h_t_rowptr);
+    all.insert(all.end(), toff.begin(), toff.end());
+    all.insert(all.end(), r->h_t_index.begin(), r->h_t_index.end());
+    MI_HIP(r->ceed, hipMemcpy(r->d_t_rowptr, all.data(), sizeof(int) * all.size(), hipMemcpyHostToDevice));
+  } else {
+    MI_HIP(r->ceed, hipMemcpy(r->d_t_rowptr, r->h_t_rowptr.data(), sizeof(int) * (nr + 1), hipMemcpyHostToDevice));
+    MI_HIP(r->ceed, hipMemcpy(r->d_t_offset, toff.data(), sizeof(int) * nr, hipMemcpyHostToDevice));
+    MI_HIP(r->ceed, hipMemcpy(r->d_t_index, r->h_t_index.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+    std::vector<int>().swap(r->h_t_index);
   }
   r->t_ready = true;
   return 0;
 }
 
-GatherTiles rstr_gather_tiles(CeedElemRestriction r) {
-  GatherTiles g{};
-  g.ntile    = r->t_ntile;
-  g.stride   = r->t_stride;
-  g.tile_row = r->d_t_tile;
-  g.rowptr   = r->d_t_rowptr;
-  g.slot     = r->d_t_slot;
-  g.toff     = r->d_t_offset;
-  g.pos      = r->d_t_pos;
-  return g;
+// The slots of the element nodes in the node-sorted E-vector, for the operators that write one
+int rstr_sorted_slots(CeedElemRestriction r, const int **perm) {
+  MI_CALL(rstr_transpose_map(r));
+  if (!r->perm_ready) {
+    if (g_no_alloc) return MI_ERR(r->ceed, CEED_ERROR_UNSUPPORTED, "allocation-free apply: the E-vector's order is not built yet");
+    const size_t n = r->h_offsets.size();
+    if (!r->d_t_perm) MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_perm, sizeof(int) * std::max<size_t>(n, 1)));
+    if (n <= kHostLayout) {
+      std::vector<int> all(n);
+      for (size_t j = 0; j < n; j++) all[r->h_t_index[j]] = (int)j;
+      if (n) MI_HIP(r->ceed, hipMemcpy(r->d_t_perm, all.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+    } else {
+      MI_HIP(r->ceed, launch_inverse_permutation(r->d_t_index, (long long)n, r->d_t_perm, r->ceed->stream));
+      MI_HIP(r->ceed, hipStreamSynchronize(r->ceed->stream));  // an operator on another stream may read it next
+    }
+    r->perm_ready = true;
+  }
+  *perm = r->d_t_perm;
+  return 0;
+}
+
+// The tiles of the gather of an element-ordered E-vector, for the operators that have one: consecutive rows with at most `target`
+// slots each (a row with more is a tile by itself).  Few slots are split into smaller tiles, so that more blocks share the
+// latency.  The host places the tiles' boundaries, by a search for each one.
+// Measured with the transpose map, on the first apply of a residual: all on the host with an upload for every table, 64^3 p=2 took
+// 61-70 ms and 40^3 p=4 108-118 ms; now 27-33 and 57-68 ms.
+int rstr_gather_tiles(CeedElemRestriction r, GatherTiles *g) {
+  MI_CALL(rstr_transpose_map(r));
+  if (!r->tiles_ready) {
+    if (g_no_alloc) return MI_ERR(r->ceed, CEED_ERROR_UNSUPPORTED, "allocation-free apply: the gather's tiles are not built yet");
+    const std::vector<int> &rowptr = r->h_t_rowptr, &index = r->h_t_index;
+    const size_t            n      = r->h_offsets.size();
+    const int               target = (int)std::clamp<size_t>(n / 1024, 64, kGatherSlots);
+    std::vector<int>        tile{0};
+    for (int r0 = 0; r0 < r->t_nrows; r0 = tile.back()) {  // every row has a slot: at most target rows
+      const auto first = rowptr.begin() + r0 + 1, last = rowptr.begin() + std::min(r0 + target, r->t_nrows) + 1;
+      const int  fit = (int)(std::upper_bound(first, last, rowptr[r0] + target) - first);
+      tile.push_back(r0 + std::max(fit, 1));
+    }
+    const size_t nt = tile.size();
+    if (!r->d_tiles) MI_HIP(r->ceed, hipMalloc((void **)&r->d_tiles, sizeof(int) * (nt + n + (n + 1) / 2)));
+    GatherTiles t{};
+    t.ntile    = (int)nt - 1;
+    t.stride   = r->t_stride;
+    t.tile_row = r->d_tiles;
+    t.rowptr   = r->d_t_rowptr;
+    t.slot     = r->d_tiles + nt;
+    t.toff     = r->d_t_offset;
+    t.pos      = (const unsigned short *)(t.slot + n);
+    if (n <= kHostLayout) {
+      std::vector<int>            all(tile);
+      std::vector<unsigned short> pos(n);
+      all.insert(all.end(), index.begin(), index.end());
+      all.resize(nt + n + (n + 1) / 2);
+      int *slot = all.data() + nt;
+      for (size_t k = 0; k + 1 < nt; k++) {
+        const int j0 = rowptr[tile[k]], j1 = rowptr[tile[k + 1]];
+        std::sort(slot + j0, slot + j1);
+        for (int j = j0; j < j1; j++) pos[j] = (unsigned short)(std::lower_bound(slot + j0, slot + j1, index[j]) - (slot + j0));
+      }
+      memcpy(slot + n, pos.data(), sizeof(pos[0]) * n);
+      MI_HIP(r->ceed, hipMemcpy(r->d_tiles, all.data(), sizeof(int) * all.size(), hipMemcpyHostToDevice));
+    } else {
+      MI_HIP(r->ceed, hipMemcpy(r->d_tiles, tile.data(), sizeof(int) * nt, hipMemcpyHostToDevice));
+      MI_HIP(r->ceed, launch_layout_tiles(t, r->d_t_index, r->d_tiles + nt, (unsigned short *)(r->d_tiles + nt + n), r->ceed->stream));
+      MI_HIP(r->ceed, hipStreamSynchronize(r->ceed->stream));
+    }
+    r->tiles       = t;
+    r->tiles_ready = true;
+    std::vector<int>().swap(r->h_t_rowptr);
+  }
+  *g = r->tiles;
+  return 0;
 }
 
 // Device workspace of at least len doubles, owned by the Ceed and reused by every operator apply on its stream.
@@ -1080,11 +1117,7 @@ extern "C" int CeedElemRestrictionDestroy(CeedElemRestriction *rstr) {
   if (r->d_offsets) (void)hipFree(r->d_offsets);
   if (r->d_t_rowptr) (void)hipFree(r->d_t_rowptr);
   if (r->d_t_perm) (void)hipFree(r->d_t_perm);
-  if (r->d_t_index) (void)hipFree(r->d_t_index);
-  if (r->d_t_offset) (void)hipFree(r->d_t_offset);
-  if (r->d_t_tile) (void)hipFree(r->d_t_tile);
-  if (r->d_t_slot) (void)hipFree(r->d_t_slot);
-  if (r->d_t_pos) (void)hipFree(r->d_t_pos);
+  if (r->d_tiles) (void)hipFree(r->d_tiles);
   Ceed c = r->ceed;
   delete r;
   CeedDestroy(&c);

@@ -82,18 +82,20 @@ struct CeedElemRestriction_private {
   CeedInt              strides[3] = {0, 0, 0};
   std::vector<CeedInt> h_offsets;
   int                 *d_offsets = nullptr;
-  // node-sorted E-vector map of the two-pass scatter: element node i = e * elem_size + j writes its contribution to
-  // slot t_perm[i]; the slots of L-vector row k (offset t_offset[k]) are t_rowptr[k]..t_rowptr[k+1]-1, ordered by i
+  // maps of the two-pass scatter: L-vector row k (offset t_offset[k]) sums the element nodes i = e * elem_size + j of
+  // t_index[t_rowptr[k]..t_rowptr[k+1]-1], in ascending order; in a node-sorted E-vector the element node i has slot t_perm[i]
   bool                 t_ready      = false;
   int                  t_nrows      = 0;
   bool                 t_covers_all = false;  // the rows cover every L-vector entry
   int                  t_stride     = 0;      // row k's offset is k t_stride (0: no such stride)
-  int                 *d_t_rowptr = nullptr, *d_t_perm = nullptr, *d_t_offset = nullptr;
-  int                 *d_t_index = nullptr;  // element node of each slot (inverse of t_perm)
-  // tiles of rows for the gather of an element-ordered E-vector (GatherTiles)
-  int                  t_ntile = 0;
-  int                 *d_t_tile = nullptr, *d_t_slot = nullptr;
-  unsigned short      *d_t_pos = nullptr;
+  int                 *d_t_rowptr = nullptr, *d_t_offset = nullptr, *d_t_index = nullptr;  // one allocation, at d_t_rowptr
+  std::vector<int>     h_t_rowptr, h_t_index;  // until the tiles are built; of a small restriction
+  bool                 perm_ready = false;
+  int                 *d_t_perm   = nullptr;  // inverse of t_index
+  // tiles of rows for the gather of an element-ordered E-vector, once an operator needs them
+  bool                 tiles_ready = false;
+  GatherTiles          tiles{};
+  int                 *d_tiles = nullptr;  // the tiles' rows, slots and positions
 };
 
 struct CeedBasis_private {
@@ -231,7 +233,8 @@ int  ceed_set_error(Ceed ceed, const char *file, int line, const char *func, int
 
 int vec_device_read(CeedVector v, const double **d);
 int rstr_transpose_map(CeedElemRestriction r);
-GatherTiles rstr_gather_tiles(CeedElemRestriction r);  // of a restriction with its transpose map
+int rstr_sorted_slots(CeedElemRestriction r, const int **perm);
+int rstr_gather_tiles(CeedElemRestriction r, GatherTiles *g);
 // Element-node slots grouped by offset, in increasing offset order, each group listing its slots in increasing order:
 // rows r = 0..toff.size()-1 hold slots index[rowptr[r] .. rowptr[r+1]) of offset toff[r].  O(n + max offset).
 void group_by_offset(const std::vector<CeedInt> &offsets, std::vector<int> &rowptr, std::vector<int> &index, std::vector<int> &toff);

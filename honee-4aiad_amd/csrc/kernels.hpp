@@ -156,6 +156,10 @@ struct GatherTiles {
   const int            *tile_row, *rowptr, *slot, *toff;
   const unsigned short *pos;
 };
+// slot and pos of the tiles from index, the element nodes in row order
+hipError_t launch_layout_tiles(const GatherTiles &g, const int *index, int *slot, unsigned short *pos, hipStream_t s);
+// perm[index[i]] = i, i < n
+hipError_t launch_inverse_permutation(const int *index, long long n, int *perm, hipStream_t s);
 hipError_t launch_node_gather_tiles(const GatherTiles &g, int comp_stride, const double *ev, const float *ev32, double *v, bool overwrite,
                                     hipStream_t s);
 // The same for 5 x 5 point blocks: v[25 (t_offset[k] / 5) + i] += sum over the node's slots of ev[t_index[j] * 25 + i]

@@ -128,6 +128,30 @@ __global__ void __launch_bounds__(256) k_node_gather(int nrows, int ncomp, int c
   }
 }
 
+__global__ void __launch_bounds__(256) k_inverse_permutation(const int *__restrict__ index, long long n, int *__restrict__ perm) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) perm[index[i]] = (int)i;
+}
+
+// Slots of a tile in ascending order and the place there of each, by counting the smaller ones (they differ); a block per tile.
+// Run once per restriction.
+__global__ void __launch_bounds__(256) k_layout_tiles(GatherTiles g, const int *__restrict__ index, int *__restrict__ slot,
+                                                      unsigned short *__restrict__ pos) {
+  __shared__ int s[kGatherSlots];
+  const int      r0 = g.tile_row[blockIdx.x], j0 = g.rowptr[r0], m = g.rowptr[g.tile_row[blockIdx.x + 1]] - j0;
+  if (m > kGatherSlots) {  // one row, ascending as it is; its places are not read
+    for (int j = threadIdx.x; j < m; j += 256) slot[j0 + j] = index[j0 + j];
+    return;
+  }
+  for (int j = threadIdx.x; j < m; j += 256) s[j] = index[j0 + j];
+  __syncthreads();
+  for (int j = threadIdx.x; j < m; j += 256) {
+    int rank = 0;
+    for (int i = 0; i < m; i++) rank += s[i] < s[j] ? 1 : 0;
+    slot[j0 + rank] = s[j];
+    pos[j0 + j]     = (unsigned short)rank;
+  }
+}
+
 // The same sum for the element-ordered E-vector of 5 components, a tile of consecutive rows per block.  The block loads the
 // tile's slots in ascending address order, lanes along the 40 bytes of a slot and on to the next, so that each line is asked
 // for by one or two wave loads; it then sums each (row, component) from LDS over the row's slots in ascending order, as in
@@ -336,6 +360,18 @@ hipError_t launch_node_gather(int nrows, int ncomp, int comp_stride, const int *
   if (n <= 0) return hipSuccess;
   const int grid = grid_for((n + NPT - 1) / NPT);
   hipLaunchKernelGGL((k_node_gather<NPT>), dim3(grid), dim3(kBlock), 0, s, nrows, ncomp, comp_stride, t_rowptr, t_offset, ev, v, overwrite);
+  return hipGetLastError();
+}
+
+hipError_t launch_inverse_permutation(const int *index, long long n, int *perm, hipStream_t s) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_inverse_permutation, dim3(grid_for(n)), dim3(kBlock), 0, s, index, n, perm);
+  return hipGetLastError();
+}
+
+hipError_t launch_layout_tiles(const GatherTiles &g, const int *index, int *slot, unsigned short *pos, hipStream_t s) {
+  if (g.ntile <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_layout_tiles, dim3(g.ntile), dim3(256), 0, s, g, index, slot, pos);
   return hipGetLastError();
 }
 

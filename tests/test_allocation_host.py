@@ -1,0 +1,65 @@
+"""Allocations and uploads of the backend's host code, on a HIP runtime of host memory that counts kernels instead of running them
+(fake_hip.c): what a first apply uploads, and that a failed allocation is an error and leaves the objects usable."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes as ct, sys
+import numpy as np
+from helpers import make_case, product_context
+from pyhonee.driver import NewtonianProblem
+hip = ct.CDLL(None)
+hip.fake_h2d_bytes.restype = hip.fake_dev_bytes.restype = ct.c_longlong
+hip.fake_launches.restype = ct.c_long
+hip.fake_launches.argtypes = [ct.c_char_p]
+hip.fake_fail_malloc.argtypes = hip.fake_fail_host_malloc.argtypes = [ct.c_long]
+def problem(shape=(4, 4, 4), degree=2):
+    case = make_case(shape=shape, degree=degree, periodic=(False, False, False), state_var=1, stabilization=2, seed=7)
+    return case, NewtonianProblem(case["mesh"], case["tab"], product_context(case), 1)
+def uploaded(f):
+    before = hip.fake_h2d_bytes()
+    f()
+    return hip.fake_h2d_bytes() - before
+def refused(f):
+    try:
+        f()
+    except RuntimeError as e:
+        return str(e)
+    raise AssertionError("not refused")
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    lib = tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", str(lib), os.path.join(HERE, "fake_hip.c")], check=True)
+    return str(lib)
+
+
+def _run(fake, body):
+    env = dict(os.environ, LD_PRELOAD=fake, PYTHONPATH=os.pathsep.join(sys.path))
+    r = subprocess.run([sys.executable, "-c", PRELUDE + body], env=env, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stdout[-500:], r.stderr[-2000:])
+
+
+def test_first_apply_uploads_the_map_alone(fake):
+    """The offsets, the rows with their element nodes, a few words a tile and the basis tables; the rest of the gather's tables is
+    laid out by the device.  Operators that do not gather with tiles have none."""
+    _run(fake, """
+case, prob = problem((8, 8, 8))
+n, rows = case["mesh"].offsets.size, case["mesh"].nnodes
+g = np.zeros_like(case["q"])
+apply = lambda: prob.ifunction(case["q"], case["qdot"], g)
+first, again = uploaded(apply), uploaded(apply)
+assert first - again <= 4 * (2 * n + 2 * rows + 1) + 4 * (n // 32) + 1024, (first, again, n, rows)
+assert hip.fake_launches(b"k_layout_tiles") == 1
+prob.setup_diff_filter(grid_based_width=True)
+filt = lambda: prob.diff_filter_lhs(np.zeros((rows, 11)))
+first, again = uploaded(filt), uploaded(filt)
+assert hip.fake_launches(b"k_layout_tiles") == 1
+""")

@@ -42,3 +42,24 @@ def test_rows_of_many_contributions(degree, shape, fp32):
     assert rel_err(g, v_ref)[0] < 1e-12 and rel_err(g, v_ref)[1] < 1e-11, rel_err(g, v_ref)
     tol = 2e-5 if fp32 else 1e-12
     assert rel_err(v, j_ref)[0] < tol, rel_err(v, j_ref)
+
+
+@pytest.mark.parametrize("degree,shape", [(1, (3, 2, 2)), (1, (16, 8, 8)), (1, (41, 5, 5)), (2, (7, 7, 6)), (2, (9, 9, 8)), (3, (9, 7, 5))])
+def test_shuffled_node_numbers(degree, shape):
+    """The tables of the gather as the host lays them out (up to 8192 element nodes, the second case) and as the device does (the
+    third and on), for nodes in no order along the elements; the second apply runs on the tables of the first."""
+    print(f"node gather shuffled degree={degree} shape={shape}", flush=True)
+    sys.stdout.flush()
+    case = make_case(shape=shape, degree=degree, periodic=(False, True, False), seed=5 + degree)
+    number = case["rng"].permutation(case["mesh"].nnodes).astype(np.int32)
+    case["mesh"].offsets = np.ascontiguousarray(number[np.asarray(case["mesh"].offsets)])
+    tab = M.tabulate(degree, 0)
+    om, oc = O.Mesh(case["mesh"], tab), O.newt_from_dict(case["ctx"])
+    v_ref, _ = O.ifunction(om, oc, om.setup_qdata(), case["q"], case["qdot"])
+    prob = NewtonianProblem(case["mesh"], tab, context_from_dict(case["ctx"]), 1)
+    g = [np.full_like(case["q"], 3.0) for _ in range(2)]
+    for x in g:
+        prob.ifunction(case["q"], case["qdot"], x)
+    prob.close()
+    assert rel_err(g[0], v_ref)[0] < 1e-12 and rel_err(g[0], v_ref)[1] < 1e-11, rel_err(g[0], v_ref)
+    assert (g[0] == g[1]).all()
