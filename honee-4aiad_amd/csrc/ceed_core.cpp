@@ -683,11 +683,9 @@ extern "C" int CeedMiJacobiCg(CeedOperator op, CeedVector dinv, CeedVector rhs, 
   const CeedSize n    = rhs->length;
   for (CeedVector v : {dinv, x, r, p, Ap})
     if (v->length != n) return MI_ERR(ceed, CEED_ERROR_DIMENSION, "vector lengths differ");
-  if (!ceed->d_cg) {
-    MI_HIP(ceed, hipMalloc((void **)&ceed->d_cg, sizeof(double) * kCgScratch));
-    MI_HIP(ceed, hipHostMalloc((void **)&ceed->h_cg, sizeof(double) * 2, hipHostMallocMapped | hipHostMallocCoherent));
-    MI_HIP(ceed, hipHostGetDevicePointer((void **)&ceed->g_cg, ceed->h_cg, 0));
-  }
+  if (!ceed->d_cg) MI_HIP(ceed, hipMalloc((void **)&ceed->d_cg, sizeof(double) * kCgScratch));
+  if (!ceed->h_cg) MI_HIP(ceed, hipHostMalloc((void **)&ceed->h_cg, sizeof(double) * 2, hipHostMallocMapped | hipHostMallocCoherent));
+  if (!ceed->g_cg) MI_HIP(ceed, hipHostGetDevicePointer((void **)&ceed->g_cg, ceed->h_cg, 0));
   auto              *h_seq = reinterpret_cast<unsigned long long *>(ceed->h_cg + 1);
   unsigned long long seq   = 0;
   __atomic_store_n(h_seq, 0ull, __ATOMIC_RELEASE);

@@ -42,7 +42,8 @@ def fake(tmp_path_factory):
 
 
 def _run(fake, body):
-    env = dict(os.environ, LD_PRELOAD=fake, PYTHONPATH=os.pathsep.join(sys.path))
+    preload = " ".join(p for p in (fake, os.environ.get("LD_PRELOAD")) if p)
+    env = dict(os.environ, LD_PRELOAD=preload, PYTHONPATH=os.pathsep.join(sys.path))
     r = subprocess.run([sys.executable, "-c", PRELUDE + body], env=env, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, (r.returncode, r.stdout[-500:], r.stderr[-2000:])
 
@@ -62,4 +63,17 @@ prob.setup_diff_filter(grid_based_width=True)
 filt = lambda: prob.diff_filter_lhs(np.zeros((rows, 11)))
 first, again = uploaded(filt), uploaded(filt)
 assert hip.fake_launches(b"k_layout_tiles") == 1
+""")
+
+
+def test_conjugate_gradients_without_host_memory(fake):
+    """The solve allocates device and mapped host memory at its first call; without the latter it is an error, also again."""
+    _run(fake, """
+case, prob = problem()
+prob.setup_diff_filter(grid_based_width=True)
+hip.fake_fail_host_malloc(0)
+assert "OutOfMemory" in refused(lambda: prob.diff_filter_apply(case["q"]))
+hip.fake_fail_host_malloc(0)
+assert "OutOfMemory" in refused(lambda: prob.diff_filter_apply(case["q"]))
+assert "not published" in refused(lambda: prob.diff_filter_apply(case["q"]))  # the kernels do not run here
 """)
