@@ -1026,7 +1026,8 @@ int ceed_workspace(Ceed ceed, size_t len, double **d) {
     if (ceed->d_work) {
       MI_HIP(ceed, hipStreamSynchronize(ceed->stream));
       MI_HIP(ceed, hipFree(ceed->d_work));
-      ceed->d_work = nullptr;
+      ceed->d_work   = nullptr;
+      ceed->work_len = 0;
     }
     MI_HIP(ceed, hipMalloc((void **)&ceed->d_work, sizeof(double) * len));
     ceed->work_len = len;

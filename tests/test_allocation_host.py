@@ -77,3 +77,19 @@ hip.fake_fail_host_malloc(0)
 assert "OutOfMemory" in refused(lambda: prob.diff_filter_apply(case["q"]))
 assert "not published" in refused(lambda: prob.diff_filter_apply(case["q"]))  # the kernels do not run here
 """)
+
+
+def test_workspace_that_could_not_grow(fake):
+    """The E-vector's workspace is freed before a larger one is allocated; without that one, the next smaller apply allocates its own
+    (with none the kernel would add to an output that nothing has cleared)."""
+    _run(fake, """
+case, prob = problem()
+g, pb = np.zeros_like(case["q"]), np.zeros((case["mesh"].nnodes, 5, 5))
+apply = lambda: prob.ifunction(case["q"], case["qdot"], g)
+apply()
+assert hip.fake_launches(b"k_node_gather_tiles") == 1
+hip.fake_fail_malloc(1)  # the point blocks' vector, then the workspace
+assert "OutOfMemory" in refused(lambda: prob.ijacobian_point_block_diagonal(pb, 90.0))
+apply()
+assert hip.fake_launches(b"k_node_gather_tiles") == 2
+""")
