@@ -1232,28 +1232,29 @@ extern "C" int CeedBasisCreateProjection(CeedBasis from, CeedBasis to, CeedBasis
 }
 
 int basis_device_tables(CeedBasis b) {
-  if (b->d_interp_1d) return 0;
+  if (b->tables_ready) return 0;
   if (!b->tensor) return MI_ERR(b->ceed, CEED_ERROR_UNSUPPORTED, "non-tensor bases are not supported by the fused kernels");
   if (b->collo_grad_1d.empty()) return MI_ERR(b->ceed, CEED_ERROR_UNSUPPORTED, "basis needs Q_1d >= P_1d");
   const int P = b->P_1d, Q = b->Q_1d;
-  MI_HIP(b->ceed, hipMalloc((void **)&b->d_interp_1d, sizeof(double) * P * Q));
-  MI_HIP(b->ceed, hipMalloc((void **)&b->d_grad_1d, sizeof(double) * P * Q));
-  MI_HIP(b->ceed, hipMalloc((void **)&b->d_collo, sizeof(double) * Q * Q));
-  MI_HIP(b->ceed, hipMalloc((void **)&b->d_weight_1d, sizeof(double) * Q));
-  MI_HIP(b->ceed, hipMemcpy(b->d_interp_1d, b->interp_1d.data(), sizeof(double) * P * Q, hipMemcpyHostToDevice));
-  MI_HIP(b->ceed, hipMemcpy(b->d_grad_1d, b->grad_1d.data(), sizeof(double) * P * Q, hipMemcpyHostToDevice));
-  MI_HIP(b->ceed, hipMemcpy(b->d_collo, b->collo_grad_1d.data(), sizeof(double) * Q * Q, hipMemcpyHostToDevice));
+  auto upload = [&](double **d, const double *h, size_t len) -> int {
+    if (!*d) MI_HIP(b->ceed, hipMalloc((void **)d, sizeof(double) * len));
+    MI_HIP(b->ceed, hipMemcpy(*d, h, sizeof(double) * len, hipMemcpyHostToDevice));
+    return 0;
+  };
   std::vector<double> w = b->q_weight_1d;
   w.resize(Q, 0.0);
-  MI_HIP(b->ceed, hipMemcpy(b->d_weight_1d, w.data(), sizeof(double) * Q, hipMemcpyHostToDevice));
+  MI_CALL(upload(&b->d_interp_1d, b->interp_1d.data(), P * Q));
+  MI_CALL(upload(&b->d_grad_1d, b->grad_1d.data(), P * Q));
+  MI_CALL(upload(&b->d_collo, b->collo_grad_1d.data(), Q * Q));
+  MI_CALL(upload(&b->d_weight_1d, w.data(), Q));
   std::vector<double> prod(3 * Q * P);
   for (int i = 0; i < Q * P; i++) {
     prod[i]             = b->interp_1d[i] * b->interp_1d[i];
     prod[Q * P + i]     = b->grad_1d[i] * b->interp_1d[i];
     prod[2 * Q * P + i] = b->grad_1d[i] * b->grad_1d[i];
   }
-  MI_HIP(b->ceed, hipMalloc((void **)&b->d_prod, sizeof(double) * 3 * Q * P));
-  MI_HIP(b->ceed, hipMemcpy(b->d_prod, prod.data(), sizeof(double) * 3 * Q * P, hipMemcpyHostToDevice));
+  MI_CALL(upload(&b->d_prod, prod.data(), 3 * Q * P));
+  b->tables_ready = true;
   return 0;
 }
 

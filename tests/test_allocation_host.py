@@ -93,3 +93,26 @@ assert "OutOfMemory" in refused(lambda: prob.ijacobian_point_block_diagonal(pb, 
 apply()
 assert hip.fake_launches(b"k_node_gather_tiles") == 2
 """)
+
+
+def test_first_apply_with_a_failed_allocation(fake):
+    """Whichever allocation of a first apply fails (vectors, basis tables, maps, workspace), in the end all is there that a first apply
+    allocates: later in the same apply, where its preparation is tried again, or in the next one, after an error."""
+    _run(fake, """
+def first_apply(fail):
+    case, prob = problem((3, 2, 2))
+    g, start, errors = np.zeros_like(case["q"]), hip.fake_dev_bytes(), 0
+    hip.fake_fail_malloc(fail)
+    try:
+        prob.ifunction(case["q"], case["qdot"], g)
+    except RuntimeError as e:
+        assert "OutOfMemory" in str(e), e
+        errors = 1
+        prob.ifunction(case["q"], case["qdot"], g)
+    hip.fake_fail_malloc(-1)
+    return hip.fake_dev_bytes() - start, errors
+needed, _ = first_apply(-1)
+sizes, errors = zip(*[first_apply(k) for k in range(20)])
+assert all(size == needed for size in sizes), (needed, sizes)
+assert 0 < sum(errors) < 20, errors
+""")
