@@ -57,10 +57,19 @@ struct HoneeMiMlp_ {
   long long   idx_len = 0;
 };
 
+// A buffer of n values in place of the one at *d; without memory for it there is none
+template <class T>
+static int replace(T **d, size_t n) {
+  if (*d) HIPCHK(hipFree(*d));
+  *d = nullptr;
+  HIPCHK(hipMalloc((void **)d, sizeof(T) * n));
+  return 0;
+}
+
 static int ensure_partials(HoneeMiMlp p, int nblocks) {
   if (nblocks <= p->partial_blocks) return 0;
-  if (p->partial) HIPCHK(hipFree(p->partial));
-  HIPCHK(hipMalloc((void **)&p->partial, sizeof(float) * (size_t)nblocks * (p->np + 1)));
+  p->partial_blocks = 0;
+  if (replace(&p->partial, (size_t)nblocks * (p->np + 1))) return 1;
   p->partial_blocks = nblocks;
   return 0;
 }
@@ -73,10 +82,8 @@ static int stage(HoneeMiMlp p, int n, const float *X, const float *T, int mem_ty
     return 0;
   }
   if (n > p->staged) {
-    if (p->X) HIPCHK(hipFree(p->X));
-    if (p->T) HIPCHK(hipFree(p->T));
-    HIPCHK(hipMalloc((void **)&p->X, sizeof(float) * (size_t)n * p->d.ni));
-    HIPCHK(hipMalloc((void **)&p->T, sizeof(float) * (size_t)n * p->d.no));
+    p->staged = 0;
+    if (replace(&p->X, (size_t)n * p->d.ni) || replace(&p->T, (size_t)n * p->d.no)) return 1;
     p->staged = n;
   }
   HIPCHK(hipMemcpyAsync(p->X, X, sizeof(float) * (size_t)n * p->d.ni, hipMemcpyHostToDevice, p->s));
@@ -181,8 +188,8 @@ int HoneeMiMlpTrain(HoneeMiMlp p, int n, const float *X, const float *T, int mem
   if (n <= 0 || o->batch <= 0 || o->epochs <= 0) return fail("HoneeMiMlpTrain: empty training set or schedule");
   if (stage(p, n, X, T, mem_type, &dX, &dT)) return 1;
   if (n > p->idx_len) {
-    if (p->idx) HIPCHK(hipFree(p->idx));
-    HIPCHK(hipMalloc((void **)&p->idx, sizeof(int) * (size_t)n));
+    p->idx_len = 0;
+    if (replace(&p->idx, n)) return 1;
     p->idx_len = n;
   }
   const int nbatch = (n + o->batch - 1) / o->batch;

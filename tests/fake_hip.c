@@ -50,6 +50,9 @@ int hipMemcpy(void *d, const void *s, size_t n, int kind) {
   return memcpy(d, s, n), OK;
 }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *stream) { return hipMemcpy(d, s, n, kind); }
+int hipMemsetAsync(void *d, int v, size_t n, void *stream) { return memset(d, v, n), OK; }
+int hipStreamCreate(void **s) { return *s = NULL, OK; }
+int hipStreamDestroy(void *s) { return OK; }
 int hipStreamSynchronize(void *s) { return OK; }
 int hipEventCreateWithFlags(void **e, unsigned f) { return *e = NULL, OK; }
 int hipEventDestroy(void *e) { return OK; }

@@ -116,3 +116,29 @@ sizes, errors = zip(*[first_apply(k) for k in range(20)])
 assert all(size == needed for size in sizes), (needed, sizes)
 assert 0 < sum(errors) < 20, errors
 """)
+
+
+def test_training_buffers_that_could_not_grow(fake):
+    """The network's staging, partials and sample order are freed before larger ones are allocated; without those, the smaller batches
+    that ran before get buffers of their own, and nothing is freed twice."""
+    _run(fake, """
+from pyhonee import train as TR
+def arrays(n):
+    return np.ones((n, 6), dtype=np.float32), np.ones((n, 6), dtype=np.float32)
+o, failures = TR.options(batch=64), 0
+for k in range(6):
+    mlp = TR.Mlp(seed=1)
+    small, large = arrays(200), arrays(4000)
+    mlp.train(*small, o), mlp.loss_grad(*small)
+    for f in (lambda a: mlp.loss_grad(*a), lambda a: mlp.train(*a, o)):
+        hip.fake_fail_malloc(k)
+        try:
+            f(large)
+        except RuntimeError:
+            failures += 1
+        hip.fake_fail_malloc(-1)
+        f(small)
+        f(large)
+    mlp.close()
+assert failures > 3, failures
+""")
