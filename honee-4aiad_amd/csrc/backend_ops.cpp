@@ -1321,13 +1321,22 @@ int op_plan_apply(CeedOperator op, CeedVector in, CeedVector out, bool overwrite
   }
 }
 
-// The diagonals of the volume operators go through the element-ordered E-vector and a per-node gather in a fixed order:
-// point blocks (25 doubles per element node of workspace; 2.4 -> 1.0 ms at 32^3 p=3 against 25 FP64 atomics per element node)
-// always, the Jacobi diagonal (5 doubles; 24x16x20 p=3 101 -> 75 + 12 us against 5 atomics per element node) where the scatter
-// does so and allocation is not ruled out; else it adds atomically.
+// The point blocks go through the element-ordered E-vector (25 doubles per element node of workspace) and a per-node gather in a
+// fixed order: 2.4 -> 1.0 ms at 32^3 p=3 against 25 FP64 atomics per element node.  The Jacobi diagonal (5 values) does so, where
+// the scatter does and allocation is not ruled out, if that is faster than its atomics; else it adds atomically.
+// With as many points as nodes the atomics set the time of a large mesh, with more points they are hidden, and the gather is a
+// launch of 2 us.  Measured atomic / two-pass, IJacobian and Mass_5 diagonal, us: 32^3 p=3 386 / 289 and 353 / 182, 12^3 p=3 (101 k
+// element nodes) 26.8 / 24.9 and 22.3 / 18.1, 16^3 p=2 (104 k) 28.4 / 27.3 and 24.7 / 20.4, 24^3 p=1 (106 k) 25.0 / 27.4 and 21.5 /
+// 20.6, 32^3 p=1 (254 k) 50.8 / 49.5 and 43.2 / 33.6, 12^3 p=4 (198 k) 53.8 / 55.5 and 42.6 / 41.6, 16^3 p=4 (480 k) 107 / 106 and
+// 93 / 83, 8^3 p=3 (29 k) 14.9 / 16.2 and 10.8 / 12.5; with a point more per direction 32^3 p=3 704 / 731 and 479 / 512, 48^3 p=2
+// 1024 / 1061 and 790 / 820, 64^3 p=1 1031 / 1066 and 591 / 615.
+static bool diag_two_pass(Ceed ceed, const OpPlan *p) {
+  const long long nodes = (long long)p->nelem * p->r_q->elem_size;
+  return ceed->scatter == 1 && !g_no_alloc && p->P == p->Q && nodes >= (p->P == 3 || p->P == 4 ? 100000 : 200000);
+}
 static int diag_evec_begin(Ceed ceed, OpPlan *p, VolumeArgs &a, bool point_block) {
   a.ev = nullptr;
-  if (!point_block && (ceed->scatter != 1 || g_no_alloc)) return 0;
+  if (!point_block && !diag_two_pass(ceed, p)) return 0;
   GatherTiles tiles;
   if (point_block) MI_CALL(rstr_transpose_map(p->r_q));
   else MI_CALL(rstr_gather_tiles(p->r_q, &tiles));
@@ -1351,6 +1360,7 @@ bool op_diagonal_overwrites(CeedOperator op, CeedVector diag, bool point_block) 
   if (!op->plan && plan_bind(op)) return false;
   const OpPlan *p = op->plan;
   if (p->kind != QfKind::IJacobian && p->kind != QfKind::MassNewtonian && p->kind != QfKind::Mass5) return false;
+  if (!point_block && !diag_two_pass(op->ceed, p)) return false;
   if (rstr_transpose_map(p->r_q)) return false;
   if (!p->r_q->t_covers_all || diag->length != (point_block ? 5 : 1) * p->r_q->l_size) return false;
   return !point_block || (p->r_q->comp_stride == 1 && p->r_q->t_stride == 5);

@@ -1,5 +1,5 @@
-"""Allocations and uploads of the backend's host code, on a HIP runtime of host memory that counts kernels instead of running them
-(fake_hip.c): what a first apply uploads, and that a failed allocation is an error and leaves the objects usable."""
+"""The backend's host code on a HIP runtime of host memory that counts kernels instead of running them (fake_hip.c): what a first
+apply uploads, which route a diagonal takes, and that a failed allocation is an error and leaves the objects usable."""
 import os
 import subprocess
 import sys
@@ -12,15 +12,16 @@ PRELUDE = """
 import ctypes as ct, sys
 import numpy as np
 from helpers import make_case, product_context
+from pyhonee import mesh as M
 from pyhonee.driver import NewtonianProblem
 hip = ct.CDLL(None)
 hip.fake_h2d_bytes.restype = hip.fake_dev_bytes.restype = ct.c_longlong
 hip.fake_launches.restype = ct.c_long
 hip.fake_launches.argtypes = [ct.c_char_p]
 hip.fake_fail_malloc.argtypes = hip.fake_fail_host_malloc.argtypes = [ct.c_long]
-def problem(shape=(4, 4, 4), degree=2):
+def problem(shape=(4, 4, 4), degree=2, q_extra=0, resource="/gpu/hip/mi355x"):
     case = make_case(shape=shape, degree=degree, periodic=(False, False, False), state_var=1, stabilization=2, seed=7)
-    return case, NewtonianProblem(case["mesh"], case["tab"], product_context(case), 1)
+    return case, NewtonianProblem(case["mesh"], M.tabulate(degree, q_extra), product_context(case), 1, resource)
 def uploaded(f):
     before = hip.fake_h2d_bytes()
     f()
@@ -141,4 +142,27 @@ for k in range(6):
         f(large)
     mlp.close()
 assert failures > 3, failures
+""")
+
+
+@pytest.mark.parametrize("shape,degree,q_extra,scatter,gathered", [
+    ((30, 30, 28), 1, 0, "twopass", 1), ((30, 30, 27), 1, 0, "twopass", 0), ((16, 16, 15), 2, 0, "twopass", 1), ((15, 15, 15), 2, 0, "twopass", 0),
+    ((12, 12, 11), 3, 0, "twopass", 1), ((11, 11, 12), 3, 0, "twopass", 0), ((16, 10, 10), 4, 0, "twopass", 1), ((3, 2, 2), 3, 0, "twopass", 0),
+    ((30, 30, 28), 1, 1, "twopass", 0), ((16, 16, 15), 2, 1, "twopass", 0), ((12, 12, 11), 3, 0, "atomic", 0)])
+def test_route_of_the_jacobi_diagonal(fake, shape, degree, q_extra, scatter, gathered):
+    """Through the E-vector, whose gather overwrites the output, where that is faster; else atomically into a cleared vector.  The
+    point blocks have their own gather, which overwrites in the two-pass scatter."""
+    _run(fake, f"""
+case, prob = problem({shape}, {degree}, {q_extra}, "/gpu/hip/mi355x:scatter={scatter}")
+g, pb = np.zeros_like(case["q"]), np.zeros((case["mesh"].nnodes, 5, 5))
+prob.ifunction(case["q"], case["qdot"], g)
+count = lambda name: hip.fake_launches(name)
+before = count(b"k_node_gather_tiles"), count(b"k_fill")
+prob.ijacobian_diagonal(g, 90.0)
+assert count(b"k_node_gather_tiles") - before[0] == {gathered}
+assert count(b"k_fill") - before[1] == 1 - {gathered}
+before = count(b"k_node_gather_blocks"), count(b"k_fill")
+prob.ijacobian_point_block_diagonal(pb, 90.0)
+assert count(b"k_node_gather_blocks") - before[0] == 1
+assert count(b"k_fill") - before[1] == {int(scatter == "atomic")}
 """)
