@@ -40,7 +40,8 @@ __device__ __forceinline__ void with_component(int c, F &&f) {
 // ------------------------------------------------------------------------------------------------------------------
 // Diagonal of a linear operator whose quadrature-point action is Op::action (IJacobian)
 // ------------------------------------------------------------------------------------------------------------------
-template <int P, int Q, class Op, typename T>
+// EV: into the element-ordered E-vector, else added atomically (two kernels: a choice at run time cost the atomic one 2 %)
+template <int P, int Q, class Op, typename T, bool EV>
 __global__ void __launch_bounds__(elems_per_block<Q>() * Q * Q * Q, 2) k_diagonal(VolumeArgs a, const CeedMiNewtonianContext ctx) {
   using Dm          = Dims<P, Q>;
   constexpr int EPB = elems_per_block<Q>();
@@ -105,7 +106,7 @@ __global__ void __launch_bounds__(elems_per_block<Q>() * Q * Q * Q, 2) k_diagona
       double r[1] = {0};
       basis3::ContractPairs<P, Q, 1>{tc}.add(Wd, sBB, sGB, sGG, r);
       if (ok && t < Dm::P3) {
-        if (a.ev) a.ev[((long long)e * Dm::P3 + t) * 5 + c] = r[0];
+        if constexpr (EV) a.ev[((long long)e * Dm::P3 + t) * 5 + c] = r[0];
         else atomicAdd(&a.v[off + c * a.comp_stride], r[0]);
       }
     }
@@ -317,7 +318,11 @@ template <int P, int Q, class Op, typename T>
 hipError_t launch_diag(const VolumeArgs &a, const CeedMiNewtonianContext &ctx, hipStream_t stream) {
   constexpr int EPB   = elems_per_block<Q>();
   const int     block = EPB * Q * Q * Q;
-  auto          k     = k_diagonal<P, Q, Op, T>;
+  auto          k     = k_diagonal<P, Q, Op, T, false>;
+  if (a.ev) {
+    if constexpr (P == Q) k = k_diagonal<P, Q, Op, T, true>;
+    else return hipErrorInvalidValue;  // diag_two_pass: the E-vector is for P = Q
+  }
   const int     grid  = grid_for(k, block, ((long long)a.nelem + EPB - 1) / EPB);
   hipLaunchKernelGGL(k, dim3(grid), dim3(block), 0, stream, a, ctx);
   return hipGetLastError();
