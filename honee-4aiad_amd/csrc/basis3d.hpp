@@ -550,10 +550,12 @@ struct LineStage {
   __device__ LineStage(const double *B_, const double *Dc_, double (*X_)[NST][kSlot], int tid_)
       : B((Table)(unsigned long long)B_), Dc((Table)(unsigned long long)Dc_), X(&X_[0][0][0]), tid(tid_) {}
 
-  // Point of node t of an element; 0 for the threads t of an element's points that own no node (P < Q), whose values go unused
+  // Point of node t of an element; for the threads t of an element's points that own no node (P < Q) a point where no node sits:
+  // what they read there goes unused
   static constexpr __device__ int node(int t) {
     if (P == Q) return t;
-    return t < P * P * P ? t % P + Q * ((t / P) % P + Q * (t / (P * P))) : 0;
+    const int at = t % P + Q * ((t / P) % P + Q * (t / (P * P)));
+    return at < Q3 ? at : Q3 - 1;
   }
 
   // The thread's lines among the LA x LB lines at a SA + b SB of NC components of every element: line r of the thread starts

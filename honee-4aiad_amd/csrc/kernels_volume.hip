@@ -245,12 +245,13 @@ __global__ void __launch_bounds__(block_threads<Q>(), 2) k_volume(VolumeArgs a, 
         int tt = threadIdx.x;
         asm volatile("" : "+v"(tt));
         Lines(a.bt.B, a.bt.Dc, sX, tt).template transpose<5, Op::kOutV, Op::kOutG>(0, 5);
-        // read back by the thread that writes the next batch's node values there
-        if (nd) {
-          const int at = Lines::node(t);
+        // read back by the thread that writes the next batch's node values there; by all threads alike (a condition costs 10
+        // registers, and the p=2 explicit residual its third wave: 64^3 330 -> 382 us)
+        int tr = t;
+        if constexpr (P < Q) asm volatile("" : "+v"(tr));  // not another address that stays live
+        const int at = Lines::node(tr);
 #pragma unroll
-          for (int c = 0; c < 5; c++) r[c] = X[c][at];
-        }
+        for (int c = 0; c < 5; c++) r[c] = X[c][at];
       } else {
         int tt = t;
         asm volatile("" : "+v"(tt));

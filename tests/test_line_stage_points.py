@@ -1,5 +1,6 @@
 """Places of an element's nodes in the line stage's LDS slots, checked at compile time for every (P, Q) pair: every thread of an
-element's points gets a place inside a slot, also where the element has fewer nodes than points, and the nodes' places differ."""
+element's points gets a place inside a slot, also where the element has fewer nodes than points; the nodes' places differ, and the
+other threads' is none of them."""
 import os
 import subprocess
 
@@ -15,11 +16,8 @@ constexpr bool places() {
   bool taken[L::Q3] = {};
   for (int t = 0; t < L::Q3; t++) {
     const int at = L::node(t);
-    if (at < 0 || at >= L::Q3) return false;
-    if (t < P * P * P) {
-      if (taken[at]) return false;
-      taken[at] = true;
-    }
+    if (at < 0 || at >= L::Q3 || taken[at]) return false;
+    if (t < P * P * P) taken[at] = true;
   }
   return true;
 }
