@@ -902,6 +902,8 @@ void group_by_offset(const std::vector<CeedInt> &offsets, std::vector<int> &rowp
 // Up to this many element nodes the scatter's tables are laid out on the host and uploaded at once, above by the device.  The
 // device's launches and waits cost as much as a few thousand nodes do on the host: first apply of a residual on 18 elements of
 // degree 1 (144 nodes) 174 us, by the device 250 us, by the host with an upload for every table 193-213 us.
+// Above, each large table has an allocation of its own: beyond 2 MB an allocation takes 0.3 ms instead of a few us (first closure
+// residual at 24^3 p=2 3.6 ms, 4.0-4.2 ms with the tables in two allocations).
 constexpr size_t kHostLayout = 8192;
 
 // Transpose of the offsets for the two-pass scatter: L-vector offsets in ascending order (rows), each with the
@@ -919,10 +921,12 @@ int rstr_transpose_map(CeedElemRestriction r) {
   r->t_stride     = nr > 1 ? toff[1] : r->num_comp;
   for (size_t k = 0; k < nr && r->t_stride; k++)
     if ((long long)toff[k] != (long long)k * r->t_stride) r->t_stride = 0;
-  if (!r->d_t_rowptr) MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_rowptr, sizeof(int) * (2 * nr + 1 + n)));
+  const bool   small = n <= kHostLayout;
+  if (!r->d_t_rowptr) MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_rowptr, sizeof(int) * (2 * nr + 1 + (small ? n : 0))));
+  if (!small && !r->d_t_large) MI_HIP(r->ceed, hipMalloc((void **)&r->d_t_large, sizeof(int) * n));
   r->d_t_offset = r->d_t_rowptr + nr + 1;
-  r->d_t_index  = r->d_t_offset + nr;
-  if (n <= kHostLayout) {
+  r->d_t_index  = small ? r->d_t_offset + nr : r->d_t_large;
+  if (small) {
     std::vector<int> all(r->h_t_rowptr);
     all.insert(all.end(), toff.begin(), toff.end());
     all.insert(all.end(), r->h_t_index.begin(), r->h_t_index.end());
@@ -977,7 +981,9 @@ int rstr_gather_tiles(CeedElemRestriction r, GatherTiles *g) {
       tile.push_back(r0 + std::max(fit, 1));
     }
     const size_t nt = tile.size();
-    if (!r->d_tiles) MI_HIP(r->ceed, hipMalloc((void **)&r->d_tiles, sizeof(int) * (nt + n + (n + 1) / 2)));
+    const bool   small = n <= kHostLayout;
+    if (!r->d_tiles) MI_HIP(r->ceed, hipMalloc((void **)&r->d_tiles, sizeof(int) * (nt + n + (small ? (n + 1) / 2 : 0))));
+    if (!small && !r->d_tile_pos) MI_HIP(r->ceed, hipMalloc((void **)&r->d_tile_pos, sizeof(unsigned short) * n));
     GatherTiles t{};
     t.ntile    = (int)nt - 1;
     t.stride   = r->t_stride;
@@ -985,8 +991,8 @@ int rstr_gather_tiles(CeedElemRestriction r, GatherTiles *g) {
     t.rowptr   = r->d_t_rowptr;
     t.slot     = r->d_tiles + nt;
     t.toff     = r->d_t_offset;
-    t.pos      = (const unsigned short *)(t.slot + n);
-    if (n <= kHostLayout) {
+    t.pos      = small ? (const unsigned short *)(t.slot + n) : r->d_tile_pos;
+    if (small) {
       std::vector<int>            all(tile);
       std::vector<unsigned short> pos(n);
       all.insert(all.end(), index.begin(), index.end());
@@ -1001,7 +1007,7 @@ int rstr_gather_tiles(CeedElemRestriction r, GatherTiles *g) {
       MI_HIP(r->ceed, hipMemcpy(r->d_tiles, all.data(), sizeof(int) * all.size(), hipMemcpyHostToDevice));
     } else {
       MI_HIP(r->ceed, hipMemcpy(r->d_tiles, tile.data(), sizeof(int) * nt, hipMemcpyHostToDevice));
-      MI_HIP(r->ceed, launch_layout_tiles(t, r->d_t_index, r->d_tiles + nt, (unsigned short *)(r->d_tiles + nt + n), r->ceed->stream));
+      MI_HIP(r->ceed, launch_layout_tiles(t, r->d_t_index, r->d_tiles + nt, r->d_tile_pos, r->ceed->stream));
       MI_HIP(r->ceed, hipStreamSynchronize(r->ceed->stream));
     }
     r->tiles       = t;
@@ -1115,8 +1121,10 @@ extern "C" int CeedElemRestrictionDestroy(CeedElemRestriction *rstr) {
   }
   if (r->d_offsets) (void)hipFree(r->d_offsets);
   if (r->d_t_rowptr) (void)hipFree(r->d_t_rowptr);
+  if (r->d_t_large) (void)hipFree(r->d_t_large);
   if (r->d_t_perm) (void)hipFree(r->d_t_perm);
   if (r->d_tiles) (void)hipFree(r->d_tiles);
+  if (r->d_tile_pos) (void)hipFree(r->d_tile_pos);
   Ceed c = r->ceed;
   delete r;
   CeedDestroy(&c);

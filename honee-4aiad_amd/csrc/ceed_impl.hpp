@@ -88,14 +88,16 @@ struct CeedElemRestriction_private {
   int                  t_nrows      = 0;
   bool                 t_covers_all = false;  // the rows cover every L-vector entry
   int                  t_stride     = 0;      // row k's offset is k t_stride (0: no such stride)
-  int                 *d_t_rowptr = nullptr, *d_t_offset = nullptr, *d_t_index = nullptr;  // one allocation, at d_t_rowptr
+  int                 *d_t_rowptr = nullptr, *d_t_offset = nullptr, *d_t_index = nullptr;  // one allocation, at d_t_rowptr, but
+  int                 *d_t_large = nullptr;                                                // for a large index
   std::vector<int>     h_t_rowptr, h_t_index;  // until the tiles are built; of a small restriction
   bool                 perm_ready = false;
   int                 *d_t_perm   = nullptr;  // inverse of t_index
   // tiles of rows for the gather of an element-ordered E-vector, once an operator needs them
   bool                 tiles_ready = false;
   GatherTiles          tiles{};
-  int                 *d_tiles = nullptr;  // the tiles' rows, slots and positions
+  int                 *d_tiles    = nullptr;  // the tiles' rows and slots, and of a small restriction the positions
+  unsigned short      *d_tile_pos = nullptr;
 };
 
 struct CeedBasis_private {
