@@ -594,15 +594,6 @@ static int VelocityGradientProjectionSetup(HoneeMiProblem p) {
   return 0;
 }
 
-// KSPCG with PCJACOBI (inverse diagonal dinv) and KSP_NORM_NATURAL from a zero initial guess: converged when
-// sqrt(r.z) <= max(rtol sqrt(r0.z0), atol), at most max_it iterations (KSPSolve_CG recurrences).  work holds three
-// vectors of the system size.
-static int CgJacobi(HoneeMiProblem p, CeedOperator op, CeedVector dinv, CeedVector R, CeedVector X, CeedVector work[3], double rtol, double atol,
-                    int max_it, int *iterations) {
-  CHK(p, CeedMiJacobiCg(op, dinv, R, X, work[0], work[1], work[2], rtol, atol, max_it, iterations));
-  return 0;
-}
-
 // GridAnisotropyTensorProjectionSetupApply (src/grid_anisotropy_tensor.c:14-111): R = AnisotropyTensorProjection,
 // KSPCG with PCJACOBI (diagonal of Mass_7), natural norm, rtol 1e-10, zero initial guess.
 static int GridAnisotropyTensorProjection(HoneeMiProblem p) {
@@ -624,7 +615,7 @@ static int GridAnisotropyTensorProjection(HoneeMiProblem p) {
   CHK(p, CeedOperatorApply(op_rhs, CEED_VECTOR_NONE, R, CEED_REQUEST_IMMEDIATE));
   CHK(p, CeedOperatorLinearAssembleDiagonal(op_mass, dinv, CEED_REQUEST_IMMEDIATE));
   CHK(p, JacobiInverse(p, dinv));
-  CHK(p, CgJacobi(p, op_mass, dinv, R, p->grid_aniso, work, 1e-10, 1e-50, 10000, &p->grid_aniso_its));
+  CHK(p, CeedMiJacobiCg(op_mass, dinv, R, p->grid_aniso, work[0], work[1], work[2], 1e-10, 1e-50, 10000, &p->grid_aniso_its));
   for (int i = 0; i < 5; i++) CHK(p, CeedVectorDestroy(vs[i]));
   CHK(p, CeedOperatorDestroy(&op_rhs));
   CHK(p, CeedOperatorDestroy(&op_mass));
@@ -867,8 +858,9 @@ static int DiffFilterApply(HoneeMiProblem p) {
     CHK(p, JacobiInverse(p, p->filter_dinv));
     p->filter_pc_ready = 1;
   }
-  return CgJacobi(p, p->op_filter_lhs, p->filter_dinv, p->filter_rhs, p->filtered, p->cg_work, p->filter_rtol, p->filter_atol, p->filter_max_it,
-                  &p->filter_its);
+  CHK(p, CeedMiJacobiCg(p->op_filter_lhs, p->filter_dinv, p->filter_rhs, p->filtered, p->cg_work[0], p->cg_work[1], p->cg_work[2], p->filter_rtol,
+                        p->filter_atol, p->filter_max_it, &p->filter_its));
+  return 0;
 }
 
 int HoneeMiSetFilterWidthScaling(HoneeMiProblem p, const double scaling[3]) {

@@ -371,7 +371,8 @@ int check_finite(HoneeMiTS ts, const double *x, const char *what, Publish pub = 
 int mass_setup(HoneeMiTS ts, const double *state) {
   HoneeMiProblem p = ts->p;
   const bool block = ts->o.mass_pc == 1;
-  if (!ts->mass_pc_ready) {    if (block) {
+  if (!ts->mass_pc_ready) {
+    if (block) {
       TS_OP(ts, HoneeMiMassPointBlockDiagonal(p, kMemDevice, state, ts->mass_dinv));
     } else if (ts->o.mass_jacobi_rowsum) {
       TS_HIP(ts, launch_set(ts->w, 1.0, ts->n, ts->s));

@@ -84,7 +84,7 @@ __device__ __forceinline__ void dots(const double *__restrict__ w, const double 
 // partial[j][block] = sum over this block's slice of w[i] V[j ldv + i], j < k, 8 vectors to a row of blocks (w is read once per
 // row, 1/8 of the bytes, and the rows share the latency).
 // Bound by the basis vectors' bytes (L2 and the memory-side cache hold those of a small problem).  Measured at 553 k entries: 6.1 us
-// for 7 vectors, 11.2 us for 12; with a launch for every 8 vectors, a tree of barriers for every sum and a kernel that adds the
+// for 7 vectors, 11.2 us for 12 (in a GMRES solve with 10.5 on average 10.5 us); with a launch for every 8 vectors, a tree of barriers for every sum and a kernel that adds the
 // partials, 15.3 and 27.7 us.  At 10.6 M entries 117 and 202 us (5.8 TB/s), with that 166 and 287 us, and 271 and 279 us where the
 // vectors of a row that is not full were counted at run time.
 __global__ void __launch_bounds__(kRed) k_mdot(const double *__restrict__ w, const double *__restrict__ V, long long ldv, int k, long long n,
@@ -157,9 +157,10 @@ __device__ __forceinline__ void basis_sum(double (&acc)[U], const double *c, con
 
 // out[j] = sum of partial[j][0 .. nb), j < k; w[i] -= sum_{j < k} out[j] V[j ldv + i] (in order j = 0, 1, ...);
 // partial[slot][block] = sum of the new w[i]^2.  slot >= k: a block may overwrite no partials that another one still reads.
-// Bound as k_mdot; measured there 12.3 us and 6.0 us for k_normalize, 11.4 + 3.6 us with a kernel of 4.1 us between them.
+// Bound as k_mdot; measured in that solve 12.4 us and 5.9 us for k_normalize, 11.4 + 3.6 us with a kernel of 4.1 us between them.  A
+// whole step (three launches against five) at 4.4 M entries, 7 vectors: 120 -> 95 us, 20 vectors: 350 -> 287 us.
 __global__ void __launch_bounds__(kRed) k_project_out(double *__restrict__ w, const double *__restrict__ V, long long ldv, int k, long long n,
-                                                          int slot, double *__restrict__ partial, int nb, double *__restrict__ out) {
+                                                      int slot, double *__restrict__ partial, int nb, double *__restrict__ out) {
   __shared__ double s[kRed / 64];
   __shared__ double c[kMaxDots];
   for (int j = threadIdx.x >> 6; j < k; j += kRed / 64) {
@@ -437,7 +438,8 @@ hipError_t launch_project_out(double *w, const double *V, long long ldv, int k, 
 
 hipError_t launch_normalize(double *y, const double *partial, int slot, double *out, long long n, hipStream_t s, const Publish &pub) {
   if (slot < 0 || slot >= kMaxDots || pub.count > kThreads) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_normalize, dim3(elementwise_grid((n + kNormalize - 1) / kNormalize)), dim3(kThreads), 0, s, y, partial, krylov_reduction_blocks(n), slot, out, n, pub);
+  const int grid = elementwise_grid((n + kNormalize - 1) / kNormalize);
+  hipLaunchKernelGGL(k_normalize, dim3(grid), dim3(kThreads), 0, s, y, partial, krylov_reduction_blocks(n), slot, out, n, pub);
   return hipGetLastError();
 }
 

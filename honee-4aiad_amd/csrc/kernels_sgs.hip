@@ -30,8 +30,9 @@ template <int Q>
 constexpr int sgs_elems_per_block() {
   return (Q * Q * Q >= 64) ? 1 : 64 / (Q * Q * Q);
 }
-// Most components of a k_filter_lhs chunk (11: 6 + 5).  With 4 + 4 + 3 the deconvolution pairs at 32^3 p=2 took 15.5 ms
-// against 14.6: more barriers and passes over the tensor outweigh the LDS saved.
+// Most components of a k_filter_lhs chunk (11: 6 + 5), at Q = 4 and 5; smaller elements have k_filter_lhs_lanes.  Measured apply of 11
+// components, us, with at most 4 / 6 / 11: 24^3 p=3 127 / 119 / 110, 4^3 p=3 10.9 / 10.9 / 10.6, 16^3 p=4 78 / 94 / 94, 4^3 p=4 15.7 /
+// 18.8 / 15.8: no one value is best; as two operators of 5 and 6 components through k_field they took 154, 21.5, 134 and 24.7.
 constexpr int kFilterChunk = 6;
 
 // Threads of a k_field block: its elements' points in whole waves
@@ -335,8 +336,9 @@ __global__ void __launch_bounds__(sgs_block_threads<Q>()) k_field(FieldArgs a, c
 // for N components alike, which in the reference directions is the 3 x 3 matrix K = wdetJ alpha dXdx dXdx^T on the reference
 // gradient.  K and the node offsets are formed once per element and serve all components, NC of which go through the stage
 // at a time (11 components at once would leave one block of LDS to a SIMD).
-// Bound by LDS and instruction issue.  Measured at 32^3 p=2, 11 components (now k_filter_lhs_lanes): 139 us as two operators of
-// 5 and 6 components through k_field, each with its own copy of the point data -> 102 us.
+// Bound by LDS and instruction issue.  Measured as a composite of 5 and 6 components, one output per thread in k_field before, with
+// the gathers: 32^3 p=2 167 -> 133 us, 24^3 p=3 154 -> 144, 16^3 p=4 134 -> 116.  Few lines leave threads idle in small problems: 4^3 p=4
+// 24.7 -> 26.6, and one component alone 16^3 p=4 44.0 -> 46.4, 24^3 p=3 56.6 -> 58.8.
 template <int P, int Q, int N>
 __global__ void __launch_bounds__(sgs_block_threads<Q>()) k_filter_lhs(FieldArgs a, const CeedMiDiffFilterContext ctx) {
   using Dm          = Dims<P, Q>;

@@ -75,9 +75,9 @@ __global__ void k_rstr_t(const int *off, int nelem, int esize, int ncomp, int cs
 }
 
 // Deterministic second scatter pass: one thread per (L-vector node, component) item.  Row k's contributions are the
-// E-vector slots t_rowptr[k] .. t_rowptr[k+1]-1 (node-sorted E-vector); they are summed in ascending order.  Each thread handles NPT items a grid stride apart
-// and issues all their row-pointer loads, then all their contribution loads (up to 8 per row, the most a hexahedral
-// mesh node has), so a thread waits on two memory round trips for NPT items.
+// E-vector slots t_rowptr[k] .. t_rowptr[k+1]-1 (node-sorted E-vector); they are summed in ascending order.  Each thread
+// handles NPT items a grid stride apart and issues all their row-pointer loads, then all their contribution loads (up to 8
+// per row, the most a hexahedral mesh node has), so a thread waits on two memory round trips for NPT items.
 template <int NPT>
 __global__ void __launch_bounds__(256) k_node_gather(int nrows, int ncomp, int cs, const int *__restrict__ rowptr, const int *__restrict__ toff,
                                                      const double *__restrict__ ev, double *__restrict__ v, bool overwrite) {
@@ -158,7 +158,7 @@ __global__ void __launch_bounds__(256) k_layout_tiles(GatherTiles g, const int *
 // k_node_gather (identical results).  A thread per row that reads its slots straight from memory asks for each line 5 to 10
 // times and spends the time on requests that wait for a line already on its way (measured: 0.9 of the cycles, and L2 to L1
 // traffic of 4.7 times the E-vector at p=2).
-// Tiles hold at most kGatherSlots slots (20 KB of LDS: 7 blocks a CU) and as many rows; a row with more slots is a tile by
+// Tiles hold at most kGatherSlots slots (23.6 KB of LDS with the places and row starts: 6 blocks a CU) and as many rows; a row with more slots is a tile by
 // itself, summed straight from memory.  The tiles are split into 8 contiguous ranges, one per XCD (block b runs on XCD
 // b % 8; the grid is a multiple of 8), so that a range's E-vector lines go to one L2.
 // Measured against a thread per row: 64^3 p=2 177 -> 122 us (3.4 TB/s), 40^3 p=4 196 -> 158 us, 32^3 p=3 50 -> 44 us.
@@ -251,7 +251,8 @@ __global__ void k_dot(const double *x, const double *y, long long n, double *par
 // Streaming kernels over the vectors of one iteration, bound by their bytes: 2 vectors read for p.Ap, 5 read and 2 written
 // by the update, 3 read and 1 written by the direction, against 21 by separate dot, axpy and multiply calls.  A kernel that
 // needs a scalar sums the block partials before it itself (4 KB per block, out of L2), which costs no launch and no host read.
-// Measured at 2.9 M entries: 53 us an iteration (dot 9.0, residual 29.2, direction 15.1), 142 us before (with the fill and the reads' synchronizations).
+// Measured at 2.9 M entries: 53 us an iteration (dot 9.0, residual 29.2, direction 15.1), 142 us before (with the fill and the
+// reads' synchronizations).
 constexpr int kCgThreads = 512;
 
 __device__ __forceinline__ double cg_block_sum(double v, double *s) {  // s: one value per wave
