@@ -2,8 +2,8 @@
 src/smartsim/sgs_dd_training.c).
 
 * DifferentialFilter_RHS (three state-variable sets): relative 2-norm <= 1e-12, max-norm <= 1e-11;
-* the LHS composite (DifferentialFilter_LHS_5 + _6 over the interleaved 11-component filtered field) and its Jacobi
-  diagonal, isotropic, grid-based anisotropic and with van Driest damping on a wall-normal direction: 1e-12;
+* the LHS (DifferentialFilter_LHS_11 over the interleaved filtered field; _1, _5 and _6 are in
+  test_gpu_filter_components.py) and its Jacobi diagonal, isotropic, grid-based anisotropic and with van Driest damping on a wall-normal direction: 1e-12;
 * the filter solve (KSPCG + Jacobi, natural norm, rtol 1e-10): the oracle's iteration count (+-1) and the solution to
   1e-9 relative;
 * the training pairs (filter, projected filtered velocity gradient, closure inputs, filtered SGS stress) against the

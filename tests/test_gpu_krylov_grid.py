@@ -1,7 +1,8 @@
-"""The reductions of the Krylov solvers at the edges of their grid: fewer entries than a block's 512 threads, a ragged last
-block, and more than the 256 blocks take twice; restarts below, at and above the 8 basis vectors that a row of blocks
-takes, and the largest.  Explicit steps with the consistent mass solved by GMRES to 1e-10, against the oracle's: 1e-11 on the
-state, as in test_gpu_ts.py (the update is a small part of it)."""
+"""GMRES at the edges of its kernels' grid: fewer entries than a block's 512 threads, a ragged last block, and more than the
+256 blocks take twice; restarts below, at and above the 8 basis vectors that a row of blocks takes, and the largest.
+Explicit steps with the consistent mass solved by GMRES to 1e-10, against the oracle's: 1e-11 on the state, as in
+test_gpu_ts.py (the update is a small part of it).  A solver reaches that solution with wrong sums too: the reductions
+themselves are compared in test_gpu_reductions.py."""
 import sys
 
 import numpy as np

@@ -40,7 +40,8 @@ def test_residual_and_jacobian_at_block_edges(degree, q_extra, shape, scatter):
 @pytest.mark.parametrize("degree", [1, 2, 3, 4])
 @pytest.mark.parametrize("shape", [(1, 1, 1), (3, 1, 1), (3, 3, 1)])
 def test_filter_operator_at_block_edges(degree, shape):
-    """The same stage with 5 and 6 components in the filter operator, whose right-hand side has 11 outputs."""
+    """The filter operator: its right-hand side runs the same stage with 11 outputs, its left-hand side with 6 components at a time at
+    degree 4 (degrees 1 and 2 have a kernel of a lane per component, degree 3 the 4 x 4 x 4 element's stages)."""
     print(f"line stage filter degree={degree} shape={shape}", flush=True)
     sys.stdout.flush()
     case = make_case(shape=shape, degree=degree, periodic=(False, False, False), seed=13 + degree)
