@@ -31,7 +31,7 @@ HBM_PEAK_GBS = 8000.0
 # profiles/ifunction_newtonian_tgv32_p3_traffic.md.  A stored figure, not measured by the run that reports it (the
 # line says so); other workloads report traffic null.
 # With --qdata recompute the same two runs give 520.6 MB (fused kernel 381.5 MB, node gather 139.1 MB).
-PMC_TRAFFIC_BYTES = {((32, 32, 32), 3, "twopass", "stored"): 691.1e6, ((32, 32, 32), 3, "twopass", "recompute"): 520.6e6}
+PMC_TRAFFIC_BYTES = {((32, 32, 32), 3, "twopass", "stored"): 681.9e6, ((32, 32, 32), 3, "twopass", "recompute"): 517.6e6}
 METRIC = "GDoF/s Newtonian residual+Jacobian apply (p=3); LES error per GPU-second"
 FP64_PEAK_TFLOPS, FP32_PEAK_TFLOPS = 78.6, 157.3
 # Floating-point operations per quadrature point of the QFunction bodies at the default workload (primitive
