@@ -1336,10 +1336,10 @@ static bool diag_two_pass(Ceed ceed, const OpPlan *p) {
 }
 static int diag_evec_begin(Ceed ceed, OpPlan *p, VolumeArgs &a, bool point_block) {
   a.ev = nullptr;
+  GatherTiles tiles;  // on either route, as by an apply: an allocation-free apply may come next
+  if (ceed->scatter == 1 && !g_no_alloc) MI_CALL(rstr_gather_tiles(p->r_q, &tiles));
   if (!point_block && !diag_two_pass(ceed, p)) return 0;
-  GatherTiles tiles;
-  if (point_block) MI_CALL(rstr_transpose_map(p->r_q));
-  else MI_CALL(rstr_gather_tiles(p->r_q, &tiles));
+  MI_CALL(rstr_transpose_map(p->r_q));
   return ceed_workspace(ceed, (size_t)p->nelem * p->r_q->elem_size * (point_block ? 25 : 5), &a.ev);
 }
 static int diag_evec_finish(Ceed ceed, OpPlan *p, const VolumeArgs &a, bool point_block, bool overwrite) {

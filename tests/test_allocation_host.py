@@ -166,3 +166,25 @@ prob.ijacobian_point_block_diagonal(pb, 90.0)
 assert count(b"k_node_gather_blocks") - before[0] == 1
 assert count(b"k_fill") - before[1] == {int(scatter == "atomic")}
 """)
+
+
+@pytest.mark.parametrize("shape,point_block", [((3, 2, 2), False), ((16, 16, 15), False), ((3, 2, 2), True)])
+def test_allocation_free_apply_behind_a_diagonal(fake, shape, point_block):
+    """An assembled diagonal prepares an operator for the allocation-free apply as an apply does, whichever route it took."""
+    _run(fake, f"""
+from ceed_objects import INTERP, NONE, CeedObjects
+case, prob = problem({shape})
+mesh, tab, c = case["mesh"], case["tab"], CeedObjects(prob)
+r = c._restriction(mesh.nelem, tab.P ** 3, 5, 5 * mesh.nnodes, 5 * np.asarray(mesh.offsets))
+f = (r, c._basis(5, tab.P, prob._keep["B"], prob._keep["D"]), c._pointer("CEED_VECTOR_ACTIVE"))
+op = c.operator("qfunctions/mass.h:Mass_5", None, [("u", 5, INTERP), ("qdata", 10, NONE)], [("v", 5, INTERP)],
+                {{"u": f, "qdata": (c.strided(10), c._pointer("CEED_BASIS_NONE"), c.vector(prob.qdata())), "v": f}})
+v, w = c.vector(np.zeros(5 * mesh.nnodes)), c.vector(np.zeros(5 * mesh.nnodes))
+d = c.vector(np.zeros(({25 if point_block else 5}) * mesh.nnodes))
+c._call("CeedOperatorLinearAssemble{'PointBlock' if point_block else ''}Diagonal", op, d, None)
+c._call("CeedVectorSetValue", w, ct.c_double(0.0))  # the output and the input have device arrays
+c._call("CeedVectorScale", v, ct.c_double(1.0))
+size = hip.fake_dev_bytes()
+c._call("CeedMiOperatorApplyNoAlloc", op, v, w)
+assert hip.fake_dev_bytes() == size
+""")

@@ -9,12 +9,12 @@ import numpy as np
 import pytest
 
 import pyoracle as O
+from ceed_objects import COPY_VALUES, GRAD, INTERP, NONE, CeedObjects
 from helpers import make_case, oracle_setup, product_context, rel_err
-from pyhonee.driver import CEED_MEM_HOST, NewtonianContext, NewtonianProblem, load_libs
+from pyhonee.driver import CEED_MEM_HOST, NewtonianContext, NewtonianProblem
 
 pytestmark = pytest.mark.gpu
 
-COPY_VALUES, (NONE, INTERP, GRAD) = 0, (0, 1, 2)
 FILTER = dict(grid_based_width=True, width_scaling=(1.5, 0.7, 1.0))
 
 
@@ -23,78 +23,28 @@ class FilterContext(ct.Structure):
                 ("damping_function", ct.c_int), ("damping_constant", ct.c_double), ("newt_ctx", NewtonianContext)]
 
 
-class FilterLHS:
+class FilterLHS(CeedObjects):
     """Composite of DifferentialFilter_LHS_N over the component ranges [(offset, N), ...] of an 11-component field."""
 
     def __init__(self, prob, aniso, parts):
-        self.lib, self.prob, self.parts = load_libs()[0], prob, parts
-        mesh, tab, ceed = prob.mesh, prob.tab, ct.c_void_p(prob.ceed)
-        self.ceed, self.n, Q3 = ceed, 11 * mesh.nnodes, tab.Q ** 3
-        x = self._restriction(mesh.nelem, 8, 3, 3 * prob.m.nxnodes, 3 * np.asarray(mesh.xoffsets))
-        qd, an = (self._made("CeedElemRestrictionCreateStrided", ceed, mesh.nelem, Q3, n, ct.c_longlong(mesh.nelem * Q3 * n), self._symbol("CEED_STRIDES_BACKEND"))
-                  for n in (10, 7))
-        bx = self._basis(3, 2, prob._keep["Bx"], prob._keep["Dx"])
+        super().__init__(prob)
+        mesh, tab, ceed = prob.mesh, prob.tab, self.ceed
+        self.n = 11 * mesh.nnodes
+        x, bx = self._restriction(mesh.nelem, 8, 3, 3 * prob.m.nxnodes, 3 * np.asarray(mesh.xoffsets)), self._basis(3, 2, prob._keep["Bx"], prob._keep["Dx"])
         ctx = FilterContext(True, (ct.c_double * 3)(*FILTER["width_scaling"]), 0.1, 0.0, 0, 25.0, prob.ctx)
         qctx = self._made("CeedQFunctionContextCreate", ceed)
         self._call("CeedQFunctionContextSetData", qctx, CEED_MEM_HOST, COPY_VALUES, ct.c_size_t(ct.sizeof(ctx)), ct.byref(ctx))
-        vx, vq, va = self.vector(prob._keep["xcoord"]), self.vector(prob.qdata()), self.vector(aniso)
-        self.op = self._made("CeedOperatorCreateComposite", ceed)
-        self.host = ct.CFUNCTYPE(ct.c_int, ct.c_void_p, ct.c_int, ct.c_void_p, ct.c_void_p)(lambda *a: 1)
         active, no_basis = self._pointer("CEED_VECTOR_ACTIVE"), self._pointer("CEED_BASIS_NONE")
+        passive = {"anisotropy tensor": (self.strided(7), no_basis, self.vector(aniso)), "x": (x, bx, self.vector(prob._keep["xcoord"])),
+                   "qdata": (self.strided(10), no_basis, self.vector(prob.qdata()))}
+        self.op = self._made("CeedOperatorCreateComposite", ceed)
         for offset, N in parts:
-            r = self._restriction(mesh.nelem, tab.P ** 3, N, self.n, 11 * np.asarray(mesh.offsets) + offset)
-            b = self._basis(N, tab.P, prob._keep["B"], prob._keep["D"])
-            qf = self._made("CeedQFunctionCreateInterior", ceed, 1, self.host, f"qfunctions/differential_filter.h:DifferentialFilter_LHS_{N}".encode())
-            self._call("CeedQFunctionSetContext", qf, qctx)
-            ins = [("q", N, INTERP), ("Grad_q", 3 * N, GRAD), ("anisotropy tensor", 7, NONE), ("x", 3, INTERP), ("qdata", 10, NONE)]
-            for name, size, mode in ins:
-                self._call("CeedQFunctionAddInput", qf, name.encode(), size, mode)
-            for name, size, mode in (("v", N, INTERP), ("Grad_v", 3 * N, GRAD)):
-                self._call("CeedQFunctionAddOutput", qf, name.encode(), size, mode)
-            sub = self._made("CeedOperatorCreate", ceed, qf, None, None)
-            for name, f in (("q", (r, b, active)), ("Grad_q", (r, b, active)), ("anisotropy tensor", (an, no_basis, va)), ("x", (x, bx, vx)),
-                            ("qdata", (qd, no_basis, vq)), ("v", (r, b, active)), ("Grad_v", (r, b, active))):
-                self._call("CeedOperatorSetField", sub, name.encode(), *f)
+            f = (self._restriction(mesh.nelem, tab.P ** 3, N, self.n, 11 * np.asarray(mesh.offsets) + offset),
+                 self._basis(N, tab.P, prob._keep["B"], prob._keep["D"]), active)
+            sub = self.operator(f"qfunctions/differential_filter.h:DifferentialFilter_LHS_{N}", qctx,
+                                [("q", N, INTERP), ("Grad_q", 3 * N, GRAD), ("anisotropy tensor", 7, NONE), ("x", 3, INTERP), ("qdata", 10, NONE)],
+                                [("v", N, INTERP), ("Grad_v", 3 * N, GRAD)], {"q": f, "Grad_q": f, **passive, "v": f, "Grad_v": f})
             self._call("CeedOperatorCompositeAddSub", self.op, sub)
-
-    def _symbol(self, name):
-        return ct.byref(ct.c_int.in_dll(self.lib, name))
-
-    def _pointer(self, name):
-        return ct.c_void_p.in_dll(self.lib, name)
-
-    def _call(self, name, *args):
-        if getattr(self.lib, name)(*args):
-            msg = ct.c_char_p()
-            self.lib.CeedGetErrorMessage(self.ceed, ct.byref(msg))
-            raise RuntimeError(f"{name}: {msg.value.decode()}")
-
-    def _made(self, name, *args):
-        h = ct.c_void_p()
-        self._call(name, *args, ct.byref(h))
-        return h
-
-    def _restriction(self, nelem, size, ncomp, length, offsets):
-        off = np.ascontiguousarray(offsets, dtype=np.int32)
-        return self._made("CeedElemRestrictionCreate", self.ceed, nelem, size, ncomp, 1, ct.c_longlong(length), CEED_MEM_HOST, COPY_VALUES,
-                          off.ctypes.data_as(ct.c_void_p))
-
-    def _basis(self, ncomp, P, B, D):
-        k = self.prob._keep
-        return self._made("CeedBasisCreateTensorH1", self.ceed, 3, ncomp, P, self.prob.tab.Q, *(a.ctypes.data_as(ct.c_void_p) for a in (B, D, k["qref"], k["qweight"])))
-
-    def vector(self, a):
-        a = np.ascontiguousarray(a, dtype=np.float64).ravel()
-        v = self._made("CeedVectorCreate", self.ceed, ct.c_longlong(a.size))
-        self._call("CeedVectorSetArray", v, CEED_MEM_HOST, COPY_VALUES, a.ctypes.data_as(ct.c_void_p))
-        return v
-
-    def read(self, v):
-        p, out = ct.POINTER(ct.c_double)(), np.zeros(self.n)
-        self._call("CeedVectorGetArrayRead", v, CEED_MEM_HOST, ct.byref(p))
-        out[:] = np.ctypeslib.as_array(p, (self.n,))
-        self._call("CeedVectorRestoreArrayRead", v, ct.byref(p))
-        return out.reshape(-1, 11)
 
     def apply(self, vin, vout):
         self._call("CeedOperatorApply", self.op, vin, vout, None)
@@ -131,10 +81,10 @@ def test_operator_of_components(degree, shape, scatter, parts):
     dref = O.diff_filter_lhs_diagonal(om, f, qd, acol, 11).reshape(-1, 11) * mine
     for _ in range(2):
         lhs.apply(vin, vout)
-        e2, emax = rel_err(lhs.read(vout), ref)
+        e2, emax = rel_err(lhs.read(vout, lhs.n).reshape(-1, 11), ref)
         assert e2 < 1e-12 and emax < 1e-11, (e2, emax)
     lhs.diagonal(vout)
-    e2, emax = rel_err(lhs.read(vout), dref)
+    e2, emax = rel_err(lhs.read(vout, lhs.n).reshape(-1, 11), dref)
     assert e2 < 1e-12 and emax < 1e-11, (e2, emax)
     prob.close()
 
